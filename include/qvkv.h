@@ -136,8 +136,8 @@ int qvkv_max_arena(const qvkv_dev *dev, uint64_t *out);
  * append_q8_fast, append_nts, gather_split, gather_q8_fast, gather_t, gather_uf, copy_u,
  * copy_t, attn_full, attn_stream, attn_stream_wg, stream_unit_cost, attn_target, fused_q8,
  * attn_waves4_f16, attn_waves3_q8, attn_pack, attn_ids_below, attn_xcd, prefill_v2,
- * prefill_lds_pad, prefill_exact_p, prefill_dma, prefill_q8_fast, prelude_fast,
- * prelude_wide, prelude_full_wg.  An unknown name is QVKV_E_SHAPE. */
+ * prefill_lds_pad, prefill_exact_p, prefill_dma, prefill_chunks, prefill_q8_fast,
+ * prelude_fast, prelude_wide, prelude_full_wg.  An unknown name is QVKV_E_SHAPE. */
 int qvkv_tune(const char *name, int value);
 int qvkv_tune_get(const char *name, int *value);
 /* Every knob back to its default. */
@@ -241,7 +241,9 @@ int qvkv_attention_noalloc_async(qvkv_dev *dev, const qvkv_layout *layout, const
  * q row q_at[i] + j ([q_rows][heads][d] f32) and writes the same out row.  It attends
  * (causally) over positions 0..pos0[i]+j of its table exactly as qvkv_attention_async
  * would for an item with pos = pos0[i]+j; max_pos bounds pos0[i]+n_tok[i]-1 and max_tok
- * bounds n_tok[i].  Replaces the host prefill of the reference's forward pass, which
+ * bounds n_tok[i].  A launch with few rows shares each row block's context out to several
+ * workgroups, whose partial results go to a workspace of the stream (grown on first use; on
+ * a stream being captured that would have to grow it, the launch runs unsplit instead).  Replaces the host prefill of the reference's forward pass, which
  * stores a segment's rows and then runs math::attend per (token, head)
  * (crates/qubivex-arch/src/lib.rs:1296-1320); the reference has no device prefill.
  * q8_0 pools at d = 128 use a form that holds dequantised values in f16: a value scale

@@ -73,6 +73,12 @@ struct StreamState {
     int *d_err = nullptr;  // [0]: latched bits (ERR_*), [1]: taken by the last check
     void *ws = nullptr;    // attention workspace (partials of context chunks)
     uint64_t ws_bytes = 0;
+    // prefill workspace (partials of split row blocks): its own buffer, so that a prefill
+    // never replaces the attention workspace that a captured decode step replays with
+    void *pws = nullptr;
+    uint64_t pws_bytes = 0;
+    bool pws_captured = false;                          // a capture has recorded pws
+    std::vector<std::pair<void *, uint64_t>> pws_kept;  // outgrown, but recorded by a capture
     std::mutex check_mu;   // one check at a time per stream
     // The attention launches of this stream, one at a time: the workspace is grown (which
     // waits for this stream to drain) and handed to the launch under it.  Other streams'
@@ -200,6 +206,34 @@ int ensure(qvkv_dev *dev, hipStream_t s, void **buf, uint64_t *have, uint64_t ne
 int ensure_attention(qvkv_dev *dev, StreamState *st, const qvkv::AttnPlan &p) {
     if (!p.ws_bytes) return QVKV_OK;
     return ensure(dev, st->stream, &st->ws, &st->ws_bytes, p.ws_bytes);
+}
+
+// A prefill plan with the stream's prefill workspace grown for its split, or the plan without
+// the split where it cannot grow: on a stream that is being captured (no allocation, no
+// wait there), and when the device has no memory for it (the unsplit launch needs none).
+// A buffer that a capture has recorded is never freed before the device closes: its graph
+// may be replayed after a larger launch.  Caller holds st->ws_mu.
+qvkv::PrefillPlan ensure_prefill(qvkv_dev *dev, StreamState *st, const qvkv::PrefillPlan &p) {
+    if (p.n_chunks == 1) return p;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st->stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return qvkv::PrefillPlan{};
+    }
+    const bool capturing = cap != hipStreamCaptureStatusNone;
+    if (st->pws_bytes < p.ws_bytes) {
+        if (capturing) return qvkv::PrefillPlan{};
+        if (st->pws_captured) {
+            st->pws_kept.push_back({st->pws, st->pws_bytes});
+            st->pws = nullptr;
+            st->pws_bytes = 0;
+            st->pws_captured = false;
+        }
+        if (ensure(dev, st->stream, &st->pws, &st->pws_bytes, p.ws_bytes) != QVKV_OK)
+            return qvkv::PrefillPlan{};
+    }
+    st->pws_captured |= capturing;
+    return p;
 }
 
 // The state of `stream`, created on first use.  Caller holds dev->mu.
@@ -497,6 +531,8 @@ void qvkv_close(qvkv_dev *dev) {
     (void)hipDeviceSynchronize();
     for (StreamState *st : dev->streams) {
         dev_free(dev, st->ws, st->ws_bytes);
+        dev_free(dev, st->pws, st->pws_bytes);
+        for (const auto &k : st->pws_kept) dev_free(dev, k.first, k.second);
         dev_free(dev, st->d_err, 256);
         delete st;
     }
@@ -821,11 +857,17 @@ int qvkv_prefill_attention_async(qvkv_dev *dev, const qvkv_layout *layout, const
     if (!pool || !q || !blocks || !table_at || !pos0 || !q_at || !n_tok || !out)
         return fail(QVKV_E_SHAPE, "shape mismatch in prefill attention: null pointer");
     if (int rc = set_device(dev)) return rc;
+    // the workspace's locks, as in qvkv_attention_async
+    std::unique_lock<std::mutex> host_lk(dev->host_mu, std::defer_lock);
+    if ((hipStream_t)stream == dev->stream) host_lk.lock();
     StreamState *st;
     if (int rc = state_of(dev, stream, &st)) return rc;
-    return launched(dev, qvkv::launch_prefill(g, pool, pool_blocks, q, blocks, n_table, table_at,
+    std::lock_guard<std::mutex> wl(st->ws_mu);
+    const qvkv::PrefillPlan p = ensure_prefill(
+        dev, st, qvkv::plan_prefill(g, n_seg, heads, max_pos, max_tok));
+    return launched(dev, qvkv::launch_prefill(g, p, pool, pool_blocks, q, blocks, n_table, table_at,
                                               pos0, q_at, n_tok, n_seg, heads, max_pos, max_tok,
-                                              q_rows, out, st->d_err, st->stream),
+                                              q_rows, out, st->pws, st->d_err, st->stream),
                     "prefill attention launch");
 }
 
@@ -996,12 +1038,16 @@ hipError_t attend_tokens(qvkv_dev *dev, const Geometry &g, const qvkv::AttnPlan 
                          uint64_t n_table, const uint32_t *dtable_at, const uint32_t *dpos,
                          uint32_t s, uint32_t heads, uint32_t max_pos, float *dout,
                          bool f16_values = true) {
-    if (sg.max_tok >= 2)
-        return qvkv::launch_prefill(g, pool, held, dq, dblocks, n_table,
+    if (sg.max_tok >= 2) {
+        const uint32_t n_seg = (uint32_t)sg.n_tok.size();
+        const qvkv::PrefillPlan pp = ensure_prefill(
+            dev, dev->own, qvkv::plan_prefill(g, n_seg, heads, max_pos, sg.max_tok, f16_values));
+        return qvkv::launch_prefill(g, pp, pool, held, dq, dblocks, n_table,
                                     st.at<uint32_t>(dev, ss.ta), st.at<uint32_t>(dev, ss.p0),
                                     st.at<uint32_t>(dev, ss.qa), st.at<uint32_t>(dev, ss.nt),
-                                    (uint32_t)sg.n_tok.size(), heads, max_pos, sg.max_tok, s,
-                                    dout, dev->own->d_err, dev->stream, f16_values);
+                                    n_seg, heads, max_pos, sg.max_tok, s, dout, dev->own->pws,
+                                    dev->own->d_err, dev->stream, f16_values);
+    }
     return qvkv::launch_attention(g, plan, pool, held, dq, dblocks, n_table, dtable_at, dpos, s,
                                   heads, max_pos, dout, dev->own->ws, dev->own->d_err, dev->stream);
 }

@@ -106,6 +106,7 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     X(PREFILL_LDS_PAD, "prefill_lds_pad", 0)                                                    \
     X(PREFILL_EXACT_P, "prefill_exact_p", 0)                                                    \
     X(PREFILL_DMA, "prefill_dma", 1)                                                            \
+    X(PREFILL_CHUNKS, "prefill_chunks", 0)      /* chunks per row block; 0: by the plan */     \
     X(PREFILL_Q8_FAST, "prefill_q8_fast", 1)                                                    \
     X(PRELUDE_FAST, "prelude_fast", 1)                                                          \
     X(PRELUDE_WIDE, "prelude_wide", 1)                                                          \
@@ -124,12 +125,21 @@ void reset_tune();
 // Paged prefill attention over segments of consecutive tokens (kernels.hip).
 int check_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t max_tok,
                   const char **why);
-hipError_t launch_prefill(const Geometry &g, const void *pool, uint64_t pool_blocks,
-                          const float *q, const uint32_t *blocks, uint64_t n_table,
-                          const uint32_t *table_at, const uint32_t *pos0, const uint32_t *q_at,
-                          const uint32_t *n_tok, uint32_t n_seg, uint32_t heads,
-                          uint32_t max_pos, uint32_t max_tok, uint64_t q_rows, float *out,
-                          int *err, hipStream_t s, bool f16_values = true);
+// The plan of a prefill launch: workgroups per row block (64 query rows of a (segment, KV
+// head)), and the workspace that a split launch (n_chunks > 1) keeps its partials in.
+constexpr uint32_t PREFILL_MAX_CHUNKS = 16;
+struct PrefillPlan {
+    uint32_t n_chunks = 1;
+    uint64_t ws_bytes = 0;
+};
+PrefillPlan plan_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t max_pos,
+                         uint32_t max_tok, bool f16_values = true);
+hipError_t launch_prefill(const Geometry &g, const PrefillPlan &plan, const void *pool,
+                          uint64_t pool_blocks, const float *q, const uint32_t *blocks,
+                          uint64_t n_table, const uint32_t *table_at, const uint32_t *pos0,
+                          const uint32_t *q_at, const uint32_t *n_tok, uint32_t n_seg,
+                          uint32_t heads, uint32_t max_pos, uint32_t max_tok, uint64_t q_rows,
+                          float *out, void *ws, int *err, hipStream_t s, bool f16_values = true);
 // New key and value rows of a fused append + attention (n_items rows of kv_out floats
 // each, stored at each item's position pos[i] and attended there); null in a plain
 // attention launch.  The fused form runs at d = 64, 128, 256 for f16 pools, and for q8_0

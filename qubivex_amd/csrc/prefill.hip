@@ -23,6 +23,10 @@ namespace qvkv {
         const uint32_t *__restrict__ q_at, const uint32_t *__restrict__ n_tok, uint32_t n_seg,  \
         uint32_t H, uint32_t max_pos, uint32_t max_tok, uint64_t q_rows, uint32_t n_cb,         \
         float *__restrict__ out, Geo geo, int *err
+// (the forms that split the context: n_ch chunks per row block, their partials in ws; n_sub:
+// row_block)
+#define QV_PREFILL_SPLIT_PARAMS                                                                 \
+    QV_PREFILL_PARAMS, uint32_t n_ch, uint32_t n_sub, float *__restrict__ ws, uint64_t n_parts
 
 template <int D, bool Q8>
 __global__ __launch_bounds__(256) void k_prefill_mfma(QV_PREFILL_PARAMS) {
@@ -150,6 +154,77 @@ __global__ __launch_bounds__(256) void k_prefill_mfma(QV_PREFILL_PARAMS) {
 // are exact f16 x f16 in f32 accumulators as in decode.
 // ---------------------------------------------------------------------------------
 
+// ---- the context split of a row block (64 query rows) ----
+//
+// A launch of few row blocks (one request's chunk, a few new tokens after a cached prefix)
+// leaves most of the chip's 768 workgroup slots empty, so each row block's tiles are shared
+// out to n_ch workgroups (chunk c takes tiles [c n / n_ch, (c + 1) n / n_ch) of its n);
+// their partials (unnormalised rows, and each row's max and sum) go to ws:
+//   rows [row block][chunk][64][D] f32, then (max, sum) [row block][chunk][64][2]
+// and k_prefill_merge combines them.
+struct TileRange {
+    uint32_t first, end;
+};
+__device__ __forceinline__ TileRange chunk_tiles(uint32_t n, uint32_t ch, uint32_t n_ch) {
+    return TileRange{n * ch / n_ch, n * (ch + 1) / n_ch};
+}
+
+// The row block and chunk of a workgroup.  Workgroups are dealt to the 8 XCDs round-robin
+// (id % 8).  The row blocks of one (segment, KV head, chunk) read the same tiles, so they
+// form a group on one XCD (its L2 serves the repeats), and consecutive groups go to
+// different XCDs: segments of different lengths then load the XCDs alike (with each XCD
+// taking an eighth of the launch in order, 8 segments of 8 to 64 tokens put the longest
+// on one XCD).  Few groups are cut into n_sub interleaved parts each, so that their number
+// is a multiple of 8.  Blocks of later tokens, whose contexts are longest, start first.
+struct RowBlock {
+    uint32_t qb, ch, sg;
+};
+__device__ __forceinline__ RowBlock row_block(uint32_t n_cb, uint32_t n_ch, uint32_t n_sub,
+                                              bool xcd_map) {
+    const uint32_t bid = blockIdx.x, per = (n_cb + n_sub - 1) / n_sub;
+    const uint32_t i = xcd_map ? bid / 8 : bid;
+    const uint32_t part = xcd_map ? i / per * 8 + bid % 8 : i / per;
+    const uint32_t at = i % per * n_sub + part % n_sub, group = part / n_sub;
+    // (at >= n_cb, in a last part: past every block, as n_cb - 1 - at wraps)
+    return RowBlock{n_cb - 1 - at, group % n_ch, group / n_ch};
+}
+
+// One wave's 16 rows (row rw0 + 4 (lane / 16) + i at d = 16 j + lane % 16), normalised to
+// `out`, or as chunk `part` of a split row block (r_in: the wave's first row in the block).
+template <int D>
+__device__ __forceinline__ void store_rows(const f4 *acc, float m, float l, uint32_t rw0,
+                                           uint32_t nrows, uint32_t r_in, uint32_t part,
+                                           uint32_t n_ch, uint32_t GS, uint32_t H, uint32_t qa,
+                                           uint32_t g, float *out, float *ws, uint64_t n_parts) {
+    const uint32_t lane = threadIdx.x & 63u, col = lane & 15u, grp = lane >> 4;
+    float lr[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) lr[i] = __shfl(l, 4 * (int)grp + i);
+    if (n_ch == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t rr = rw0 + 4 * grp + i;
+            if (rr >= nrows) continue;
+            const uint32_t tr = rr / GS, hr = rr % GS;
+            float *orow = out + ((uint64_t)(qa + tr) * H + (uint64_t)g * GS + hr) * D;
+            const float inv = 1.0f / lr[i];
+#pragma unroll
+            for (int j = 0; j < D / 16; j++) orow[16 * j + col] = acc[j][i] * inv;
+        }
+        return;
+    }
+    float *rows = ws + ((uint64_t)part * 64u + r_in) * D;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < D / 16; j++) rows[(4 * grp + i) * D + 16 * j + col] = acc[j][i];
+    if (grp == 0) {  // lane col holds row col's max and (after the caller's sums) its total
+        float *ml = ws + n_parts * 64u * D + ((uint64_t)part * 64u + r_in + col) * 2;
+        ml[0] = m;
+        ml[1] = l;
+    }
+}
+
 // a compile-time flag passed to a generic lambda
 template <bool V>
 struct Flag {
@@ -193,7 +268,7 @@ __device__ __forceinline__ uint32_t vswz(uint32_t r) {
 // probabilities, so the weights the output is normalised by are exactly those applied.
 template <int D, bool DMA, bool PS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DMA ? 3 : 1)))
-void k_prefill_f16(QV_PREFILL_PARAMS) {
+void k_prefill_f16(QV_PREFILL_SPLIT_PARAMS) {
     constexpr int TP = PrefillLds<D>::TP;
     constexpr int KS = D / 32;                 // QK k-steps
     constexpr int NDB = D / 16;                // PV d blocks
@@ -206,20 +281,15 @@ void k_prefill_f16(QV_PREFILL_PARAMS) {
 
     const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
     const uint32_t GS = H / G;
-    uint32_t bid = blockIdx.x;
-    if (geo.xcd_map) {
-        const uint32_t nb = gridDim.x, qn = nb / 8, rn = nb % 8;
-        const uint32_t x = bid % 8, i = bid / 8;
-        bid = x < rn ? x * (qn + 1) + i : rn * (qn + 1) + (x - rn) * qn + i;
-    }
-    const uint32_t qb = bid % n_cb;
-    const uint32_t sg = bid / n_cb;
+    const RowBlock rb = row_block(n_cb, n_ch, n_sub, geo.xcd_map != 0);
+    const uint32_t qb = rb.qb, ch = rb.ch, sg = rb.sg;
+    if (qb >= n_cb) return;
     const uint32_t g = sg % G;
     const uint32_t seg = sg / G;
     if (seg >= n_seg) return;
     const uint32_t nt = n_tok[seg], p0s = pos0[seg], qa = q_at[seg], tab = table_at[seg];
     if (nt == 0) return;
-    const bool lead = threadIdx.x == 0 && qb == 0 && g == 0;
+    const bool lead = threadIdx.x == 0 && qb == 0 && ch == 0 && g == 0;
     if (nt > max_tok || (uint64_t)p0s + nt - 1 > max_pos) {
         if (lead) flag(err, ERR_POS);
         return;
@@ -238,7 +308,9 @@ void k_prefill_f16(QV_PREFILL_PARAMS) {
     if (r0 >= nrows) return;  // the whole workgroup: no barrier has run yet
     const uint32_t wg_last = min(nt - 1, (r0 + 63u) / GS);
     const uint32_t n_wg = p0s + wg_last + 1;   // positions the workgroup's rows see
-    const uint32_t ntiles = (n_wg + TP - 1) / TP;
+    const TileRange tr = chunk_tiles((n_wg + TP - 1) / TP, ch, n_ch);
+    const uint32_t t_first = tr.first, ntiles = tr.end;  // tiles t_first .. ntiles - 1
+    if (t_first >= ntiles) return;
 
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
     const uint32_t col = lane & 15u, grp = lane >> 4;
@@ -313,7 +385,8 @@ void k_prefill_f16(QV_PREFILL_PARAMS) {
     // ids at or past pool_ids are bad (the clamp only matters for id 0xffffffff in a pool of
     // 2^32 blocks or more, which no device holds: a block is at least 2 KiB)
     const uint32_t pool_ids = pool_blocks > 0xffffffffull ? 0xffffffffu : (uint32_t)pool_blocks;
-    uint32_t at_bi = 0, at_row = 0;         // block index / row of the next half to resolve
+    // block index / row of the next half to resolve
+    uint32_t at_bi = geo.fd_b.div(t_first * TP), at_row = t_first * TP - at_bi * B;
     auto step16 = [&]() {
         at_row += 16u;
         if (at_row == B) {
@@ -354,7 +427,7 @@ void k_prefill_f16(QV_PREFILL_PARAMS) {
         if (b == nullptr || r >= valid) return u4v{0u, 0u, 0u, 0u};
         return *(const u4v *)(b + off);
     };
-    auto load = [&](uint32_t t) {  // t = 0, 1, 2, ... in order
+    auto load = [&](uint32_t t) {  // t = t_first, t_first + 1, ... in order
         const uint32_t p0 = t * TP;
         const uint8_t *b0 = resolved(0), *b1 = resolved(1);
         if (t + 1 < ntiles) resolve(t + 1);
@@ -504,13 +577,13 @@ void k_prefill_f16(QV_PREFILL_PARAMS) {
         }
     };
 
-    resolve(0);
+    resolve(t_first);
     if constexpr (!DMA) {
-        load(0);
+        load(t_first);
         store(0);
         __syncthreads();
-        for (uint32_t t = 0; t < ntiles; t++) {
-            const int buf = (int)(t & 1u);
+        for (uint32_t t = t_first; t < ntiles; t++) {
+            const int buf = (int)((t - t_first) & 1u);
             if (t + 1 < ntiles) load(t + 1);
             tile(
                 t * TP,
@@ -575,7 +648,7 @@ void k_prefill_f16(QV_PREFILL_PARAMS) {
                 c_v[u] = __builtin_amdgcn_readfirstlane(isv ? 1u : 0u);
             }
         }();
-        // t = 0, 1, 2, ... in order; steady: t + 2 is below the last tile, so tile t is whole
+        // t = t_first, t_first + 1, ... in order; steady: t + 2 is below the last tile, so tile t is whole
         // and both halves of t + 1 start before n_wg
         auto issue = [&](auto steady, uint32_t t, DmaSlot<D> &sl) {
             constexpr bool STEADY = decltype(steady)::value;
@@ -668,9 +741,9 @@ void k_prefill_f16(QV_PREFILL_PARAMS) {
         };
         const Flag<false> any;
         const Flag<true> steady;
-        issue(any, 0, s0);
-        if (ntiles > 1) issue(any, 1, s1);
-        uint32_t t = 0;
+        issue(any, t_first, s0);
+        if (t_first + 1 < ntiles) issue(any, t_first + 1, s1);
+        uint32_t t = t_first;
         // steady steps t .. t + 2 issue tiles up to t + 4 and resolve up to t + 5, which must
         // not be the last tile (its second half may start past n_wg)
         for (; t + 7 <= ntiles; t += 3) {
@@ -689,19 +762,8 @@ void k_prefill_f16(QV_PREFILL_PARAMS) {
     // ---- row totals; lane (col, grp) holds O rows 4 grp + i at d = 16 j + col
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
-    float lr[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) lr[i] = __shfl(l, 4 * (int)grp + i);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t rr = rw0 + 4 * grp + i;
-        if (rr >= nrows) continue;
-        const uint32_t tr = rr / GS, hr = rr % GS;
-        float *orow = out + ((uint64_t)(qa + tr) * H + (uint64_t)g * GS + hr) * D;
-        const float inv = 1.0f / lr[i];
-#pragma unroll
-        for (int j = 0; j < NDB; j++) orow[16 * j + col] = acc[j][i] * inv;
-    }
+    store_rows<D>(acc, m, l, rw0, nrows, rw0 - r0, (sg * n_cb + qb) * n_ch + ch, n_ch, GS, H, qa, g,
+                  out, ws, n_parts);
 }
 
 // ---------------------------------------------------------------------------------
@@ -728,7 +790,7 @@ struct Q8PrefillSlot {
 
 template <int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-void k_prefill_q8(QV_PREFILL_PARAMS) {
+void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS) {
     static_assert(D == 128, "q8_0 MFMA-throughput prefill is built for d = 128");
     constexpr int TP = 32;
     constexpr int KS = D / 32;                 // QK k-steps = quantization groups
@@ -738,20 +800,15 @@ void k_prefill_q8(QV_PREFILL_PARAMS) {
 
     const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
     const uint32_t GS = H / G;
-    uint32_t bid = blockIdx.x;
-    if (geo.xcd_map) {
-        const uint32_t nb = gridDim.x, qn = nb / 8, rn = nb % 8;
-        const uint32_t x = bid % 8, i = bid / 8;
-        bid = x < rn ? x * (qn + 1) + i : rn * (qn + 1) + (x - rn) * qn + i;
-    }
-    const uint32_t qb = bid % n_cb;
-    const uint32_t sg = bid / n_cb;
+    const RowBlock rb = row_block(n_cb, n_ch, n_sub, geo.xcd_map != 0);
+    const uint32_t qb = rb.qb, ch = rb.ch, sg = rb.sg;
+    if (qb >= n_cb) return;
     const uint32_t g = sg % G;
     const uint32_t seg = sg / G;
     if (seg >= n_seg) return;
     const uint32_t nt = n_tok[seg], p0s = pos0[seg], qa = q_at[seg], tab = table_at[seg];
     if (nt == 0) return;
-    const bool lead = threadIdx.x == 0 && qb == 0 && g == 0;
+    const bool lead = threadIdx.x == 0 && qb == 0 && ch == 0 && g == 0;
     if (nt > max_tok || (uint64_t)p0s + nt - 1 > max_pos) {
         if (lead) flag(err, ERR_POS);
         return;
@@ -770,7 +827,9 @@ void k_prefill_q8(QV_PREFILL_PARAMS) {
     if (r0 >= nrows) return;  // the whole workgroup: no barrier has run yet
     const uint32_t wg_last = min(nt - 1, (r0 + 63u) / GS);
     const uint32_t n_wg = p0s + wg_last + 1;
-    const uint32_t ntiles = (n_wg + TP - 1) / TP;
+    const TileRange tr = chunk_tiles((n_wg + TP - 1) / TP, ch, n_ch);
+    const uint32_t t_first = tr.first, ntiles = tr.end;  // tiles t_first .. ntiles - 1
+    if (t_first >= ntiles) return;
 
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
     const uint32_t col = lane & 15u, grp = lane >> 4;
@@ -851,7 +910,8 @@ void k_prefill_q8(QV_PREFILL_PARAMS) {
     // ids at or past pool_ids are bad (the clamp only matters for id 0xffffffff in a pool of
     // 2^32 blocks or more, which no device holds)
     const uint32_t pool_ids = pool_blocks > 0xffffffffull ? 0xffffffffu : (uint32_t)pool_blocks;
-    uint32_t at_bi = 0, at_row = 0;         // block index / row of the next half to resolve
+    // block index / row of the next half to resolve
+    uint32_t at_bi = geo.fd_b.div(t_first * TP), at_row = t_first * TP - at_bi * B;
     uint32_t nx_blk[2] = {0u, 0u}, nx_row[2] = {0u, 0u};
     bool nx_in[2] = {false, false};
     auto resolve = [&](uint32_t t) {        // the halves of tile t, after those of t - 1
@@ -875,7 +935,7 @@ void k_prefill_q8(QV_PREFILL_PARAMS) {
         return Half{nx_in[k] && !bad ? pool + (uint64_t)nx_blk[k] * geo.bb : nullptr,
                     g * B + nx_row[k]};
     };
-    auto load = [&](uint32_t t) {  // t = 0, 1, 2, ... in order
+    auto load = [&](uint32_t t) {  // t = t_first, t_first + 1, ... in order
         const uint32_t p0 = t * TP;
         const Half h0 = resolved(0), h1 = resolved(1);
         if (t + 1 < ntiles) resolve(t + 1);
@@ -1054,11 +1114,11 @@ void k_prefill_q8(QV_PREFILL_PARAMS) {
         if (t + 1 < ntiles) store(nxt);
         __syncthreads();
     };
-    resolve(0);
-    load(0);
+    resolve(t_first);
+    load(t_first);
     store(sb0);
     __syncthreads();
-    for (uint32_t t = 0; t < ntiles; t += 2) {
+    for (uint32_t t = t_first; t < ntiles; t += 2) {
         step(t, sb0, sb1);
         if (t + 1 < ntiles) step(t + 1, sb1, sb0);
     }
@@ -1066,19 +1126,71 @@ void k_prefill_q8(QV_PREFILL_PARAMS) {
     if (!wave_live) return;
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
-    float lr[4];
+    store_rows<D>(acc, m, l, rw0, nrows, rw0 - r0, (sg * n_cb + qb) * n_ch + ch, n_ch, GS, H, qa, g,
+                  out, ws, n_parts);
+}
+
+// Merge of a split launch: workgroup = 1024 / D rows of one row block, D / 4 lanes per row,
+// 4 values each; the chunks' partials in chunk order, 4 chunks' loads in flight.
+template <int D>
+__global__ __launch_bounds__(256) void k_prefill_merge(const float *__restrict__ ws,
+                                                       uint64_t n_table,
+                                                       const uint32_t *__restrict__ table_at,
+                                                       const uint32_t *__restrict__ pos0,
+                                                       const uint32_t *__restrict__ q_at,
+                                                       const uint32_t *__restrict__ n_tok,
+                                                       uint32_t H, uint32_t max_pos,
+                                                       uint32_t max_tok, uint64_t q_rows,
+                                                       uint32_t n_cb, float *__restrict__ out,
+                                                       Geo geo, uint32_t n_ch, uint64_t n_parts) {
+    constexpr uint32_t RPB = 1024 / D, LPR = D / 4;
+    const uint32_t G = (uint32_t)geo.G, GS = H / G, B = (uint32_t)geo.B;
+    const uint32_t ub = blockIdx.x / (64 / RPB);  // row block: (segment, KV head, qb)
+    const uint32_t r = blockIdx.x % (64 / RPB) * RPB + threadIdx.x / LPR;
+    const uint32_t qb = ub % n_cb, sg = ub / n_cb, g = sg % G, seg = sg / G;
+    const uint32_t nt = n_tok[seg], p0s = pos0[seg], qa = q_at[seg], tab = table_at[seg];
+    const uint32_t rr = qb * 64u + r, nrows = nt * GS;
+    // (segments that the attention refused and flagged wrote no partials)
+    if (nt == 0 || nt > max_tok || (uint64_t)p0s + nt - 1 > max_pos || (uint64_t)qa + nt > q_rows ||
+        (uint64_t)tab + (p0s + nt + B - 1) / B > n_table || rr >= nrows)
+        return;
+    const uint32_t n_wg = p0s + min(nt - 1, (qb * 64u + 63u) / GS) + 1;
+    const uint32_t tiles = (n_wg + 31) / 32;
+    const uint32_t d = threadIdx.x % LPR * 4;
+    const float *rows = ws + ((uint64_t)ub * n_ch * 64u + r) * D + d;
+    const float *ml = ws + n_parts * 64u * D + ((uint64_t)ub * n_ch * 64u + r) * 2;
+    float M = -INFINITY, L = 0.0f;
+    f4 O = f4{0.f, 0.f, 0.f, 0.f};
+    for (uint32_t c0 = 0; c0 < n_ch; c0 += 4) {
+        float mc[4], lc[4];
+        f4 oc[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) lr[i] = __shfl(l, 4 * (int)grp + i);
+        for (int k = 0; k < 4; k++) {
+            const uint32_t c = c0 + k;
+            const TileRange t = chunk_tiles(tiles, c < n_ch ? c : 0u, n_ch);
+            const bool live = c < n_ch && t.first < t.end;
+            mc[k] = live ? ml[(uint64_t)c * 128u] : -INFINITY;
+            lc[k] = live ? ml[(uint64_t)c * 128u + 1] : 0.0f;
+            oc[k] = live ? *(const f4 *)(rows + (uint64_t)c * 64u * D) : f4{0.f, 0.f, 0.f, 0.f};
+        }
+        float mn = M;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t rr = rw0 + 4 * grp + i;
-        if (rr >= nrows) continue;
-        const uint32_t tr = rr / GS, hr = rr % GS;
-        float *orow = out + ((uint64_t)(qa + tr) * H + (uint64_t)g * GS + hr) * D;
-        const float inv = 1.0f / lr[i];
+        for (int k = 0; k < 4; k++) mn = fmaxf(mn, mc[k]);
+        const float ms = mn == -INFINITY ? 0.0f : mn;
+        const float f0 = __builtin_amdgcn_exp2f(M - ms);  // (0 from -infinity)
+        L *= f0;
+        O *= f0;
 #pragma unroll
-        for (int j = 0; j < NDB; j++) orow[16 * j + col] = acc[j][i] * inv;
+        for (int k = 0; k < 4; k++) {
+            const float f = __builtin_amdgcn_exp2f(mc[k] - ms);  // 0: no tile that the row sees
+            L = fmaf(lc[k], f, L);
+#pragma unroll
+            for (int e = 0; e < 4; e++) O[e] = fmaf(oc[k][e], f, O[e]);
+        }
+        M = mn;
     }
+    const float inv = 1.0f / L;
+    *(f4 *)(out + ((uint64_t)(qa + rr / GS) * H + (uint64_t)g * GS + rr % GS) * D + d) = O * inv;
 }
 
 // Prefill, generic form: one wave per (segment, token, query head).
@@ -1130,12 +1242,59 @@ int check_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t ma
     return QVKV_OK;
 }
 
-hipError_t launch_prefill(const Geometry &g, const void *pool, uint64_t pool_blocks,
-                          const float *q, const uint32_t *blocks, uint64_t n_table,
-                          const uint32_t *table_at, const uint32_t *pos0, const uint32_t *q_at,
-                          const uint32_t *n_tok, uint32_t n_seg, uint32_t heads,
-                          uint32_t max_pos, uint32_t max_tok, uint64_t q_rows, float *out,
-                          int *err, hipStream_t s, bool f16_values) {
+// Which kernel a prefill launch runs.
+enum class PrefillForm { GENERIC, TILE, F16, Q8 };
+static PrefillForm prefill_form(const Geometry &g, bool f16_values) {
+    const bool q8 = g.dtype == QVKV_Q8_0;
+    if (!(g.D == 64 || g.D == 128 || g.D == 256)) return PrefillForm::GENERIC;
+    if (!q8 && (g.D == 64 || g.D == 128) && tune(KNOB_PREFILL_V2)) return PrefillForm::F16;
+    // f16_values: the q8_0 MFMA-throughput form, which holds dequantised values in f16
+    if (q8 && g.D == 128 && f16_values && tune(KNOB_PREFILL_Q8_FAST)) return PrefillForm::Q8;
+    return PrefillForm::TILE;
+}
+
+PrefillPlan plan_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t max_pos,
+                         uint32_t max_tok, bool f16_values) {
+    PrefillPlan p;
+    const PrefillForm form = prefill_form(g, f16_values);
+    if (form != PrefillForm::F16 && form != PrefillForm::Q8) return p;
+    // Chunks per row block: the count whose estimated time is least.  A CU holds 3
+    // workgroups (768 on the chip); a 32-position tile takes a workgroup about `tile_us`
+    // with 3 on its CU and 0.6 / 0.8 of that with one or two; each workgroup spends about
+    // 4 us outside its tiles, and a split launch 5 us more on its merge plus the partials'
+    // traffic (written and read once).  Measured at 2 k positions, f16, d = 128, in us by
+    // chunks 1 / 2 / 3 / 4 / 8: 32 row blocks 49 / 32 / 26 / 22 / 20, 128 blocks 51 / 36 /
+    // 33 / 31 / 41, 256 blocks 53 / 45 / 46 / 53 / 67, 512 blocks 65 / 83 / 81 / 92 / 134; a
+    // 512-token chunk at 8 k (256 blocks of 272 tiles) 188 -> 124 us with 3.
+    const uint64_t slots = 768;
+    const uint64_t blocks =
+        (uint64_t)n_seg * g.G * (((uint64_t)max_tok * (heads / (uint32_t)g.G) + 63) / 64);
+    const uint64_t tiles = ((uint64_t)max_pos + 32) / 32;
+    const double tile_us = (form == PrefillForm::Q8 ? 2.2 : 1.14) * (g.D / 128.0);
+    const int forced = tune(KNOB_PREFILL_CHUNKS);
+    double best = 0.0;
+    for (uint32_t n = 1; n <= PREFILL_MAX_CHUNKS; n++) {
+        if (n > 1 && (tiles < 2ull * n || blocks * n > 8 * slots) && forced == 0) break;
+        const uint64_t rem = blocks * n % slots;
+        const double rounds = (double)(blocks * n / slots) +
+                              (rem == 0 ? 0.0 : rem <= slots / 3 ? 0.6 : rem <= 2 * slots / 3 ? 0.8 : 1.0);
+        double us = rounds * ((double)((tiles + n - 1) / n) * tile_us + 4.0);
+        if (n > 1) us += 5.0 + (double)(blocks * n) * 64.0 * (g.D + 2) * 8.0 / 4e6;
+        if (n == 1 || (forced == 0 ? us < best : (int)n <= forced)) {
+            best = us;
+            p.n_chunks = n;
+        }
+    }
+    if (p.n_chunks > 1) p.ws_bytes = blocks * p.n_chunks * 64ull * (uint64_t)(g.D + 2) * 4ull;
+    return p;
+}
+
+hipError_t launch_prefill(const Geometry &g, const PrefillPlan &plan, const void *pool,
+                          uint64_t pool_blocks, const float *q, const uint32_t *blocks,
+                          uint64_t n_table, const uint32_t *table_at, const uint32_t *pos0,
+                          const uint32_t *q_at, const uint32_t *n_tok, uint32_t n_seg,
+                          uint32_t heads, uint32_t max_pos, uint32_t max_tok, uint64_t q_rows,
+                          float *out, void *ws, int *err, hipStream_t s, bool f16_values) {
     if (n_seg == 0 || max_tok == 0) return hipSuccess;
     const Geo geo = to_geo(g);
     const uint8_t *pp = (const uint8_t *)pool;
@@ -1151,32 +1310,40 @@ hipError_t launch_prefill(const Geometry &g, const void *pool, uint64_t pool_blo
         return hipGetLastError();
     }
     const uint32_t GS = heads / (uint32_t)g.G;
-    if (!q8 && (g.D == 64 || g.D == 128) && tune(KNOB_PREFILL_V2)) {
+    const PrefillForm form = prefill_form(g, f16_values);
+    if (form == PrefillForm::F16 || form == PrefillForm::Q8) {
         const uint32_t n_qb = (uint32_t)(((uint64_t)max_tok * GS + 63) / 64);
-        const unsigned grid2 = (unsigned)((uint64_t)n_seg * g.G * n_qb);
-        const unsigned pad = (unsigned)tune(KNOB_PREFILL_LDS_PAD);
-#define QV_PF2(DD, DMA, PS)                                                                    \
-    hipLaunchKernelGGL((k_prefill_f16<DD, DMA, PS>), dim3(grid2), dim3(256), pad, s, pp,         \
-                       pool_blocks, q, blocks, n_table, table_at, pos0, q_at, n_tok, n_seg,     \
-                       heads, max_pos, max_tok, q_rows, n_qb, out, geo, err)
+        const uint32_t n_ch = plan.n_chunks;
+        const uint64_t row_blocks = (uint64_t)n_seg * g.G * n_qb;
+        // groups of row blocks (row_block), and the parts that make their number a multiple of 8
+        const uint64_t groups = (uint64_t)n_seg * g.G * n_ch;
+        uint32_t n_sub = 1;
+        while (groups < 128 && groups * n_sub % 8 != 0 && n_sub * 2 <= n_qb) n_sub *= 2;
+        const unsigned grid2 = (unsigned)((groups * n_sub + 7) / 8 * 8 * ((n_qb + n_sub - 1) / n_sub));
+        const unsigned pad = form == PrefillForm::F16 ? (unsigned)tune(KNOB_PREFILL_LDS_PAD) : 0u;
+#define QV_PF2(KERNEL)                                                                         \
+    hipLaunchKernelGGL(KERNEL, dim3(grid2), dim3(256), pad, s, pp, pool_blocks, q, blocks,       \
+                       n_table, table_at, pos0, q_at, n_tok, n_seg, heads, max_pos, max_tok,    \
+                       q_rows, n_qb, out, geo, err, n_ch, n_sub, (float *)ws, row_blocks * n_ch)
         // P as one f16 (the default) or as high part + residual (knob prefill_exact_p=1)
         const bool ps = tune(KNOB_PREFILL_EXACT_P) != 0;
-        if (g.D == 64) { if (ps) QV_PF2(64, false, true); else QV_PF2(64, false, false); }
+        if (form == PrefillForm::Q8) QV_PF2((k_prefill_q8<128>));
+        else if (g.D == 64) { if (ps) QV_PF2((k_prefill_f16<64, false, true>)); else QV_PF2((k_prefill_f16<64, false, false>)); }
         else if (tune(KNOB_PREFILL_DMA)) {
-            if (ps) QV_PF2(128, true, true); else QV_PF2(128, true, false);
+            if (ps) QV_PF2((k_prefill_f16<128, true, true>)); else QV_PF2((k_prefill_f16<128, true, false>));
         } else {
-            if (ps) QV_PF2(128, false, true); else QV_PF2(128, false, false);
+            if (ps) QV_PF2((k_prefill_f16<128, false, true>)); else QV_PF2((k_prefill_f16<128, false, false>));
         }
 #undef QV_PF2
-        return hipGetLastError();
-    }
-    // f16_values: the q8_0 MFMA-throughput form, which holds dequantised values in f16
-    if (q8 && g.D == 128 && f16_values && tune(KNOB_PREFILL_Q8_FAST)) {
-        const uint32_t n_qb = (uint32_t)(((uint64_t)max_tok * GS + 63) / 64);
-        const unsigned grid3 = (unsigned)((uint64_t)n_seg * g.G * n_qb);
-        hipLaunchKernelGGL((k_prefill_q8<128>), dim3(grid3), dim3(256), 0, s, pp, pool_blocks, q,
-                           blocks, n_table, table_at, pos0, q_at, n_tok, n_seg, heads, max_pos,
-                           max_tok, q_rows, n_qb, out, geo, err);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess || n_ch == 1) return e;
+        const unsigned mgrid = (unsigned)(row_blocks * 64 / (1024 / g.D));
+#define QV_PM(DD)                                                                              \
+    hipLaunchKernelGGL(k_prefill_merge<DD>, dim3(mgrid), dim3(256), 0, s, (const float *)ws,     \
+                       n_table, table_at, pos0, q_at, n_tok, heads, max_pos, max_tok, q_rows,   \
+                       n_qb, out, geo, n_ch, row_blocks * n_ch)
+        if (g.D == 64) QV_PM(64); else QV_PM(128);
+#undef QV_PM
         return hipGetLastError();
     }
     const uint32_t n_cb = (uint32_t)(((uint64_t)max_tok * GS + 31) / 32);
