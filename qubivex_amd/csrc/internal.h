@@ -67,7 +67,7 @@ hipError_t launch_prelude(float *q, float *k, float *v, uint32_t s, uint32_t hea
 
 // Attention: the launch plan decides the split over the context and the workspace.
 struct AttnPlan {
-    int kind;           // 0: MFMA kernel, 1: generic kernel, 2: MFMA split by work
+    int kind;           // 0: MFMA kernel, 1: generic kernel, 2: MFMA split by work, 3: MFMA, wide workgroups
     uint32_t hc;        // head chunks of <= 8 query heads per KV head
     uint32_t n_chunks;  // context chunks per (item, kv head, head chunk); kind 2: workgroups
     uint32_t tpc;       // 16-position tiles per chunk
@@ -92,8 +92,9 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     X(COPY_U, "copy_u", 1)                                                                      \
     X(COPY_T, "copy_t", 64)                                                                     \
     X(ATTN_FULL, "attn_full", 512)              /* units from which a launch runs unsplit */    \
+    X(ATTN_WIDE, "attn_wide", -1)               /* tiles up to which units run wide; -1: rule */ \
     X(ATTN_STREAM, "attn_stream", 1)            /* 1: split by work, 0: context chunks */       \
-    X(ATTN_STREAM_WG, "attn_stream_wg", 768)                                                    \
+    X(ATTN_STREAM_WG, "attn_stream_wg", 0)      /* 0: by the launch's tiles */                  \
     X(STREAM_UNIT_COST, "stream_unit_cost", 8)  /* a unit's set-up cost in tiles */             \
     X(ATTN_TARGET, "attn_target", 1536)         /* context-chunk split: workgroups aimed at */  \
     X(FUSED_Q8, "fused_q8", 1)                  /* fused append + attention for q8_0 */         \

@@ -904,9 +904,9 @@ __global__ __launch_bounds__(T) void k_block_copy(uint8_t *__restrict__ pool,
     pool, pool_blocks, q, blocks, n_table, table_at, pos, n_items, H, max_pos, out, ws, hc_n,   \
         n_chunks, tpc, geo, err, nr
 
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS = false>
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS = false, int NW = 4>
 __device__ __forceinline__ void attn_body(QV_ATTN_PARAMS);
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS = false>
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS = false, int NW = 4>
 __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint64_t pool_blocks,
                                           const float *__restrict__ q,
                                           const uint32_t *__restrict__ blocks, uint32_t H,
@@ -948,7 +948,16 @@ void k_attn_mfma_w(QV_ATTN_PARAMS) {
     attn_body<D, Q8, NT, PK, false>(QV_ATTN_ARGS);
 }
 
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS>
+// Launches of few short units: one workgroup of 12 waves (d = 128) or 16 (d = 64) on each, so
+// that a CU which has a unit to itself streams it with all the waves its registers hold.
+constexpr int wide_waves(int D) { return D == 64 ? 16 : 12; }
+template <int D, bool Q8, bool PK, bool NR>
+__global__ __launch_bounds__(64 * wide_waves(D)) __attribute__((amdgpu_waves_per_eu(wide_waves(D) / 4)))
+void k_attn_wide(QV_ATTN_PARAMS) {
+    attn_body<D, Q8, true, PK, NR, true, wide_waves(D)>(QV_ATTN_ARGS);
+}
+
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS, int NW>
 __device__ __forceinline__ void attn_body(QV_ATTN_PARAMS) {
     const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
     const uint32_t GS = H / G;
@@ -986,11 +995,11 @@ __device__ __forceinline__ void attn_body(QV_ATTN_PARAMS) {
 
     const uint64_t oh0 = (uint64_t)item * H + (uint64_t)g * GS + hc * 8;
     if (n_chunks == 1) {
-        attn_unit<D, Q8, NT, PK, NR, IDS>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
+        attn_unit<D, Q8, NT, PK, NR, IDS, NW>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
                                  t_begin, t_end, out + oh0 * D, D, nullptr, 0, nr);
     } else {
         float *ml = ws + (uint64_t)n_items * H * n_chunks * D;
-        attn_unit<D, Q8, NT, PK, NR, IDS>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
+        attn_unit<D, Q8, NT, PK, NR, IDS, NW>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
                                  t_begin, t_end, ws + (oh0 * n_chunks + chunk) * D,
                                  (uint64_t)n_chunks * D, ml + (oh0 * n_chunks + chunk) * 2,
                                  (uint64_t)n_chunks * 2, nr);
@@ -999,10 +1008,10 @@ __device__ __forceinline__ void attn_body(QV_ATTN_PARAMS) {
 
 // One unit's attention: KV head g of item `item` (positions 0..n-1, table at `tab`), query
 // heads hc*8 .. hc*8+7 of its group, over 16-position tiles t_begin .. t_end-1 shared out to
-// the 4 waves.  Head hh's result goes to o_base[hh * o_stride + d]: the output (ml_base
+// the NW waves.  Head hh's result goes to o_base[hh * o_stride + d]: the output (ml_base
 // null) or, for part of the context, the unnormalised partial with its max and sum at
 // ml_base[hh * ml_stride] (log2 domain).
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS>
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS, int NW>
 __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint64_t pool_blocks,
                                           const float *__restrict__ q,
                                           const uint32_t *__restrict__ blocks, uint32_t H,
@@ -1011,8 +1020,8 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
                                           uint32_t t_end, float *o_base, uint64_t o_stride,
                                           float *ml_base, uint64_t ml_stride, NewRows nr) {
     constexpr int NJ = D / 16;  // MFMA steps over d
-    __shared__ float sm[4][8], sl[4][8];
-    __shared__ float so[4][8][D];
+    __shared__ float sm[NW][8], sl[NW][8];
+    __shared__ float so[NW][8][D];
     const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
     const uint32_t GS = H / G;
     const uint32_t lane = threadIdx.x & 63u;
@@ -1032,7 +1041,7 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
     __shared__ __attribute__((aligned(16))) float nrow[Q8 && NR ? 2 * D : 4];
     if constexpr (Q8 && NR) {
         const uint32_t t_last = (n - 1) / 16;
-        if (t_last >= t_begin && t_last < t_end && w == (t_last - t_begin) % 4u) {
+        if (t_last >= t_begin && t_last < t_end && w == (t_last - t_begin) % NW) {
             const uint64_t at = (uint64_t)item * geo.kv_out + (uint64_t)g * D;
 #pragma unroll
             for (int i = 0; i < (2 * D + 255) / 256; i++) {  // 64 lanes x 4 floats a load
@@ -1070,9 +1079,9 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
         // NR: the unit's last tile holds the appended position, patched from nrow
         const uint32_t t_last = NR ? (n - 1) / 16 : t_end;
         uint32_t ids = 0;
-        for (uint32_t tt = t_begin + w, k = 0; tt < t_end; tt += 4, k = (k + 1) & 63u) {
+        for (uint32_t tt = t_begin + w, k = 0; tt < t_end; tt += NW, k = (k + 1) & 63u) {
             if (k == 0) {
-                const uint32_t tl = tt + 4u * lane;
+                const uint32_t tl = tt + NW * lane;
                 ids = tl < t_end ? blocks[tab + tl * 16u / B] : 0u;
             }
             Tile<D, Q8> cur;
@@ -1100,9 +1109,9 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
         const uint32_t t_last = NR ? (n - 1) / 16 : t_end;
         uint32_t tt = t_begin + w;
         uint32_t ids = 0;
-        for (uint32_t k = 0; tt < t_end && tt != t_last; tt += 4, k = (k + 1) & 63u) {
+        for (uint32_t k = 0; tt < t_end && tt != t_last; tt += NW, k = (k + 1) & 63u) {
             if (IDS && k == 0) {
-                const uint32_t tl = tt + 4u * lane;
+                const uint32_t tl = tt + NW * lane;
                 ids = tl < t_end ? blocks[tab + tl * 16u / B] : 0u;
             }
             Tile<D, Q8> cur;
@@ -1156,18 +1165,18 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
     }
     __syncthreads();
 
-    // ---- merge the 4 waves; write the result or this chunk's partial
-    for (uint32_t idx = threadIdx.x; idx < 8u * D; idx += 256u) {
+    // ---- merge the waves; write the result or this chunk's partial
+    for (uint32_t idx = threadIdx.x; idx < 8u * D; idx += 64u * NW) {
         const uint32_t hh = idx / D, d = idx - hh * D;
         const uint32_t hi2 = hc * 8 + hh;
         if (hi2 >= GS) continue;
         float M = sm[0][hh];
 #pragma unroll
-        for (int x = 1; x < 4; x++) M = fmaxf(M, sm[x][hh]);
+        for (int x = 1; x < NW; x++) M = fmaxf(M, sm[x][hh]);
         const float Ms = M == -INFINITY ? 0.0f : M;
         float L = 0.0f, O = 0.0f;
 #pragma unroll
-        for (int x = 0; x < 4; x++) {
+        for (int x = 0; x < NW; x++) {
             const float f = sm[x][hh] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(sm[x][hh] - Ms);
             L = fmaf(sl[x][hh], f, L);
             O = fmaf(so[x][hh][d], f, O);
@@ -1186,15 +1195,144 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
 }
 
 
+// Tiles t0 .. t1-1 of one unit by one wave (attn_unit's tile loop over consecutive tiles), left
+// in LDS as the wave's unnormalised rows o[8][D] with their max m[8] (log2 domain) and sum l[8].
+// nrow: the wave's own 2 D floats for the new rows (q8_0 NR).
+template <int D, bool Q8, bool NT, bool PK, bool NR>
+__device__ __forceinline__ void attn_wave(const uint8_t *__restrict__ pool, uint64_t pool_blocks,
+                                          const float *__restrict__ q,
+                                          const uint32_t *__restrict__ blocks, uint32_t H,
+                                          const Geo &geo, int *err, uint32_t item, uint32_t g,
+                                          uint32_t hc, uint32_t n, uint32_t tab, uint32_t t0,
+                                          uint32_t t1, NewRows nr, float *so, float *sm, float *sl,
+                                          float *nrow) {
+    constexpr int NJ = D / 16;  // MFMA steps over d
+    const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
+    const uint32_t GS = H / G;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t c = lane & 15u, qg = lane >> 4;
+    const bool hi_col = c < 8;
+    const uint32_t hidx = PK ? (c & 3u) : hc * 8 + (c & 7u);  // query head within the group
+    const bool hvalid = hidx < GS;
+    const uint32_t sigma = (c >> 2) & 1u;
+    const uint32_t t_last = NR ? (n - 1) / 16 : t1;  // holds the appended position
+    if constexpr (Q8 && NR) {
+        if (t_last >= t0 && t_last < t1) {
+            const uint64_t at = (uint64_t)item * geo.kv_out + (uint64_t)g * D;
+#pragma unroll
+            for (int i = 0; i < (2 * D + 255) / 256; i++) {
+                const uint32_t e = 4u * (lane + 64u * i);
+                if (e < 2u * D)
+                    *(float4 *)(nrow + e) = *(const float4 *)(e < D ? nr.k + at + e
+                                                                    : nr.v + at + (e - D));
+            }
+        }
+    }
+    h4 qf[NJ];
+    {
+        const float qs = (1.0f / sqrtf((float)D)) * LOG2E_F;
+        const float *qrow = q + ((uint64_t)item * H + (uint64_t)g * GS + hidx) * D;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int d0 = 32 * (j >> 1) + 8 * (int)qg + 4 * (j & 1);
+            float4 x = hvalid ? *(const float4 *)(qrow + d0) : make_float4(0.f, 0.f, 0.f, 0.f);
+            qf[j] = h4{split_part(mul_rn(x.x, qs), hi_col), split_part(mul_rn(x.y, qs), hi_col),
+                       split_part(mul_rn(x.z, qs), hi_col), split_part(mul_rn(x.w, qs), hi_col)};
+        }
+    }
+    SoftmaxState<D> st;
+    st.m = -INFINITY;
+    st.l = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) st.acc[j] = f4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (Q8) {
+        uint32_t ids = 0;  // the table entries of the next 64 tiles, one per lane
+        for (uint32_t tt = t0, k = 0; tt < t1; tt++, k = (k + 1) & 63u) {
+            if (k == 0) {
+                const uint32_t tl = tt + lane;
+                ids = tl < t1 ? blocks[tab + tl * 16u / B] : 0u;
+            }
+            Tile<D, Q8> cur;
+            load_tile_of<D, Q8, NT>(cur, tt, __builtin_amdgcn_readlane(ids, k), pool, pool_blocks,
+                                    g, c, qg, geo, err);
+            if (NR && tt == t_last && cur.ok) {  // (the block is valid)
+                // the first head chunk also stores the rows
+                uint8_t *base = hc == 0 ? (uint8_t *)pool + (uint64_t)blocks[tab + (n - 1) / B] * geo.bb
+                                        : nullptr;
+                const uint64_t rowidx = (uint64_t)g * B + (n - 1) % B;
+                q8_patch_new_row<D>(cur, (n - 1) & 15u, nrow, nrow + D,
+                                    base ? base + geo.k_off + rowidx * D : nullptr,
+                                    base ? base + geo.ks_off + rowidx * (D / 32) * 2u : nullptr,
+                                    base ? base + geo.v_off + rowidx * D : nullptr,
+                                    base ? base + geo.vs_off + rowidx * (D / 32) * 2u : nullptr,
+                                    c, qg);
+            }
+            compute_tile<D, Q8, PK>(cur, st, qf, n, n, qg, hi_col, sigma);
+        }
+    } else {
+        uint32_t tt = t0;
+        asm volatile("" : "+v"(tt));  // a vector loop: see attn_unit
+        uint32_t id = blocks[tab + tt * 16u / B];
+        for (; tt < t1 && tt != t_last; tt++) {
+            Tile<D, Q8> cur;
+            load_tile_of<D, Q8, NT>(cur, tt, id, pool, pool_blocks, g, c, qg, geo, err);
+            // the next tile's table entry travels with this tile
+            if (tt + 1 < t1) id = blocks[tab + (tt + 1) * 16u / B];
+            compute_tile<D, Q8, PK>(cur, st, qf, n, n, qg, hi_col, sigma);
+        }
+        if (NR && tt < t1) {  // tt == t_last: position n - 1 comes from the new rows
+            Tile<D, Q8> cur;
+            load_tile_of<D, Q8, NT>(cur, tt, id, pool, pool_blocks, g, c, qg, geo, err);
+            if (cur.ok) {  // (the block is valid) the first head chunk also stores the rows
+                uint8_t *row = (uint8_t *)pool + (uint64_t)id * geo.bb +
+                               ((uint64_t)g * B + (n - 1) % B) * D * 2u;
+                const uint64_t at = (uint64_t)item * geo.kv_out + (uint64_t)g * D;
+                patch_new_row<D>(cur, (n - 1) & 15u, nr.k + at, nr.v + at, row + geo.k_off,
+                                 row + geo.v_off, c, qg, hc == 0);
+            }
+            compute_tile<D, Q8, PK>(cur, st, qf, n, n, qg, hi_col, sigma);
+        }
+    }
+    float l = st.l;
+    f4 *acc = st.acc;
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float o = __shfl_xor(acc[j][i], 32);
+            acc[j][i] = Q8 ? acc[j][i] + o : split_sum32(acc[j][i], o);
+        }
+    if (qg == 0 && c < 8) {
+        sm[c] = st.m;
+        sl[c] = l;
+    }
+    if (qg < 2) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int d = Q8 ? 32 * (j >> 1) + 2 * (int)c + (j & 1) : (int)c * (D / 16) + j;
+            if (PK && qg != (uint32_t)((j >> 1) & 1)) continue;
+#pragma unroll
+            for (int i = 0; i < 4; i++) so[(PK ? i : 4 * qg + i) * D + d] = acc[j][i];
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------------
 // Decode attention split by work, for launches with few units (one layer of a decode step
-// in model order): the slots of every item, unit-major, are shared out evenly to the P
-// workgroups, so ragged contexts leave no partial rounds of workgroups.  A unit holds
-// `ucost` set-up slots (no tiles: its fixed cost in tile-equivalents) and then one slot
-// per 16-position tile; a workgroup whose range holds only set-up slots of a unit skips it.  Each
-// workgroup works through its range unit by unit: a unit wholly inside the range is
-// written out directly; a unit cut by a range boundary leaves a partial in the
-// workgroup's slot 0 (its first unit) or 1 (its last), merged by k_attn_stream_merge.
+// in model order): the slots of every item, unit-major, are shared out evenly to the 4 P
+// waves of P workgroups, so ragged contexts leave no partial rounds.  A unit holds `ucost`
+// set-up slots (no tiles: its fixed cost in tile-equivalents) and then one slot
+// per 16-position tile; a wave whose range holds only set-up slots of a unit skips it.  Each
+// wave works through its range unit by unit and on its own: no barrier until its range is
+// done, and consecutive tiles.  A unit wholly inside a wave's range is written out by it;
+// parts of one unit held by several waves of the workgroup are merged in LDS at the end, and
+// a unit cut by the workgroup's own range leaves a partial in the workgroup's slot 0 (its
+// first unit) or 1 (its last), merged by k_attn_stream_merge.  The bookkeeping is restated
+// in tests/test_attention_split.py.
+// A launch streams at 6.5-6.7 TB/s (f16, d = 128) after about 15 us of launch, prefix
+// sums, first tiles and merge: 64 units of 2176 / 8704 positions 26 / 59 us.
 // Each workgroup computes the units' prefix sums itself from pos (n_items <= 2048).
 // Workspace: partials [P][2][8][D], their (max, sum) [P][2][8][2], the prefix sums
 // [n_items + 1] (u64), then at the next 16-byte boundary one record per unit for the
@@ -1219,7 +1357,7 @@ __device__ __forceinline__ void stream_prefix(uint64_t *cum, const uint32_t *__r
                                               uint64_t n_table, uint32_t n_items,
                                               uint32_t max_pos, uint32_t per_unit_heads,
                                               uint32_t B, uint32_t ucost, int *err) {
-    __shared__ uint64_t part[256];
+    __shared__ uint64_t part[4];
     const uint32_t tid = threadIdx.x;
     const uint32_t per = (n_items + 255) / 256;  // <= 8
     uint64_t loc[8], sum = 0;
@@ -1240,22 +1378,24 @@ __device__ __forceinline__ void stream_prefix(uint64_t *cum, const uint32_t *__r
         loc[k] = v;
         sum += v;
     }
-    part[tid] = sum;
-    __syncthreads();
-    for (uint32_t off = 1; off < 256; off <<= 1) {
-        const uint64_t v = tid >= off ? part[tid - off] : 0;
-        __syncthreads();
-        part[tid] += v;
-        __syncthreads();
+    // a scan within each wave, then the waves' totals
+    uint64_t incl = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint64_t v = __shfl_up(incl, off);
+        if ((tid & 63u) >= (uint32_t)off) incl += v;
     }
-    uint64_t base = tid ? part[tid - 1] : 0;
+    if ((tid & 63u) == 63u) part[tid >> 6] = incl;
+    __syncthreads();
+    uint64_t base = incl - sum;
+    for (uint32_t k = 0; k < tid >> 6; k++) base += part[k];
 #pragma unroll
     for (uint32_t k = 0; k < 8; k++) {
         const uint32_t i = tid * per + k;
         if (k < per && i < n_items) cum[i] = base;
         base += loc[k];
     }
-    if (tid == 0) cum[n_items] = part[255];
+    if (tid == 255) cum[n_items] = base;
     __syncthreads();
 }
 
@@ -1285,14 +1425,19 @@ __device__ __forceinline__ uint64_t uni(uint64_t v) {
 
 template <int D, bool Q8, bool NT, bool PK, bool NR>
 __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
-    __shared__ uint64_t cum[STREAM_MAX_ITEMS + 1];
+    constexpr uint32_t NO_UNIT = 0xffffffffu;
+    extern __shared__ __attribute__((aligned(16))) uint64_t cum[];  // [n_items + 1]
+    // partials of the waves' cut units: slot 2 wave (its first unit) and 2 wave + 1 (its last)
+    __shared__ __attribute__((aligned(16))) float so[8][8][D];
+    __shared__ float sm[8][8], sl[8][8];
+    __shared__ uint32_t seg_unit[8], seg_ends[8], seg_units[4];
+    __shared__ __attribute__((aligned(16))) float nrow[4][Q8 && NR ? 2 * D : 4];
     const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
     const uint32_t GS = H / G;
     const uint32_t upi = G * hc_n;  // units per item
     stream_prefix(cum, pos, table_at, n_table, n_items, max_pos, upi, B, ucost, err);
     const uint64_t T = uni(cum[n_items]);
     const uint32_t P = gridDim.x, w = blockIdx.x;
-    const uint64_t s0 = (uint64_t)w * T / P, s1 = (uint64_t)(w + 1) * T / P;
     float *ml = ws + (uint64_t)P * 2 * 8 * D;
     if (w == 0) {  // the prefix sums and the units' records, for the merge
         uint64_t *wc = (uint64_t *)(ml + (uint64_t)P * 2 * 8 * 2);
@@ -1317,7 +1462,12 @@ __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
             rec[u] = r;
         }
     }
-    bool first = true;
+    // ---- the wave's share, unit by unit
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t v4 = 4ull * w + wv;
+    const uint64_t s0 = v4 * T / (4ull * P), s1 = (v4 + 1) * T / (4ull * P);
+    if ((threadIdx.x & 63u) < 2u) seg_unit[2 * wv + (threadIdx.x & 63u)] = NO_UNIT;
+    uint32_t n_units = 0;
     for (uint64_t x = s0; x < s1;) {
         const uint32_t item = uni(stream_item(cum, n_items, x));
         const uint64_t c0 = uni(cum[item]);
@@ -1335,29 +1485,83 @@ __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
         const uint32_t t0 = x > tiles_at ? (uint32_t)(x - tiles_at) : 0u;
         const uint32_t t1 = (uint32_t)(seg_end - tiles_at);
         const uint32_t n = uni(pos[item]) + 1, tab = uni(table_at[item]);
-        const uint64_t oh0 = (uint64_t)item * H + (uint64_t)g * GS + hc * 8;
-        if (t0 == 0 && seg_end == unit_end) {
-            attn_unit<D, Q8, NT, PK, NR>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n,
-                                     tab, t0, t1, out + oh0 * D, D, nullptr, 0, nr);
-        } else {
-            const uint64_t slot = 2ull * w + (first ? 0u : 1u);
-            attn_unit<D, Q8, NT, PK, NR>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n,
-                                     tab, t0, t1, ws + slot * 8 * D, D, ml + slot * 8 * 2, 2,
-                                     nr);
+        const bool starts = t0 == 0, ends = seg_end == unit_end;
+        // a unit that the wave holds whole goes out from its second slot at once (that slot
+        // is taken only by the wave's last unit)
+        const bool whole = starts && ends;
+        const uint32_t slot = 2 * wv + (whole || n_units != 0 ? 1u : 0u);
+        attn_wave<D, Q8, NT, PK, NR>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
+                                     t0, t1, nr, &so[slot][0][0], sm[slot], sl[slot], nrow[wv]);
+        if (whole) {
+            lds_order();
+            float *orow = out + ((uint64_t)item * H + (uint64_t)g * GS + hc * 8) * D;
+            const uint32_t heads = min(GS - hc * 8, 8u);
+            for (uint32_t idx = threadIdx.x & 63u; idx < heads * (D / 4); idx += 64) {
+                const f4 o = *(const f4 *)&so[slot][0][4 * idx];
+                st_g((f4 *)(orow + 4 * idx), o / sl[slot][idx / (D / 4)]);
+            }
+            lds_order();
+        } else if ((threadIdx.x & 63u) == 0) {
+            seg_unit[slot] = item * upi + ul;
+            seg_ends[slot] = (starts ? 1u : 0u) | (ends ? 2u : 0u);
         }
-        first = false;
+        n_units++;
         x = seg_end;
+    }
+    if ((threadIdx.x & 63u) == 0) seg_units[wv] = n_units;
+    __syncthreads();
+
+    // ---- units cut between waves: parts of one unit are consecutive.  A unit whose first
+    // and last tile are both here is finished; one cut by the workgroup's own range leaves
+    // its partial in slot 0 (the workgroup's first unit) or 1.
+    for (uint32_t i = 0; i < 8;) {
+        const uint32_t u = uni(seg_unit[i]);
+        if (u == NO_UNIT) {
+            i++;
+            continue;
+        }
+        uint32_t last = i, j = i + 1;
+        for (; j < 8; j++) {
+            const uint32_t uj = uni(seg_unit[j]);
+            if (uj == u) last = j;
+            else if (uj != NO_UNIT) break;
+        }
+        bool first = (i & 1u) == 0;
+        for (uint32_t k = 0; k < i / 2; k++) first = first && uni(seg_units[k]) == 0;
+        const bool done = (uni(seg_ends[i]) & 1u) && (uni(seg_ends[last]) & 2u);
+        const uint32_t item = u / upi, ul = u % upi, hc = ul % hc_n;
+        const uint32_t heads = min(GS - hc * 8, 8u);
+        float *orow = out + ((uint64_t)item * H + (uint64_t)(ul / hc_n) * GS + hc * 8) * D;
+        const uint64_t slot = 2ull * w + (first ? 0u : 1u);
+        for (uint32_t idx = threadIdx.x; idx < heads * D; idx += 256u) {
+            const uint32_t hh = idx / D;
+            float M = -INFINITY;
+            for (uint32_t k = i; k <= last; k++)
+                if (seg_unit[k] == u) M = fmaxf(M, sm[k][hh]);
+            const float Ms = M == -INFINITY ? 0.0f : M;
+            float L = 0.0f, O = 0.0f;
+            for (uint32_t k = i; k <= last; k++) {
+                if (seg_unit[k] != u) continue;
+                const float f = sm[k][hh] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(sm[k][hh] - Ms);
+                L = fmaf(sl[k][hh], f, L);
+                O = fmaf(so[k][0][idx], f, O);
+            }
+            if (done) {
+                orow[idx] = O / L;
+            } else {
+                ws[slot * 8 * D + idx] = O;
+                if (idx % D == 0) {
+                    ml[(slot * 8 + hh) * 2] = M;
+                    ml[(slot * 8 + hh) * 2 + 1] = L;
+                }
+            }
+        }
+        i = j;
     }
 }
 
 template <int D, bool Q8, bool NT, bool PK>
 __global__ __launch_bounds__(256) void k_attn_stream(QV_STREAM_PARAMS) {
-    attn_stream_body<D, Q8, NT, PK, false>(pool, pool_blocks, q, blocks, n_table, table_at, pos, n_items,
-                                    H, max_pos, out, ws, hc_n, ucost, geo, err, nr);
-}
-template <int D, bool Q8, bool NT, bool PK, int W>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W)))
-void k_attn_stream_w(QV_STREAM_PARAMS) {
     attn_stream_body<D, Q8, NT, PK, false>(pool, pool_blocks, q, blocks, n_table, table_at, pos, n_items,
                                     H, max_pos, out, ws, hc_n, ucost, geo, err, nr);
 }
@@ -1379,17 +1583,19 @@ void k_attn_stream_q8nr(QV_STREAM_PARAMS) {
                                               err, nr);
 }
 
-// Merge for k_attn_stream: block = one (item, query head), D threads.  The unit's
+// Merge for k_attn_stream: block = one (item, query head), D threads per slice of the unit's
+// partials (blockDim.x = D * slices).  The unit's
 // range [a, b) of the work order lies in workgroups w0 .. w1 (its StreamRec); with
 // w0 == w1 it was written out whole.  Workgroup w's partial of it is in slot 1 when the
 // unit starts inside w's range after its first unit, else in slot 0; workgroups between
 // them with an empty range (more workgroups than tiles) hold none.  The same bookkeeping
 // is restated in tests/test_attention_split.py and checked there on random shapes.
-__global__ __launch_bounds__(256) void k_attn_stream_merge(const float *__restrict__ ws,
-                                                           uint32_t n_items, uint32_t H,
-                                                           uint32_t G, uint32_t hc_n,
-                                                           uint32_t P, uint32_t D,
-                                                           float *__restrict__ out) {
+__global__ __launch_bounds__(1024) void k_attn_stream_merge(const float *__restrict__ ws,
+                                                            uint32_t n_items, uint32_t H,
+                                                            uint32_t G, uint32_t hc_n,
+                                                            uint32_t P, uint32_t D,
+                                                            float *__restrict__ out) {
+    __shared__ float xm[16], xl[16], xo[1024];
     const uint32_t oh = blockIdx.x;
     const uint32_t item = oh / H, h = oh % H;
     if (item >= n_items) return;
@@ -1407,46 +1613,57 @@ __global__ __launch_bounds__(256) void k_attn_stream_merge(const float *__restri
     auto empty = [&](uint32_t w) {
         return T < P && (uint64_t)w * T / P == (uint64_t)(w + 1) * T / P;
     };
-    // The unit's partials are read 4 workgroups at a time, every load of a group issued
-    // before any is used (one memory round trip per group instead of one per partial);
-    // they are combined in workgroup order.
     auto slot_of = [&](uint32_t w) { return 2ull * w + (w == w0 ? r.s0 : 0u); };
-    float M = -INFINITY;
-    for (uint32_t wb = w0; wb <= w1; wb += 4) {
-        float mc[4];
+    // Slice y takes workgroups w0 + y per .. of the range, 8 at a time with every load of a
+    // group issued before any is used (one memory round trip per group), in workgroup order.
+    const uint32_t slices = blockDim.x / D, y = threadIdx.x / D, d = threadIdx.x % D;
+    const uint32_t per = (w1 - w0 + slices) / slices;  // ceil((w1 - w0 + 1) / slices)
+    const uint32_t wa = w0 + y * per, wz = min(wa + per, w1 + 1);
+    float M = -INFINITY, L = 0.0f, O = 0.0f;
+    for (uint32_t wb = wa; wb < wz; wb += 8) {
+        float mc[8], lc[8], oc[8];
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
+        for (int k = 0; k < 8; k++) {
             const uint32_t w = wb + k;
-            mc[k] = w <= w1 && !empty(w) ? ml[(slot_of(w) * 8 + hh) * 2] : -INFINITY;
+            const bool live = w < wz && !empty(w);
+            const uint64_t slot = live ? slot_of(w) : 0u;
+            mc[k] = live ? ml[(slot * 8 + hh) * 2] : -INFINITY;
+            lc[k] = live ? ml[(slot * 8 + hh) * 2 + 1] : 0.0f;
+            oc[k] = live ? ws[(slot * 8 + hh) * D + d] : 0.0f;
         }
+        float mn = M;
 #pragma unroll
-        for (int k = 0; k < 4; k++) M = fmaxf(M, mc[k]);
-    }
-    const float Ms = M == -INFINITY ? 0.0f : M;
-    for (uint32_t d = threadIdx.x; d < D; d += blockDim.x) {
-        float L = 0.0f, O = 0.0f;
-        for (uint32_t wb = w0; wb <= w1; wb += 4) {
-            float mc[4], lc[4], oc[4];
-            bool live[4];
+        for (int k = 0; k < 8; k++) mn = fmaxf(mn, mc[k]);
+        const float ms = mn == -INFINITY ? 0.0f : mn;
+        const float f0 = __builtin_amdgcn_exp2f(M - ms);  // (0 from -infinity)
+        L *= f0;
+        O *= f0;
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint32_t w = wb + k;
-                live[k] = w <= w1 && !empty(w);
-                const uint64_t slot = live[k] ? slot_of(w) : 0u;
-                mc[k] = live[k] ? ml[(slot * 8 + hh) * 2] : -INFINITY;
-                lc[k] = live[k] ? ml[(slot * 8 + hh) * 2 + 1] : 0.0f;
-                oc[k] = live[k] ? ws[(slot * 8 + hh) * D + d] : 0.0f;
-            }
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                if (!live[k]) continue;
-                const float f = mc[k] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mc[k] - Ms);
-                L = fmaf(lc[k], f, L);
-                O = fmaf(oc[k], f, O);
-            }
+        for (int k = 0; k < 8; k++) {
+            const float f = __builtin_amdgcn_exp2f(mc[k] - ms);  // 0 for no partial
+            L = fmaf(lc[k], f, L);
+            O = fmaf(oc[k], f, O);
         }
-        out[(uint64_t)oh * D + d] = O / L;
+        M = mn;
     }
+    if (slices > 1) {
+        if (d == 0) {
+            xm[y] = M;
+            xl[y] = L;
+        }
+        xo[threadIdx.x] = O;
+        __syncthreads();
+        if (y != 0) return;
+        for (uint32_t k = 0; k < slices; k++) M = fmaxf(M, xm[k]);
+        const float ms = M == -INFINITY ? 0.0f : M;
+        L = O = 0.0f;
+        for (uint32_t k = 0; k < slices; k++) {
+            const float f = __builtin_amdgcn_exp2f(xm[k] - ms);
+            L = fmaf(xl[k], f, L);
+            O = fmaf(xo[k * D + d], f, O);
+        }
+    }
+    out[(uint64_t)oh * D + d] = O / L;
 }
 
 // Merge of context-chunk partials: block = one (item, query head), D threads.
@@ -1784,18 +2001,43 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     }
     const uint64_t units = (uint64_t)n_items * g.G * p->hc;
     const uint64_t max_tiles = ((uint64_t)max_pos + 1 + 15) / 16;
-    // workgroups to aim for: 8 per CU keeps all 256 CUs busy
-    // Launches too small to fill the chip with one workgroup per unit (below 2 per CU) are
-    // split.  By work (k_attn_stream, the default): every workgroup gets an equal share
-    // of the (unit, tile) pairs, whatever the contexts; 768 workgroups (3 per CU, one
-    // round).  Measured per layer of cfg2 (256 ragged units): 4.21 TB/s, against 3.77 for
-    // the best context-chunk split and 3.98 / 3.48 with 512 / 1024 workgroups.  Launches of
-    // 512 units and more (a layer of 128 x 8k, or of cfg3) run best unsplit: 6.0 and 4.8
-    // TB/s, against 5.7 and 3.3-4.3 split by work.
     const uint64_t full = (uint64_t)tune(KNOB_ATTN_FULL);
+    const bool q8 = g.dtype == QVKV_Q8_0;
+    // Few short units: a wide workgroup each, in one launch.  A CU draws about 37 GB/s from
+    // HBM however many waves it has, so longer contexts are spread over the chip below, at
+    // the price of a merge launch.  Measured in us per call in a graph, wide / split, f16
+    // d = 128: 8 units of 512 positions 13.2 / 15.3, of 1024 20.4 / 15.9; 256 units of
+    // 256-1024 23.3 / 28.3, of 512-2048 40.2 / 41.5; d = 64: 8 units of 1024 11.3 / 12.4, of 2048
+    // 20.6 / 12.5; q8_0 d = 128: 8 units of 1024 17.2 / 17.3, 256 units of 512-2048 28.4 / 34.5.
+    const uint64_t base = q8 ? (g.D == 64 ? 88 : 64) : (g.D == 64 ? 64 : 40);
+    // (a caller that sets the split's own knobs gets the split)
+    const bool split_set = full != (uint64_t)kKnobDefault[KNOB_ATTN_FULL] ||
+                           tune(KNOB_ATTN_STREAM) != 1 || tune(KNOB_ATTN_STREAM_WG) > 0;
+    const int wide = tune(KNOB_ATTN_WIDE);
+    const uint64_t wide_tiles = wide >= 0 ? (uint64_t)wide : split_set ? 0 : units >= 128 ? 2 * base : base;
+    if (units < full && units <= 256 && g.D != 256 && max_tiles <= wide_tiles) {
+        p->kind = 3;
+        return QVKV_OK;
+    }
+    // Other launches too small to fill the chip with one workgroup per unit (below 2 per CU)
+    // are split.  By work (k_attn_stream, the default): every wave gets an equal share
+    // of the (unit, tile) pairs, whatever the contexts.  One workgroup per CU (256) while a wave
+    // has few tiles (fewer partials to merge: one sequence of 32 k, 4 KV heads, 28.7 us against
+    // 30.3 with 512 and 32.9 with 768), two from 16384 tiles of 8 KiB (a ragged cfg2-like layer
+    // 55.6 us, 57.3 with 256, 55.9 with 768) or 4096 smaller ones (d = 64, 64 units of 2048
+    // 18.2 against 20.3), and three for large q8_0 launches, whose tiles cost more arithmetic
+    // (256 units of 1024-4096 52.1 us, 53.2 with 512, 72.9 with 256).  d = 256 runs one workgroup
+    // per CU (its registers): 128 units of 1024-4096 82 us with 256, 94 with 512, 112 with 768;
+    // q8_0 73, 91, 108.  Launches of 512 units
+    // and more (a layer of 128 x 8k, or of cfg3) run best unsplit: 6.0 and 4.8 TB/s, against
+    // 5.7 and 3.3-4.3 split by work.
     if (tune(KNOB_ATTN_STREAM) != 0 && units < full && n_items <= STREAM_MAX_ITEMS) {
         const uint64_t work = units * max_tiles;  // bound: the actual work is known on the device
-        uint64_t wgs = (uint64_t)tune(KNOB_ATTN_STREAM_WG);
+        const bool big = !q8 && g.D >= 128;       // tiles of 8 KiB and more
+        uint64_t wgs = g.D == 256      ? 256
+                       : work >= 16384 ? (q8 ? 768 : 512)
+                                       : (work >= 4096 && !big ? 512 : 256);
+        if (tune(KNOB_ATTN_STREAM_WG) > 0) wgs = (uint64_t)tune(KNOB_ATTN_STREAM_WG);
         if (wgs > (work + 3) / 4) wgs = (work + 3) / 4;  // at least a tile per wave
         if (wgs < 1) wgs = 1;
         p->kind = 2;
@@ -1907,19 +2149,15 @@ hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *po
     if (p.kind == 2) {
         const unsigned P = p.n_chunks;
 #define QV_AS(DD, QQ, PK)                                                                       \
-    hipLaunchKernelGGL((k_attn_stream<DD, QQ, true, PK>), dim3(P), dim3(256), 0, s, pp,          \
+    hipLaunchKernelGGL((k_attn_stream<DD, QQ, true, PK>), dim3(P), dim3(256), (n_items + 1) * 8, s, pp,          \
                        pool_blocks, q, blocks, n_table, table_at, pos, n_items, heads, max_pos,  \
                        out, wsf, p.hc, p.ucost, geo, err, nr)
 #define QV_AS_NR(DD)                                                                            \
-    hipLaunchKernelGGL((k_attn_stream_nr<DD>), dim3(P), dim3(256), 0, s,                        \
+    hipLaunchKernelGGL((k_attn_stream_nr<DD>), dim3(P), dim3(256), (n_items + 1) * 8, s,                        \
                        pp, pool_blocks, q, blocks, n_table, table_at, pos, n_items, heads,      \
                        max_pos, out, wsf, p.hc, p.ucost, geo, err, nr)
-#define QV_AS_W4(DD, QQ, PK)                                                                    \
-    hipLaunchKernelGGL((k_attn_stream_w<DD, QQ, true, PK, 4>), dim3(P), dim3(256), 0, s, pp,     \
-                       pool_blocks, q, blocks, n_table, table_at, pos, n_items, heads, max_pos,  \
-                       out, wsf, p.hc, p.ucost, geo, err, nr)
 #define QV_AS_Q8NR(DD, PK)                                                                      \
-    hipLaunchKernelGGL((k_attn_stream_q8nr<DD, PK>), dim3(P), dim3(256), 0, s, pp, pool_blocks,  \
+    hipLaunchKernelGGL((k_attn_stream_q8nr<DD, PK>), dim3(P), dim3(256), (n_items + 1) * 8, s, pp, pool_blocks,  \
                        q, blocks, n_table, table_at, pos, n_items, heads, max_pos, out, wsf,    \
                        p.hc, p.ucost, geo, err, nr)
         if (q8 && nr.k) {
@@ -1931,13 +2169,9 @@ hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *po
             else if (pk) QV_AS(64, true, true);
             else QV_AS(64, true, false);
         } else if (g.D == 128) {
-            if (!q8) {
-                if (nr.k) QV_AS_NR(128);
-                else if (w4) QV_AS_W4(128, false, false);
-                else QV_AS(128, false, false);
-            }
-            else if (pk) { if (w4) QV_AS_W4(128, true, true); else QV_AS(128, true, true); }
-            else { if (w4) QV_AS_W4(128, true, false); else QV_AS(128, true, false); }
+            if (!q8) { if (nr.k) QV_AS_NR(128); else QV_AS(128, false, false); }
+            else if (pk) QV_AS(128, true, true);
+            else QV_AS(128, true, false);
         } else {
             if (!q8) { if (nr.k) QV_AS_NR(256); else QV_AS(256, false, false); }
             else if (pk) QV_AS(256, true, true);
@@ -1945,13 +2179,33 @@ hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *po
         }
 #undef QV_AS_Q8NR
 #undef QV_AS_NR
-#undef QV_AS_W4
 #undef QV_AS
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_attn_stream_merge, dim3(n_items * heads), dim3(g.D), 0, s,
+        // slices of about 8 partials each, by the launch's mean partials per unit
+        const uint64_t per_unit = P / ((uint64_t)n_items * g.G * p.hc) + 1;
+        uint32_t slices = 1;
+        while (slices * 8 < per_unit && slices * 2 * g.D <= 1024) slices *= 2;
+        hipLaunchKernelGGL(k_attn_stream_merge, dim3(n_items * heads), dim3(g.D * slices), 0, s,
                            (const float *)ws, n_items, heads, (uint32_t)g.G, p.hc, P,
                            (uint32_t)g.D, out);
+        return hipGetLastError();
+    }
+    if (p.kind == 3) {
+        const unsigned units = (unsigned)((uint64_t)n_items * g.G * p.hc);
+#define QV_AW(DD, QQ, PK, NR)                                                                   \
+    hipLaunchKernelGGL((k_attn_wide<DD, QQ, PK, NR>), dim3(units), dim3(64 * wide_waves(DD)), 0, s, \
+                       pp, pool_blocks, q, blocks, n_table, table_at, pos, n_items, heads,      \
+                       max_pos, out, wsf, p.hc, 1u, 0xffffffffu, geo, err, nr)
+#define QV_AW_NR(DD, QQ, PK)                                                                    \
+    do { if (nr.k) QV_AW(DD, QQ, PK, true); else QV_AW(DD, QQ, PK, false); } while (0)
+#define QV_AW_D(DD)                                                                             \
+    do { if (!q8) QV_AW_NR(DD, false, false); else if (pk) QV_AW_NR(DD, true, true);             \
+         else QV_AW_NR(DD, true, false); } while (0)
+        if (g.D == 64) QV_AW_D(64); else QV_AW_D(128);
+#undef QV_AW_D
+#undef QV_AW_NR
+#undef QV_AW
         return hipGetLastError();
     }
     const uint64_t grid = (uint64_t)n_items * g.G * p.hc * p.n_chunks;

@@ -120,3 +120,67 @@ def test_the_check_catches_a_slot_rule_that_ignores_set_up_slots():
                        for w in range(w0, w1 + 1) if w * T // P != (w + 1) * T // P}
                 wrong += old != {s for _, s, _, _ in written[(item, ul)]}
     assert wrong > 0
+
+
+def waves(tiles, upi, P, cost):
+    """What each wave of each workgroup does: wave v of 4 P takes [floor(v T / 4P), ..); a unit it
+    holds whole goes out at once, a part of one to its LDS slot 0 (its first unit) or 1; then the
+    workgroup merges consecutive parts of one unit, finishing it or leaving one partial."""
+    cum = [0]
+    for t in tiles:
+        cum.append(cum[-1] + (t + cost) * upi)
+    T, W, written = cum[-1], 4 * P, {}
+    for w in range(P):
+        seg, units = [None] * 8, [0] * 4
+        for k in range(4):
+            x, s1 = (4 * w + k) * T // W, (4 * w + k + 1) * T // W
+            while x < s1:
+                item = max(i for i in range(len(tiles)) if cum[i] <= x < cum[i + 1])
+                per = (cum[item + 1] - cum[item]) // upi
+                ul = (x - cum[item]) // per
+                at, uend = cum[item] + ul * per + cost, cum[item] + (ul + 1) * per
+                end = min(uend, s1)
+                if end > at:
+                    t0, t1 = max(x - at, 0), end - at
+                    starts, ends = t0 == 0, end == uend
+                    if starts and ends:
+                        written.setdefault((item, ul), []).append(("out", None, t0, t1))
+                    else:
+                        slot = 2 * k + (1 if units[k] else 0)
+                        assert seg[slot] is None  # a slot holds one part
+                        seg[slot] = ((item, ul), starts, ends, t0, t1)
+                    units[k] += 1
+                x = end
+        i = 0
+        while i < 8:
+            if seg[i] is None:
+                i += 1
+                continue
+            u, last, j = seg[i][0], i, i + 1
+            while j < 8 and (seg[j] is None or seg[j][0] == u):
+                last = j if seg[j] is not None else last
+                j += 1
+            parts = [p for p in seg[i:last + 1] if p is not None]
+            assert all(a[4] == b[3] for a, b in zip(parts, parts[1:]))
+            first = i % 2 == 0 and not any(units[:i // 2])
+            done = seg[i][1] and seg[last][2]
+            written.setdefault(u, []).append(("out" if done else "part", None if done else 2 * w + (not first),
+                                              parts[0][3], parts[-1][4]))
+            i = j
+    return cum, T, written
+
+
+@pytest.mark.parametrize("cost", [0, 1, 8, 40])
+@pytest.mark.parametrize("seed", range(4))
+def test_waves_leave_what_the_workgroup_level_split_says(seed, cost):
+    """The wave-level shares give each workgroup the same units, tile ranges and slots as one
+    share per workgroup, so the merge's rule above reads exactly what they write."""
+    r = random.Random(seed * 10 + cost)
+    for _ in range(10):
+        tiles = [r.randint(1, 300) for _ in range(r.randint(1, 30))]
+        upi = r.choice([1, 2, 4, 8, 16])
+        P = r.choice([1, 2, 7, 64, 256, 512, sum(tiles) * upi + 5])
+        cum, T, got = waves(tiles, upi, P, cost)
+        _, _, want = split(tiles, upi, P, cost)
+        for u in want:  # a unit that one workgroup holds whole may be finished in either way
+            assert sorted(got[u], key=lambda p: p[2]) == sorted(want[u], key=lambda p: p[2]), u
