@@ -135,14 +135,17 @@ __global__ __launch_bounds__(256) void k_prefill_mfma(QV_PREFILL_PARAMS) {
 
 // ---------------------------------------------------------------------------------
 // Paged prefill attention, f16 pools, d = 64 or 128: the MFMA-throughput form.
+// (d = 64 streams its tiles like d = 128 at 4 workgroups per CU, in place of the
+// register-staged form: 16 chunks of 512 tokens at 8 k positions, one layer, 8 KV heads, 32
+// query heads, 1541 -> 890 us = 635 TFLOP/s useful; a 512-token prompt 19.8 -> 14 us.)
 // Workgroup = (segment, KV head, block of 64 query rows); row r = token j * GS + head h.
 // The 4 waves stage 32-position K/V tiles once in LDS and each wave computes 16 query
 // rows with v_mfma_f32_16x16x32_f16.  Two ways to stage (the math is shared):
-//   DMA (d = 128, the default): global_load_lds_dwordx4 streams tiles into three slots
+//   DMA (the default): global_load_lds_dwordx4 streams tiles into three slots
 //     two tiles ahead, no staging registers; V stays row-major and the P.V operand comes
 //     from ds_read_b64_tr_b16 (a transposed LDS read); XOR swizzles keep every read
 //     conflict-free;
-//   registers (d = 64): the next tile is loaded into registers during this tile's math
+//   registers (prefill_dma=0): the next tile is loaded into registers during this tile's math
 //     and stored double-buffered, V transposed in registers (v_perm).
 // The MFMAs:
 //   S^T[pos][row] = K . Q^T: A = K rows from LDS (MFMA h, row i <-> position
@@ -261,13 +264,13 @@ __device__ __forceinline__ uint32_t vswz(uint32_t r) {
                        : 2u * (((r >> 1) & 1u) + 2u * ((r >> 3) & 1u));
 }
 
-// DMA: the register budget of 3 waves/SIMD (170 VGPRs; the DMA form holds no staging
-// registers): 392 vs 369 TFLOP/s at 2 waves (cfg5).
+// DMA: the register budget of 3 waves/SIMD at d = 128 (170 VGPRs; the DMA form holds no staging
+// registers): 392 vs 369 TFLOP/s at 2 waves (cfg5); of 4 at d = 64 (98 VGPRs, 24 KiB of LDS).
 // PS: P carried as f16 high part + residual (P.V exact in f32, two MFMAs per d block);
 // without it P is one RNE f16 (one MFMA per d block) and the row sums add the rounded
 // probabilities, so the weights the output is normalised by are exactly those applied.
 template <int D, bool DMA, bool PS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DMA ? 3 : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!DMA ? 1 : D == 64 ? 4 : 3)))
 void k_prefill_f16(QV_PREFILL_SPLIT_PARAMS) {
     constexpr int TP = PrefillLds<D>::TP;
     constexpr int KS = D / 32;                 // QK k-steps
@@ -620,18 +623,19 @@ void k_prefill_f16(QV_PREFILL_SPLIT_PARAMS) {
         // then kept both in scratch memory and read the chosen one back through a pointer
         // on every tile of the register path.
         const uint32_t koff = (uint32_t)geo.k_off, kv_gap = (uint32_t)(geo.v_off - geo.k_off);
-        // Chunk u of this thread: wave w moves group 4 (w & 1) + u of its half's 8 groups of
-        // 64 chunks (4 LDS rows each): groups 0-3 the K rows holding the half's positions
-        // (LDS rows {0-3, 4-7, 16-19, 20-23} + 8 half), 4-7 its V rows (16 half + 4 (g - 4)
-        // ..).  Fixed for every tile: the chunk's pool offset inside a block, and for the
+        // Chunk u of this thread: wave w moves group CPT (w & 1) + u of its half's 2 CPT groups
+        // of 64 chunks (RPG = 4 LDS rows at d = 128, 8 at d = 64): even waves the K rows holding
+        // the half's positions (LDS rows {0-7, 16-23} + 8 half), odd ones its V rows
+        // (16 half ..).  Fixed for every tile: the chunk's pool offset inside a block, and for the
         // wave whether it is V and the LDS offset of its first chunk.  The load then takes
         // the half's scalar block base plus a 32-bit lane offset.
-        static_assert(CPT == 4 && CPR == 16, "the DMA form is laid out for d = 128");
+        constexpr uint32_t RPG = 64 / CPR, HG = 8 / RPG;  // rows per group, groups per 8 rows
+        static_assert(CPT == 2 * (int)HG, "a wave moves the K or the V rows of one half");
         auto chunk_u = [&](int u) -> uint32_t {  // chunk index: K 0..CH-1, then V
-            const uint32_t gi = 4u * (w & 1u) + (uint32_t)u, hf = w >> 1;
-            const uint32_t r0 = gi < 4u ? 4u * (gi & 1u) + 16u * (gi >> 1) + 8u * hf
-                                        : 16u * hf + 4u * (gi - 4u);
-            return (gi < 4u ? 0u : (uint32_t)CH) + r0 * CPR + lane;
+            const uint32_t hf = w >> 1, gu = (uint32_t)u;
+            const uint32_t r0 = (w & 1u) == 0u ? RPG * (gu % HG) + 16u * (gu / HG) + 8u * hf
+                                               : 16u * hf + RPG * gu;
+            return ((w & 1u) == 0u ? 0u : (uint32_t)CH) + r0 * CPR + lane;
         };
         // (in a lambda: the host pass of a kernel body must not see the device builtins)
         uint32_t c_off[CPT], c_lds[CPT], c_v[CPT];
@@ -719,8 +723,7 @@ void k_prefill_f16(QV_PREFILL_SPLIT_PARAMS) {
         // chunks (CPT instructions each) are still outstanding
         auto wait_tile = [&](uint32_t t) {
             if (t + 1 < ntiles) {
-                if constexpr (CPT == 4) __builtin_amdgcn_s_waitcnt(0x0f74);  // vmcnt(4)
-                else __builtin_amdgcn_s_waitcnt(0x0f72);                    // vmcnt(2)
+                __builtin_amdgcn_s_waitcnt(0x0f70 | CPT);  // vmcnt(CPT)
             } else {
                 __builtin_amdgcn_s_waitcnt(0x0f70);                         // vmcnt(0)
             }
@@ -730,7 +733,7 @@ void k_prefill_f16(QV_PREFILL_SPLIT_PARAMS) {
             constexpr bool STEADY = decltype(steady)::value;
             // Tile t landed everywhere and every wave is past tile t - 1.  A bare barrier:
             // __syncthreads' fence would also wait for the tiles still in flight.
-            if constexpr (STEADY) __builtin_amdgcn_s_waitcnt(0x0f74);  // vmcnt(4)
+            if constexpr (STEADY) __builtin_amdgcn_s_waitcnt(0x0f70 | CPT);  // vmcnt(CPT)
             else wait_tile(t);
             __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): register-path LDS stores
             asm volatile("" ::: "memory");       // no LDS access moves across the barrier
@@ -1259,25 +1262,26 @@ PrefillPlan plan_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint
     const PrefillForm form = prefill_form(g, f16_values);
     if (form != PrefillForm::F16 && form != PrefillForm::Q8) return p;
     // Chunks per row block: the count whose estimated time is least.  A CU holds 3
-    // workgroups (768 on the chip); a 32-position tile takes a workgroup about `tile_us`
-    // with 3 on its CU and 0.6 / 0.8 of that with one or two; each workgroup spends about
+    // workgroups (4 at d = 64); a 32-position tile takes a workgroup about `tile_us` with
+    // its CU full and down to 0.55-0.6 of that alone on it; each workgroup spends about
     // 4 us outside its tiles, and a split launch 5 us more on its merge plus the partials'
     // traffic (written and read once).  Measured at 2 k positions, f16, d = 128, in us by
     // chunks 1 / 2 / 3 / 4 / 8: 32 row blocks 49 / 32 / 26 / 22 / 20, 128 blocks 51 / 36 /
     // 33 / 31 / 41, 256 blocks 53 / 45 / 46 / 53 / 67, 512 blocks 65 / 83 / 81 / 92 / 134; a
-    // 512-token chunk at 8 k (256 blocks of 272 tiles) 188 -> 124 us with 3.
-    const uint64_t slots = 768;
+    // 512-token chunk at 8 k (256 blocks of 272 tiles) 188 -> 124 us with 3; d = 64, the same
+    // chunk by 1 / 2 / 3 / 4 / 6: 132 / 83 / 76 / 75 / 78.
+    const uint64_t cus = 256, slots = (form == PrefillForm::F16 && g.D == 64 ? 4 : 3) * cus;
     const uint64_t blocks =
         (uint64_t)n_seg * g.G * (((uint64_t)max_tok * (heads / (uint32_t)g.G) + 63) / 64);
     const uint64_t tiles = ((uint64_t)max_pos + 32) / 32;
-    const double tile_us = (form == PrefillForm::Q8 ? 2.2 : 1.14) * (g.D / 128.0);
+    const double tile_us = form == PrefillForm::Q8 ? 2.2 : g.D == 64 ? 0.84 : 1.14;
     const int forced = tune(KNOB_PREFILL_CHUNKS);
     double best = 0.0;
     for (uint32_t n = 1; n <= PREFILL_MAX_CHUNKS; n++) {
         if (n > 1 && (tiles < 2ull * n || blocks * n > 8 * slots) && forced == 0) break;
-        const uint64_t rem = blocks * n % slots;
+        const uint64_t per_cu = (blocks * n % slots + cus - 1) / cus;  // of the last round
         const double rounds = (double)(blocks * n / slots) +
-                              (rem == 0 ? 0.0 : rem <= slots / 3 ? 0.6 : rem <= 2 * slots / 3 ? 0.8 : 1.0);
+                              (per_cu == 0 ? 0.0 : 0.4 + 0.6 * (double)(per_cu * cus) / (double)slots);
         double us = rounds * ((double)((tiles + n - 1) / n) * tile_us + 4.0);
         if (n > 1) us += 5.0 + (double)(blocks * n) * 64.0 * (g.D + 2) * 8.0 / 4e6;
         if (n == 1 || (forced == 0 ? us < best : (int)n <= forced)) {
@@ -1328,12 +1332,17 @@ hipError_t launch_prefill(const Geometry &g, const PrefillPlan &plan, const void
         // P as one f16 (the default) or as high part + residual (knob prefill_exact_p=1)
         const bool ps = tune(KNOB_PREFILL_EXACT_P) != 0;
         if (form == PrefillForm::Q8) QV_PF2((k_prefill_q8<128>));
-        else if (g.D == 64) { if (ps) QV_PF2((k_prefill_f16<64, false, true>)); else QV_PF2((k_prefill_f16<64, false, false>)); }
-        else if (tune(KNOB_PREFILL_DMA)) {
-            if (ps) QV_PF2((k_prefill_f16<128, true, true>)); else QV_PF2((k_prefill_f16<128, true, false>));
-        } else {
-            if (ps) QV_PF2((k_prefill_f16<128, false, true>)); else QV_PF2((k_prefill_f16<128, false, false>));
-        }
+#define QV_PF2_D(DD)                                                                           \
+    do {                                                                                        \
+        if (tune(KNOB_PREFILL_DMA)) {                                                           \
+            if (ps) QV_PF2((k_prefill_f16<DD, true, true>)); else QV_PF2((k_prefill_f16<DD, true, false>)); \
+        } else {                                                                                \
+            if (ps) QV_PF2((k_prefill_f16<DD, false, true>)); else QV_PF2((k_prefill_f16<DD, false, false>)); \
+        }                                                                                       \
+    } while (0)
+        else if (g.D == 64) QV_PF2_D(64);
+        else QV_PF2_D(128);
+#undef QV_PF2_D
 #undef QV_PF2
         hipError_t e = hipGetLastError();
         if (e != hipSuccess || n_ch == 1) return e;
