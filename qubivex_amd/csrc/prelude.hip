@@ -178,9 +178,10 @@ __device__ __forceinline__ float rms_scale_of(float ss, float n, float eps) {
 
 __global__ __launch_bounds__(64) void k_prelude(float *__restrict__ q, float *__restrict__ k,
                                                 float *__restrict__ v, uint32_t heads,
-                                                uint32_t kvh, uint32_t d, PreludeArgs a) {
+                                                uint32_t kvh, uint32_t d, uint32_t parts,
+                                                PreludeArgs a) {
     extern __shared__ float xs[];
-    const uint32_t t = blockIdx.x / 3, part = blockIdx.x % 3, lane = threadIdx.x;
+    const uint32_t t = blockIdx.x / parts, part = blockIdx.x % parts, lane = threadIdx.x;
     const uint32_t n = part == 0 ? heads * d : kvh * d;
     float *x = (part == 0 ? q : part == 1 ? k : v) + (uint64_t)t * n;
     const float *bias = part == 0 ? a.q_bias : part == 1 ? a.k_bias : a.v_bias;
@@ -351,16 +352,16 @@ __device__ __forceinline__ void prelude_heads(float *__restrict__ x, const float
                 __builtin_nontemporal_store(z[h][j], &x[h * D + 64 * j + lane]);
 }
 
-// One wave per (token, q|k|v, batch of HB heads).  (Fewer heads per wave on k and v rows
+// One wave per (token, q|k|v, batch of HB heads); parts: 3, or 2 without the v rows.  (Fewer heads per wave on k and v rows
 // with few KV heads, 4 instead of 16 at cfg5's 4 KV heads, measured 17 % slower.)
 template <int D, bool FULL, int VPW = 1024>
 __global__ __launch_bounds__(256) void k_prelude_r(float *__restrict__ q, float *__restrict__ k,
                                                    float *__restrict__ v, uint32_t s,
                                                    uint32_t heads, uint32_t kvh, uint32_t uq,
-                                                   uint32_t ukv, PreludeArgs a) {
+                                                   uint32_t ukv, uint32_t parts, PreludeArgs a) {
     // heads per wave: 1024 values was the best of 512, 1024, 2048 without a full norm
     constexpr uint32_t HB = (FULL ? 4096 : VPW) / D;
-    const uint32_t per_tok = uq + 2 * ukv;
+    const uint32_t per_tok = uq + (parts - 1) * ukv;
     // the wave index as a scalar: every per-head branch below is then a scalar branch
     const uint32_t u = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
@@ -382,12 +383,13 @@ __global__ __launch_bounds__(256) void k_prelude_r(float *__restrict__ q, float 
 // in one), and a workgroup holds 4 / WPR rows.  The sum of squares stays lane l's fused
 // multiply-add chain over j in order: with WPR > 1 each wave continues the running sum the
 // wave before left in LDS.  The RoPE pairs of a head lie in one wave (a head is d/64
-// consecutive j).  rows: q rows (part 0, row = token), or k and v rows (row 2 t + 0 / 1).
+// consecutive j).  rows: q rows (part 0, row = token), or k and v rows (row 2 t + 0 / 1;
+// with 2 parts the k rows alone).
 template <int D, int WPR>
 __global__ __launch_bounds__(256) void k_prelude_full(float *__restrict__ q, float *__restrict__ k,
                                                       float *__restrict__ v, uint32_t s,
                                                       uint32_t heads, uint32_t kvh, bool kv_rows,
-                                                      PreludeArgs a) {
+                                                      uint32_t parts, PreludeArgs a) {
     constexpr uint32_t JW = 16;            // elements per lane per wave
     constexpr uint32_t JD = D / 64;        // elements per lane per head
     constexpr uint32_t RPW = 4 / WPR;      // rows per workgroup
@@ -397,9 +399,10 @@ __global__ __launch_bounds__(256) void k_prelude_full(float *__restrict__ q, flo
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t rw = w / WPR, wr = w % WPR;  // the wave's row in the workgroup, its part of it
     const uint32_t row = blockIdx.x * RPW + rw;
-    const bool live = row < (kv_rows ? 2 * s : s);
-    const uint32_t t = kv_rows ? row / 2 : row;
-    const uint32_t part = kv_rows ? 1u + (row & 1u) : 0u;
+    const bool both = kv_rows && parts == 3;  // k and v rows alternate
+    const bool live = row < (both ? 2 * s : s);
+    const uint32_t t = both ? row / 2 : row;
+    const uint32_t part = both ? 1u + (row & 1u) : kv_rows ? 1u : 0u;
     const uint32_t nh = part == 0 ? heads : kvh;
     const uint32_t J = nh * JD;            // elements per lane in the row (at most 64)
     const uint32_t j0 = wr * JW;
@@ -504,6 +507,10 @@ hipError_t launch_prelude(float *q, float *k, float *v, uint32_t s, uint32_t hea
                           uint32_t kvh, uint32_t d, const PreludeArgs &a, hipStream_t st) {
     if (s == 0) return hipSuccess;
     const bool full = a.norm == QVKV_NORM_FULL;
+    // The values take a bias and a clip only: without either their rows already hold the
+    // result, and the launch leaves them out (8192 tokens of 32 query and 4 KV heads of 128 with
+    // per-head norms 56.4 -> 50.9 us, 6.0 TB/s of what is left).
+    const uint32_t parts = a.v_bias || a.has_clip ? 3 : 2;
     if ((d == 64 || d == 128 || d == 256) && (!full || (heads * d <= 4096 && kvh * d <= 4096)) &&
         tune(KNOB_PRELUDE_FAST) != 0) {
         // per-head norms at d = 128: 2048 values per wave (one vector rms serves 16 heads;
@@ -516,12 +523,12 @@ hipError_t launch_prelude(float *q, float *k, float *v, uint32_t s, uint32_t hea
             for (int kv = 0; kv < 2; kv++) {
                 const uint32_t J = (kv ? kvh : heads) * (d / 64);
                 const int wpr = J > 32 ? 4 : J > 16 ? 2 : 1;
-                const uint64_t rows = (uint64_t)s * (kv ? 2 : 1);
+                const uint64_t rows = (uint64_t)s * (kv ? parts - 1 : 1);
                 const uint64_t grid = (rows * wpr + 3) / 4;
                 if (grid > 0x7fffffffull) return hipErrorInvalidValue;
 #define QV_PRE_FULL(DD, WW)                                                                     \
     hipLaunchKernelGGL((k_prelude_full<DD, WW>), dim3((unsigned)grid), dim3(256), 0, st, q, k, v, \
-                       s, heads, kvh, kv != 0, a)
+                       s, heads, kvh, kv != 0, parts, a)
 #define QV_PRE_FULL_D(DD)                                                                       \
     do {                                                                                        \
         if (wpr == 4) QV_PRE_FULL(DD, 4);                                                       \
@@ -540,12 +547,12 @@ hipError_t launch_prelude(float *q, float *k, float *v, uint32_t s, uint32_t hea
         }
         const uint32_t hb = (full ? 4096u : wide ? 2048u : 1024u) / d;
         const uint32_t uq = (heads + hb - 1) / hb, ukv = (kvh + hb - 1) / hb;
-        const uint64_t waves = (uint64_t)s * (uq + 2 * ukv);
+        const uint64_t waves = (uint64_t)s * (uq + (parts - 1) * ukv);
         const uint64_t grid = (waves + 3) / 4;
         if (waves > 0xffffffffull || grid > 0x7fffffffull) return hipErrorInvalidValue;
 #define QV_PRE_L(DD, FF, VPW)                                                                   \
     hipLaunchKernelGGL((k_prelude_r<DD, FF, VPW>), dim3((unsigned)grid), dim3(256), 0, st, q, k, \
-                       v, s, heads, kvh, uq, ukv, a)
+                       v, s, heads, kvh, uq, ukv, parts, a)
 #define QV_PRE(DD)                                                                              \
     do {                                                                                        \
         if (full) QV_PRE_L(DD, true, 1024);                                                     \
@@ -560,8 +567,8 @@ hipError_t launch_prelude(float *q, float *k, float *v, uint32_t s, uint32_t hea
         return hipGetLastError();
     }
     const uint64_t lds = (uint64_t)(heads > kvh ? heads : kvh) * d * 4;
-    hipLaunchKernelGGL(k_prelude, dim3(s * 3), dim3(64), (uint32_t)lds, st, q, k, v, heads, kvh,
-                       d, a);
+    hipLaunchKernelGGL(k_prelude, dim3(s * parts), dim3(64), (uint32_t)lds, st, q, k, v, heads, kvh,
+                       d, parts, a);
     return hipGetLastError();
 }
 
