@@ -546,7 +546,7 @@ __device__ __forceinline__ void store_f8(float *dst, const float *y) {
     st_g_nt((f4v *)(dst + 4), f4v{y[4], y[5], y[6], y[7]});
 }
 
-// T threads per workgroup; UF: loads in flight per thread in the f16 -> f16 copy.
+// T threads per workgroup; UF: loads in flight per thread (f16 pools).
 template <int DT, int OUT, int T = 256, int UF = 8>
 __global__ __launch_bounds__(T) void k_gather(const uint8_t *__restrict__ pool,
                                                 uint64_t pool_blocks,
@@ -619,17 +619,17 @@ __global__ __launch_bounds__(T) void k_gather(const uint8_t *__restrict__ pool,
     if (DT == QVKV_F16 && OUT == QVKV_F32) {
         // f16 -> f32: 4 values per thread (an 8-byte load, a 16-byte store), so
         // consecutive lanes store consecutive 16-byte pieces and every store instruction
-        // covers whole output lines; 8 loads in flight per thread.
+        // covers whole output lines; UF loads in flight per thread.
         const uint32_t c4 = D >> 2;
         const uint32_t per4 = G * 16u * c4;
-        constexpr int U = 8;
-        for (uint32_t b0 = part * 256u * U; b0 < 2u * per4; b0 += parts * 256u * U) {
+        constexpr int U = UF;
+        for (uint32_t b0 = part * (uint32_t)T * U; b0 < 2u * per4; b0 += parts * (uint32_t)T * U) {
             u2v x[U];
             float *dst[U];
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 dst[u] = nullptr;
-                const uint32_t idx = b0 + u * 256u + threadIdx.x;
+                const uint32_t idx = b0 + u * (uint32_t)T + threadIdx.x;
                 if (idx >= 2u * per4) continue;
                 const bool isv = idx >= per4;
                 uint32_t r = isv ? idx - per4 : idx;
@@ -709,7 +709,8 @@ __global__ __launch_bounds__(T) void k_gather(const uint8_t *__restrict__ pool,
 //     d = 32i + 8q .. +7 and 32(i+1) + 8q .. +7;
 //   V (byte c*(D/16) + 2g + u holds d = 32g + 2c + u): a piece holds NC = 256/D (>= 1)
 //     consecutive c of NG = 8/NC groups, i.e. 2*NC consecutive values of each group.
-// The row's D/32 f16 scales come in with one load.  8 pieces in flight per thread.
+// The row's D/32 f16 scales come in with one load.  U pieces in flight per thread, T threads
+// per workgroup, `parts` workgroups per tile.
 template <int D>
 __device__ __forceinline__ void store_run(float *dst, const float *y, int n) {
     if (n == 8) store_f8(dst, y);
@@ -725,8 +726,8 @@ __device__ __forceinline__ void lds_order() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
-template <int D>
-__global__ __launch_bounds__(256) void k_gather_q8(const uint8_t *__restrict__ pool,
+template <int D, int T, int U>
+__global__ __launch_bounds__(T) void k_gather_q8(const uint8_t *__restrict__ pool,
                                                    uint64_t pool_blocks,
                                                    const uint32_t *__restrict__ blocks,
                                                    uint64_t n_table,
@@ -735,9 +736,11 @@ __global__ __launch_bounds__(256) void k_gather_q8(const uint8_t *__restrict__ p
                                                    const uint64_t *__restrict__ out_at,
                                                    uint32_t n_items, uint32_t tiles_max,
                                                    uint64_t out_positions, float *out_k,
-                                                   float *out_v, Geo geo, int *err) {
-    const uint32_t item = blockIdx.x / tiles_max;
-    const uint32_t tile = blockIdx.x - item * tiles_max;
+                                                   float *out_v, uint32_t parts, Geo geo,
+                                                   int *err) {
+    const uint32_t unit = blockIdx.x / parts, part = blockIdx.x - unit * parts;
+    const uint32_t item = unit / tiles_max;
+    const uint32_t tile = unit - item * tiles_max;
     if (item >= n_items) return;
     const uint32_t len = lens[item];
     const uint32_t p0 = tile * 16u;
@@ -762,20 +765,20 @@ __global__ __launch_bounds__(256) void k_gather_q8(const uint8_t *__restrict__ p
     const uint32_t r0 = p0 % B;
     const uint8_t *base = pool + (uint64_t)blk * geo.bb;
     // d = 128 keys: a per-wave LDS copy of the wave's 8 rows (row stride 132 floats)
-    __shared__ __attribute__((aligned(16))) float kx[4][D == 128 ? 8 * 132 : 4];
+    __shared__ __attribute__((aligned(16))) float kx[T / 64][D == 128 ? 8 * 132 : 4];
     constexpr uint32_t PR = D / 16;           // pieces per row
     constexpr uint32_t NS = D / 32;           // scales per row
     constexpr uint32_t NC = D >= 256 ? 1 : 256 / D, NG = 8 / NC;
     const uint32_t per_kv = G * 16u * PR;
-    constexpr int U = 8;
-    for (uint32_t b0 = 0; b0 < 2u * per_kv; b0 += 256u * U) {
+    {
+        const uint32_t b0 = part * (uint32_t)(T * U);
         u4v x[U];
         u4v sc[U];
         float *dst[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
             dst[u] = nullptr;
-            const uint32_t idx = b0 + u * 256u + threadIdx.x;
+            const uint32_t idx = b0 + u * (uint32_t)T + threadIdx.x;
             if (idx >= 2u * per_kv) continue;
             const bool isv = idx >= per_kv;
             const uint32_t r = isv ? idx - per_kv : idx;
@@ -794,7 +797,7 @@ __global__ __launch_bounds__(256) void k_gather_q8(const uint8_t *__restrict__ p
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (!dst[u]) continue;
-            const uint32_t idx = b0 + u * 256u + threadIdx.x;
+            const uint32_t idx = b0 + u * (uint32_t)T + threadIdx.x;
             const bool isv = idx >= per_kv;
             const uint32_t j = (isv ? idx - per_kv : idx) % PR;
             const uint32_t w[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
@@ -1915,10 +1918,24 @@ hipError_t launch_gather(const Geometry &g, const void *pool, uint64_t pool_bloc
     hipLaunchKernelGGL((k_gather<DT, OT>), dim3((unsigned)(grid * parts)), dim3(256), 0, s, p,  \
                        pool_blocks, blocks, n_table, table_at, lens, out_at, n_items, tiles,   \
                        out_positions, out_k, out_v, parts, geo, err)
+    // One-wave workgroups, each one batch of a tile, as for the block copy: many short workgroups
+    // keep the stores, most of the traffic, spread over time.  Against 256 threads x 8 pieces (a
+    // tile per workgroup), in us: q8_0 d = 128, 64 items of 1024-2048, 236 -> 192 (1.02 GB, 5.3
+    // TB/s; 2, 4 and 8 pieces per thread 187, 191, 241), d = 64 197 -> 108 (8 pieces took 185
+    // VGPRs), d = 256 252 -> 209; f16 -> f32 with 4 pieces 228 -> 217 (1: 286, 2: 223, 8: 226).
+    // A launch whose workgroups would pass the grid's limit takes the larger ones.
+    auto fits = [&](uint64_t per_tile) { return grid * per_tile * 64 <= 0xffffffffull; };
+#define QV_GATHER_Q8T(DD, TT, UU)                                                              \
+    hipLaunchKernelGGL((k_gather_q8<DD, TT, UU>), dim3((unsigned)(grid * parts_of(TT * UU))),    \
+                       dim3(TT), 0, s, p, pool_blocks, blocks, n_table, table_at, lens, out_at, \
+                       n_items, tiles, out_positions, (float *)out_k, (float *)out_v,           \
+                       parts_of(TT * UU), geo, err)
 #define QV_GATHER_Q8(DD)                                                                       \
-    hipLaunchKernelGGL((k_gather_q8<DD>), dim3((unsigned)grid), dim3(256), 0, s, p,            \
-                       pool_blocks, blocks, n_table, table_at, lens, out_at, n_items, tiles,   \
-                       out_positions, (float *)out_k, (float *)out_v, geo, err)
+    do {                                                                                        \
+        auto parts_of = [&](uint32_t n) { return (2u * (uint32_t)g.G * (uint32_t)DD + n - 1) / n; }; \
+        if (fits(parts_of(64))) QV_GATHER_Q8T(DD, 64, 1);                                        \
+        else QV_GATHER_Q8T(DD, 256, 8);                                                          \
+    } while (0)
     const bool q8fast = tune(KNOB_GATHER_Q8_FAST) != 0;
     if (g.dtype == QVKV_Q8_0 && q8fast && g.D == 64) QV_GATHER_Q8(64);
     else if (g.dtype == QVKV_Q8_0 && q8fast && g.D == 128) QV_GATHER_Q8(128);
@@ -1940,9 +1957,16 @@ hipError_t launch_gather(const Geometry &g, const void *pool, uint64_t pool_bloc
 #undef QV_G64
     }
     else if (g.dtype == QVKV_F16 && out_dtype == QVKV_F16) QV_GATHER(QVKV_F16, QVKV_F16);
+    else if (g.dtype == QVKV_F16 && fits((vals + 1023) / 1024)) {
+        const uint32_t pf = (uint32_t)((vals + 1023) / 1024);  // 64 threads x 4 pieces x 4 values
+        hipLaunchKernelGGL((k_gather<QVKV_F16, QVKV_F32, 64, 4>), dim3((unsigned)(grid * pf)),
+                           dim3(64), 0, s, p, pool_blocks, blocks, n_table, table_at, lens, out_at,
+                           n_items, tiles, out_positions, out_k, out_v, pf, geo, err);
+    }
     else if (g.dtype == QVKV_F16) QV_GATHER(QVKV_F16, QVKV_F32);
     else QV_GATHER(QVKV_Q8_0, QVKV_F32);
 #undef QV_GATHER_Q8
+#undef QV_GATHER_Q8T
 #undef QV_GATHER
     return hipGetLastError();
 }
