@@ -136,7 +136,8 @@ int qvkv_max_arena(const qvkv_dev *dev, uint64_t *out);
  * append_q8_fast, append_nts, gather_split, gather_q8_fast, gather_t, gather_uf, copy_u,
  * copy_t, attn_full, attn_wide, attn_stream, attn_stream_wg, stream_unit_cost, attn_target, fused_q8,
  * attn_waves4_f16, attn_waves3_q8, attn_pack, attn_ids_below, attn_xcd, prefill_v2,
- * prefill_lds_pad, prefill_exact_p, prefill_dma, prefill_chunks, prefill_q8_fast,
+ * prefill_lds_pad, prefill_exact_p, prefill_dma, prefill_chunks, prefill_images,
+ * prefill_q8_fast,
  * prelude_fast, prelude_wide, prelude_full_wg.  An unknown name is QVKV_E_SHAPE. */
 int qvkv_tune(const char *name, int value);
 int qvkv_tune_get(const char *name, int *value);

@@ -214,7 +214,7 @@ int ensure_attention(qvkv_dev *dev, StreamState *st, const qvkv::AttnPlan &p) {
 // A buffer that a capture has recorded is never freed before the device closes: its graph
 // may be replayed after a larger launch.  Caller holds st->ws_mu.
 qvkv::PrefillPlan ensure_prefill(qvkv_dev *dev, StreamState *st, const qvkv::PrefillPlan &p) {
-    if (p.n_chunks == 1) return p;
+    if (p.ws_bytes == 0) return p;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st->stream, &cap) != hipSuccess) {
         (void)hipGetLastError();

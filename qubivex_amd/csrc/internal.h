@@ -108,6 +108,7 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     X(PREFILL_EXACT_P, "prefill_exact_p", 0)                                                    \
     X(PREFILL_DMA, "prefill_dma", 1)                                                            \
     X(PREFILL_CHUNKS, "prefill_chunks", 0)      /* chunks per row block; 0: by the plan */     \
+    X(PREFILL_IMAGES, "prefill_images", 12)     /* q8_0: row blocks that share images; 0: off */ \
     X(PREFILL_Q8_FAST, "prefill_q8_fast", 1)                                                    \
     X(PRELUDE_FAST, "prelude_fast", 1)                                                          \
     X(PRELUDE_WIDE, "prelude_wide", 1)                                                          \
@@ -128,9 +129,14 @@ int check_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t ma
                   const char **why);
 // The plan of a prefill launch: workgroups per row block (64 query rows of a (segment, KV
 // head)), and the workspace that a split launch (n_chunks > 1) keeps its partials in.
+// q8_0 launches may also keep images of their tiles there (img_segs segments at once, img_tiles
+// each per KV head, img_bytes in all); the default plan needs no workspace.
 constexpr uint32_t PREFILL_MAX_CHUNKS = 16;
+constexpr uint64_t PREFILL_IMAGE_BYTES = 512ull << 20;
 struct PrefillPlan {
     uint32_t n_chunks = 1;
+    uint32_t img_segs = 0, img_tiles = 0;
+    uint64_t img_bytes = 0;
     uint64_t ws_bytes = 0;
 };
 PrefillPlan plan_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t max_pos,

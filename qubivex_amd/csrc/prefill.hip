@@ -791,9 +791,203 @@ struct Q8PrefillSlot {
     uint32_t ks[32 * (D / 64)];   // key scales, [position][group] f16
 };
 
+// One thread's part of staging a q8_0 tile: loaded from the pool, then converted into a slot.
 template <int D>
+struct Q8Stage {
+    static constexpr uint32_t CPR = D / 8;  // 8-value (16-byte f16) pieces per row
+    // a 16-position half of a tile: its block and the first row of the half (g * B + its offset
+    // in the block), or null past the context / for a bad id
+    struct Half {
+        const uint8_t *base;
+        uint32_t row0;
+    };
+    uint32_t sp, sj, klr, kslot[2], kchunk[2];
+    u2v xk[2];
+    u4v xv;
+    u2v xvs;
+    uint32_t xks;
+    // thread = (position sp, lane sj = tid % 8 of the position) of the tile,
+    // plus the row's 4 V scales; threads 0..63 also move one word of K scales (position
+    // tid / 2).  The LDS stores are laid out to take the fewest bank passes:
+    //   K: store k (0, 1) of lane sj fills LDS slot sj + 8 ((k + si) & 1) of its row, so
+    //      each 8 lanes write one aligned 128-byte half of a row and the two rows of a
+    //      16-lane group write opposite halves; the lane loads the two stored 8-byte chunks
+    //      (4 (P % 4) + P / 4 holds logical piece P) that its slots need;
+    //   V: lane sj loads stored bytes 16 sj .. +15 and writes 8-byte quarter pieces; the
+    //      position order (sp bit 1 = si bit 0, sp bit 3 = si bit 1) puts the rows of each
+    //      2- and 4-row group of an LDS store in distinct 64-byte quarters of the banks.
+    __device__ __forceinline__ void init() {
+        const uint32_t si = threadIdx.x >> 3;
+        sp = ((si & 1u) << 1) | ((si & 2u) << 2) | ((si >> 2) & 1u) |
+                            (((si >> 3) & 1u) << 2) | (si & 16u);
+        sj = threadIdx.x & 7u;
+        klr = 16u * ((sp >> 2) & 1u) + 4u * (sp >> 3) + (sp & 3u);  // K row in LDS
+    #pragma unroll
+        for (int k = 0; k < 2; k++) {
+            kslot[k] = sj + 8u * ((k + si) & 1u);
+            const uint32_t P = kslot[k] ^ kswz<D>(klr);  // logical piece of the slot
+            kchunk[k] = 4u * (P & 3u) + (P >> 2);       // stored 8-byte chunk holding it
+        }
+    }
+    // the first `left` positions of the tile exist; the rest read as zero
+    __device__ __forceinline__ void load(const Half &h0, const Half &h1, uint32_t left, const Geo &geo) {
+        xk[0] = u2v{0u, 0u};
+        xk[1] = u2v{0u, 0u};
+        xv = u4v{0u, 0u, 0u, 0u};
+        xvs = u2v{0u, 0u};
+        xks = 0u;
+        // (chosen by value: a choice between the two structs would keep them in scratch memory)
+        const Half hp{(sp & 16u) ? h1.base : h0.base, (sp & 16u) ? h1.row0 : h0.row0};
+        if (hp.base != nullptr && sp < left) {
+            const uint32_t rw = hp.row0 + (sp & 15u);
+            xk[0] = *(const u2v *)(hp.base + geo.k_off + rw * D + 8u * kchunk[0]);
+            xk[1] = *(const u2v *)(hp.base + geo.k_off + rw * D + 8u * kchunk[1]);
+            xv = *(const u4v *)(hp.base + geo.v_off + rw * D + 16u * sj);
+            xvs = *(const u2v *)(hp.base + geo.vs_off + rw * (D / 16));
+        }
+        // K scales: threads 0..63, position tid / 2, word tid % 2
+        const uint32_t pk = threadIdx.x >> 1;
+        const Half hk{(pk & 16u) ? h1.base : h0.base, (pk & 16u) ? h1.row0 : h0.row0};
+        if (threadIdx.x < 64u && hk.base != nullptr && pk < left)
+            xks = *(const uint32_t *)(hk.base + geo.ks_off + (hk.row0 + (pk & 15u)) * (D / 16) +
+                                      4u * (threadIdx.x & 1u));
+    }
+    __device__ __forceinline__ void store(Q8PrefillSlot<D> &sl, int *err) const {
+        // K: each loaded 8-byte chunk is one logical 8-value piece, stored at its slot
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const h4 a = i8x4_to_h4_vals(xk[k].x), b = i8x4_to_h4_vals(xk[k].y);
+            *(h8 *)(sl.k + (klr * CPR + kslot[k]) * 8) =
+                h8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        }
+        // V: stored byte c * 8 + 2 gr + u holds d = 32 gr + 2 c + u; this piece holds
+        // c = 2 sj, 2 sj + 1: for each group gr, d = 32 gr + 4 sj .. +3 from bytes
+        // 2 gr, 2 gr + 1, 8 + 2 gr, 9 + 2 gr
+        bool big = false;
+#pragma unroll
+        for (int gr = 0; gr < 4; gr++) {
+            const uint32_t w0 = xv[gr >> 1], w1 = xv[2 + (gr >> 1)];
+            h2 x01, x23;
+            if (gr & 1) {
+                x01 = __builtin_bit_cast(h2, i8x2_to_h2<2>(w0));
+                x23 = __builtin_bit_cast(h2, i8x2_to_h2<2>(w1));
+            } else {
+                x01 = __builtin_bit_cast(h2, i8x2_to_h2<0>(w0));
+                x23 = __builtin_bit_cast(h2, i8x2_to_h2<0>(w1));
+            }
+            const uint32_t sbits = (xvs[gr >> 1] >> (16u * (gr & 1u))) & 0xffffu;
+            const _Float16 sc = __builtin_bit_cast(_Float16, (uint16_t)sbits);
+            // |scale| above 512 (f16 0x6000), infinities included, NaN (above 0x7c00) not
+            big |= (sbits & 0x7fffu) - 0x6001u < 0x7c00u - 0x6000u;
+            const h2 s2 = {sc, sc};
+            h2 a = x01 * s2, b = x23 * s2;       // high parts (rounded products)
+            asm volatile("" : "+v"(a), "+v"(b));  // not contracted into the residuals
+            const h2 ra = __builtin_elementwise_fma(x01, s2, -a);
+            const h2 rb = __builtin_elementwise_fma(x23, s2, -b);
+            const uint32_t P = 4u * gr + (sj >> 1), hf = sj & 1u;
+            const uint32_t off = (sp * CPR + (P ^ vswz<D>(sp))) * 8 + 4 * hf;
+            *(h4 *)(sl.vh + off) = h4{a[0], a[1], b[0], b[1]};
+            *(h4 *)(sl.vl + off) = h4{ra[0], ra[1], rb[0], rb[1]};
+        }
+        if (big) flag(err, ERR_RANGE);
+        if (threadIdx.x < 64u) sl.ks[threadIdx.x] = xks;
+    }
+};
+
+// Transposed V read (ds_read_b64_tr_b16) of a slot's row-major values: lane (col, grp) gets
+// positions 8 grp .. +7 of d = 16 j + col.
+template <int D>
+__device__ __forceinline__ h8 vread_tr(const _Float16 *v, uint32_t j) {
+    constexpr uint32_t CPR = D / 8;
+    const uint32_t lane = threadIdx.x & 63u, grp = lane >> 4, sidx = lane & 15u;
+    u2v wv[2];
+#pragma unroll
+    for (int hf = 0; hf < 2; hf++) {
+        const uint32_t r = 8u * grp + 4u * hf + (sidx >> 2);
+        const uint32_t d = 16u * j + 4u * (sidx & 3u);
+        const uint32_t pc = d >> 3;
+        const _Float16 *a = v + (r * CPR + (pc ^ vswz<D>(r))) * 8 + (d & 7u);
+        typedef short s4 __attribute__((ext_vector_type(4)));
+        wv[hf] = __builtin_bit_cast(u2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                             (__attribute__((address_space(3))) s4 *)a));
+    }
+    return __builtin_bit_cast(h8, u4v{wv[0][0], wv[0][1], wv[1][0], wv[1][1]});
+}
+
+// Images of the tiles of (segment, KV head) sg = seg * G + g, image t at (sg img_tiles + t): K and
+// the key scales as Q8PrefillSlot holds them, the values' high parts and residuals transposed:
+// row d holds its 32 positions, the 16-byte piece of positions 8 x .. +7 at x ^ (d / 4 % 4), so
+// that a P.V operand is one ds_read_b128 without bank conflicts.  Each row block had converted
+// every tile for itself: 90 of its ~190 VALU instructions per tile and wave, and 2 ds_read_b64_tr_b16
+// per operand.  One workgroup per tile; HBM-bound (272 bytes read and 776 written per position
+// and head: 16 segments of 2047 positions and 8 KV heads, 273 MB, 45 us).  The attention of their
+// 512-token chunks then takes 570 us instead of 690: 1.05 PFLOP/s of f16 MFMA issued, 40 for
+// each 16-row tile of which 16 are the useful work, against the 1.2 PFLOP/s that a large
+// f16 matrix product reaches on this part.
+template <int D>
+__global__ __launch_bounds__(256) void k_q8_images(const uint8_t *__restrict__ pool,
+                                                   uint64_t pool_blocks,
+                                                   const uint32_t *__restrict__ blocks,
+                                                   uint64_t n_table,
+                                                   const uint32_t *__restrict__ table_at,
+                                                   const uint32_t *__restrict__ pos0,
+                                                   const uint32_t *__restrict__ q_at,
+                                                   const uint32_t *__restrict__ n_tok,
+                                                   uint32_t max_pos, uint32_t max_tok,
+                                                   uint64_t q_rows, Geo geo, int *err,
+                                                   uint8_t *__restrict__ img, uint32_t img_tiles) {
+    __shared__ __attribute__((aligned(16))) Q8PrefillSlot<D> sl;
+    const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
+    const uint32_t t = blockIdx.x % img_tiles, sg = blockIdx.x / img_tiles;
+    const uint32_t g = sg % G, seg = sg / G;
+    const uint32_t nt = n_tok[seg], p0s = pos0[seg], tab = table_at[seg];
+    // (segments that the attention refuses and flags have no images)
+    if (nt == 0 || nt > max_tok || (uint64_t)p0s + nt - 1 > max_pos ||
+        (uint64_t)q_at[seg] + nt > q_rows || (uint64_t)tab + (p0s + nt + B - 1) / B > n_table)
+        return;
+    const uint32_t n = p0s + nt, p0 = t * 32u;
+    if (p0 >= n) return;
+    using Half = typename Q8Stage<D>::Half;
+    auto half = [&](uint32_t p) {
+        const uint32_t bi = geo.fd_b.div(p);
+        Half h{nullptr, g * B + (p - bi * B)};
+        if (p < n) {
+            const uint32_t id = blocks[tab + bi];
+            if (id < pool_blocks) h.base = pool + (uint64_t)id * geo.bb;
+            else if (threadIdx.x == 0) flag(err, ERR_BLOCK);
+        }
+        return h;
+    };
+    const Half h0 = half(p0), h1 = half(p0 + 16u);
+    Q8Stage<D> stage;
+    stage.init();
+    stage.load(h0, h1, n - p0, geo);
+    stage.store(sl, err);
+    __syncthreads();
+    uint8_t *to = img + ((uint64_t)sg * img_tiles + t) * sizeof(Q8PrefillSlot<D>);
+    const uint8_t *from = (const uint8_t *)&sl;
+#pragma unroll
+    for (uint32_t x = 0; x < 2; x++) {
+        const uint32_t at = (threadIdx.x + 256u * x) * 16u;
+        st_g((u4v *)(to + at), *(const u4v *)(from + at));
+    }
+    constexpr uint32_t VB = 32 * D * 2, KS_AT = 3 * VB;  // bytes of a part; the key scales
+    if (threadIdx.x < 16u) st_g((u4v *)(to + KS_AT + threadIdx.x * 16u), *(const u4v *)(from + KS_AT + threadIdx.x * 16u));
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, col = lane & 15u, grp = lane >> 4;
+#pragma unroll
+    for (uint32_t x = 0; x < 4; x++) {  // d block j = 2 w + x / 2, high parts then residuals
+        const uint32_t j = 2u * w + (x >> 1), dd = 16u * j + col;
+        const u4v v = __builtin_bit_cast(u4v, vread_tr<D>((x & 1u) ? sl.vl : sl.vh, j));
+        st_g((u4v *)(to + VB * (1u + (x & 1u)) + dd * 64u + ((grp ^ ((dd >> 2) & 3u)) * 16u)), v);
+    }
+}
+
+// IMG: the tiles come from images that k_q8_images made (their K and V parts as this kernel's
+// LDS holds them, V transposed), streamed by DMA; the row blocks of a (segment, KV head) share
+// one conversion.
+template <int D, bool IMG>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS) {
+void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS, const uint8_t *__restrict__ img, uint32_t img_tiles) {
     static_assert(D == 128, "q8_0 MFMA-throughput prefill is built for d = 128");
     constexpr int TP = 32;
     constexpr int KS = D / 32;                 // QK k-steps = quantization groups
@@ -875,41 +1069,13 @@ void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS) {
         }
     }
 
-    // ---- staging: thread = (position sp, lane sj = tid % 8 of the position) of the tile,
-    // plus the row's 4 V scales; threads 0..63 also move one word of K scales (position
-    // tid / 2).  The LDS stores are laid out to take the fewest bank passes:
-    //   K: store k (0, 1) of lane sj fills LDS slot sj + 8 ((k + si) & 1) of its row, so
-    //      each 8 lanes write one aligned 128-byte half of a row and the two rows of a
-    //      16-lane group write opposite halves; the lane loads the two stored 8-byte chunks
-    //      (4 (P % 4) + P / 4 holds logical piece P) that its slots need;
-    //   V: lane sj loads stored bytes 16 sj .. +15 and writes 8-byte quarter pieces; the
-    //      position order (sp bit 1 = si bit 0, sp bit 3 = si bit 1) puts the rows of each
-    //      2- and 4-row group of an LDS store in distinct 64-byte quarters of the banks.
-    const uint32_t si = threadIdx.x >> 3;
-    const uint32_t sp = ((si & 1u) << 1) | ((si & 2u) << 2) | ((si >> 2) & 1u) |
-                        (((si >> 3) & 1u) << 2) | (si & 16u),
-                   sj = threadIdx.x & 7u;
-    const uint32_t klr = 16u * ((sp >> 2) & 1u) + 4u * (sp >> 3) + (sp & 3u);  // K row in LDS
-    uint32_t kslot[2], kchunk[2];
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        kslot[k] = sj + 8u * ((k + si) & 1u);
-        const uint32_t P = kslot[k] ^ kswz<D>(klr);  // logical piece of the slot
-        kchunk[k] = 4u * (P & 3u) + (P >> 2);       // stored 8-byte chunk holding it
-    }
-    u2v xk[2];
-    u4v xv;
-    u2v xvs;
-    uint32_t xks;
+    Q8Stage<D> stage;
+    if constexpr (!IMG) stage.init();
     // The block of each 16-position half of a tile, resolved on the scalar unit: the block
     // base and the first row of the half (g * B + its offset in the block), or null past
     // n_wg / for a bad id.  Tiles are resolved in order, one tile ahead of their use: the
     // (block, row) split advances by counters (B is a multiple of 16) and the table
     // entries are constant-address-space loads that land during a tile's math.
-    struct Half {
-        const uint8_t *base;
-        uint32_t row0;
-    };
     // ids at or past pool_ids are bad (the clamp only matters for id 0xffffffff in a pool of
     // 2^32 blocks or more, which no device holds)
     const uint32_t pool_ids = pool_blocks > 0xffffffffull ? 0xffffffffu : (uint32_t)pool_blocks;
@@ -932,6 +1098,7 @@ void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS) {
         }
     };
     bool bad_id = false;                    // flagged once, after the tile loop
+    using Half = typename Q8Stage<D>::Half;
     auto resolved = [&](int k) -> Half {    // a half of the last resolved tile
         const bool bad = nx_in[k] && nx_blk[k] >= pool_ids;
         bad_id |= bad;
@@ -942,93 +1109,23 @@ void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS) {
         const uint32_t p0 = t * TP;
         const Half h0 = resolved(0), h1 = resolved(1);
         if (t + 1 < ntiles) resolve(t + 1);
-        xk[0] = u2v{0u, 0u};
-        xk[1] = u2v{0u, 0u};
-        xv = u4v{0u, 0u, 0u, 0u};
-        xvs = u2v{0u, 0u};
-        xks = 0u;
-        const Half &hp = (sp & 16u) ? h1 : h0;
-        if (hp.base != nullptr && p0 + sp < n_wg) {
-            const uint32_t rw = hp.row0 + (sp & 15u);
-            xk[0] = *(const u2v *)(hp.base + geo.k_off + rw * D + 8u * kchunk[0]);
-            xk[1] = *(const u2v *)(hp.base + geo.k_off + rw * D + 8u * kchunk[1]);
-            xv = *(const u4v *)(hp.base + geo.v_off + rw * D + 16u * sj);
-            xvs = *(const u2v *)(hp.base + geo.vs_off + rw * (D / 16));
-        }
-        // K scales: threads 0..63, position tid / 2, word tid % 2
-        const uint32_t pk = threadIdx.x >> 1;
-        const Half &hk = (pk & 16u) ? h1 : h0;
-        if (threadIdx.x < 64u && hk.base != nullptr && p0 + pk < n_wg)
-            xks = *(const uint32_t *)(hk.base + geo.ks_off + (hk.row0 + (pk & 15u)) * (D / 16) +
-                                      4u * (threadIdx.x & 1u));
+        stage.load(h0, h1, p0 < n_wg ? n_wg - p0 : 0u, geo);
     };
-    auto store = [&](Q8PrefillSlot<D> &sl) {
-        // K: each loaded 8-byte chunk is one logical 8-value piece, stored at its slot
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const h4 a = i8x4_to_h4_vals(xk[k].x), b = i8x4_to_h4_vals(xk[k].y);
-            *(h8 *)(sl.k + (klr * CPR + kslot[k]) * 8) =
-                h8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-        }
-        // V: stored byte c * 8 + 2 gr + u holds d = 32 gr + 2 c + u; this piece holds
-        // c = 2 sj, 2 sj + 1: for each group gr, d = 32 gr + 4 sj .. +3 from bytes
-        // 2 gr, 2 gr + 1, 8 + 2 gr, 9 + 2 gr
-        bool big = false;
-#pragma unroll
-        for (int gr = 0; gr < 4; gr++) {
-            const uint32_t w0 = xv[gr >> 1], w1 = xv[2 + (gr >> 1)];
-            h2 x01, x23;
-            if (gr & 1) {
-                x01 = __builtin_bit_cast(h2, i8x2_to_h2<2>(w0));
-                x23 = __builtin_bit_cast(h2, i8x2_to_h2<2>(w1));
-            } else {
-                x01 = __builtin_bit_cast(h2, i8x2_to_h2<0>(w0));
-                x23 = __builtin_bit_cast(h2, i8x2_to_h2<0>(w1));
-            }
-            const uint32_t sbits = (xvs[gr >> 1] >> (16u * (gr & 1u))) & 0xffffu;
-            const _Float16 sc = __builtin_bit_cast(_Float16, (uint16_t)sbits);
-            // |scale| above 512 (f16 0x6000), infinities included, NaN (above 0x7c00) not
-            big |= (sbits & 0x7fffu) - 0x6001u < 0x7c00u - 0x6000u;
-            const h2 s2 = {sc, sc};
-            h2 a = x01 * s2, b = x23 * s2;       // high parts (rounded products)
-            asm volatile("" : "+v"(a), "+v"(b));  // not contracted into the residuals
-            const h2 ra = __builtin_elementwise_fma(x01, s2, -a);
-            const h2 rb = __builtin_elementwise_fma(x23, s2, -b);
-            const uint32_t P = 4u * gr + (sj >> 1), hf = sj & 1u;
-            const uint32_t off = (sp * CPR + (P ^ vswz<D>(sp))) * 8 + 4 * hf;
-            *(h4 *)(sl.vh + off) = h4{a[0], a[1], b[0], b[1]};
-            *(h4 *)(sl.vl + off) = h4{ra[0], ra[1], rb[0], rb[1]};
-        }
-        if (big) flag(err, ERR_RANGE);
-        if (threadIdx.x < 64u) sl.ks[threadIdx.x] = xks;
-    };
-
     float m = -INFINITY, l = 0.0f;
     f4 acc[NDB];
 #pragma unroll
     for (int j = 0; j < NDB; j++) acc[j] = f4{0.f, 0.f, 0.f, 0.f};
 
+    // IMG: positions 8 grp .. +7 of d = 16 j + col lie in one 16-byte piece of V^T
+    auto vread_img = [&](const _Float16 *v, int j) {
+        const uint32_t dd = 16u * j + col;
+        return *(const h8 *)(v + dd * 32u + ((grp ^ ((dd >> 2) & 3u)) * 8u));
+    };
     auto kread = [&](const Q8PrefillSlot<D> &sl, int h, int ks) {
         const uint32_t r = 16u * h + col, p = 4u * ks + grp;
         return *(const h8 *)(sl.k + (r * CPR + (p ^ kswz<D>(r))) * 8);
     };
-    // transposed V read (ds_read_b64_tr_b16): lane col gets positions 8 grp .. +7 of
-    // d = 16 j + col
-    auto vread = [&](const _Float16 *v, int j) {
-        const uint32_t sidx = lane & 15u;
-        u2v wv[2];
-#pragma unroll
-        for (int hf = 0; hf < 2; hf++) {
-            const uint32_t r = 8u * grp + 4u * hf + (sidx >> 2);
-            const uint32_t d = 16u * j + 4u * (sidx & 3u);
-            const uint32_t pc = d >> 3;
-            const _Float16 *a = v + (r * CPR + (pc ^ vswz<D>(r))) * 8 + (d & 7u);
-            typedef short s4 __attribute__((ext_vector_type(4)));
-            wv[hf] = __builtin_bit_cast(u2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                                 (__attribute__((address_space(3))) s4 *)a));
-        }
-        return __builtin_bit_cast(h8, u4v{wv[0][0], wv[0][1], wv[1][0], wv[1][1]});
-    };
+    auto vread = [&](const _Float16 *v, int j) { return vread_tr<D>(v, j); };
 
     auto tile = [&](const Q8PrefillSlot<D> &sl, uint32_t tp0) {
         if (tp0 >= n_wave) return;
@@ -1101,7 +1198,8 @@ void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS) {
         const h8 pl = __builtin_bit_cast(h8, u4v{plw[0], plw[1], plw[2], plw[3]});
 #pragma unroll
         for (int j = 0; j < NDB; j++) {
-            const h8 bh = vread(sl.vh, j), bl = vread(sl.vl, j);
+            const h8 bh = IMG ? vread_img(sl.vh, j) : vread(sl.vh, j);
+            const h8 bl = IMG ? vread_img(sl.vl, j) : vread(sl.vl, j);
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, bh, acc[j], 0, 0, 0);
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, bh, acc[j], 0, 0, 0);
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, bl, acc[j], 0, 0, 0);
@@ -1114,16 +1212,51 @@ void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS) {
     auto step = [&](uint32_t t, const Q8PrefillSlot<D> &cur, Q8PrefillSlot<D> &nxt) {
         if (t + 1 < ntiles) load(t + 1);
         tile(cur, t * TP);
-        if (t + 1 < ntiles) store(nxt);
+        if (t + 1 < ntiles) stage.store(nxt, err);
         __syncthreads();
     };
-    resolve(t_first);
-    load(t_first);
-    store(sb0);
-    __syncthreads();
-    for (uint32_t t = t_first; t < ntiles; t += 2) {
-        step(t, sb0, sb1);
-        if (t + 1 < ntiles) step(t + 1, sb1, sb0);
+    if constexpr (!IMG) {
+        resolve(t_first);
+        load(t_first);
+        stage.store(sb0, err);
+        __syncthreads();
+        for (uint32_t t = t_first; t < ntiles; t += 2) {
+            step(t, sb0, sb1);
+            if (t + 1 < ntiles) step(t + 1, sb1, sb0);
+        }
+    } else {
+        const uint8_t *const head_img = img + (uint64_t)sg * img_tiles * sizeof(Q8PrefillSlot<D>);
+        const uint32_t ws_ = [&]() { return __builtin_amdgcn_readfirstlane(w); }();
+        auto issue = [&](uint32_t t, Q8PrefillSlot<D> &sl) {
+            const uint8_t *from = head_img + (uint64_t)t * sizeof(Q8PrefillSlot<D>);
+            uint8_t *to = (uint8_t *)&sl;
+#pragma unroll
+            for (uint32_t x = 0; x < 6; x++) {  // K, V high, V residual: 6 x 4 KiB
+                const uint8_t *src = from + (x * 4096u + threadIdx.x * 16u);
+                uint8_t *lds_dst = to + (x * 4096u + ws_ * 1024u);
+                __builtin_amdgcn_global_load_lds(src, lds_dst, 16, 0, 0);
+            }
+            if (ws_ == 0 && lane < 16u) {       // the key scales: 256 bytes
+                const uint8_t *src = from + (24576u + lane * 16u);
+                uint8_t *lds_dst = to + 24576u;
+                __builtin_amdgcn_global_load_lds(src, lds_dst, 16, 0, 0);
+            }
+        };
+        // tile t has landed everywhere and every wave is past tile t - 1, whose slot tile
+        // t + 1 then streams into (a bare barrier, as in k_prefill_f16)
+        auto istep = [&](uint32_t t, Q8PrefillSlot<D> &cur, Q8PrefillSlot<D> &nxt) {
+            __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), lgkmcnt(0)
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (t + 1 < ntiles) issue(t + 1, nxt);
+            tile(cur, t * TP);
+        };
+        issue(t_first, sb0);
+        for (uint32_t t = t_first; t < ntiles; t += 2) {
+            istep(t, sb0, sb1);
+            if (t + 1 < ntiles) istep(t + 1, sb1, sb0);
+        }
     }
     if (bad_id && threadIdx.x == 0) flag(err, ERR_BLOCK);
     if (!wave_live) return;
@@ -1245,6 +1378,17 @@ int check_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t ma
     return QVKV_OK;
 }
 
+// The parts that each group of row blocks is cut into (row_block), so that few groups make a
+// multiple of 8, and the launch's workgroups.
+static uint32_t sub_groups(uint64_t groups, uint32_t n_qb) {
+    uint32_t n_sub = 1;
+    while (groups < 128 && groups * n_sub % 8 != 0 && n_sub * 2 <= n_qb) n_sub *= 2;
+    return n_sub;
+}
+static unsigned prefill_grid(uint64_t groups, uint32_t n_sub, uint32_t n_qb) {
+    return (unsigned)((groups * n_sub + 7) / 8 * 8 * ((n_qb + n_sub - 1) / n_sub));
+}
+
 // Which kernel a prefill launch runs.
 enum class PrefillForm { GENERIC, TILE, F16, Q8 };
 static PrefillForm prefill_form(const Geometry &g, bool f16_values) {
@@ -1271,10 +1415,23 @@ PrefillPlan plan_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint
     // 512-token chunk at 8 k (256 blocks of 272 tiles) 188 -> 124 us with 3; d = 64, the same
     // chunk by 1 / 2 / 3 / 4 / 6: 132 / 83 / 76 / 75 / 78.
     const uint64_t cus = 256, slots = (form == PrefillForm::F16 && g.D == 64 ? 4 : 3) * cus;
-    const uint64_t blocks =
-        (uint64_t)n_seg * g.G * (((uint64_t)max_tok * (heads / (uint32_t)g.G) + 63) / 64);
+    const uint64_t n_qb = ((uint64_t)max_tok * (heads / (uint32_t)g.G) + 63) / 64;
     const uint64_t tiles = ((uint64_t)max_pos + 32) / 32;
-    const double tile_us = form == PrefillForm::Q8 ? 2.2 : g.D == 64 ? 0.84 : 1.14;
+    // q8_0: tile images where enough row blocks share them (knob prefill_images: the least
+    // number), for as many segments at once as 512 MiB hold.  Measured at 2 k positions, 16
+    // segments, without / with images: 4 row blocks 143 / 150 us, 8 247 / 234, 16 427 / 388, 64 1839 /
+    // 1533; 4 segments at 8 k: 8 blocks 213 / 217, 32 794 / 685.
+    const uint64_t seg_img = (uint64_t)g.G * tiles * sizeof(Q8PrefillSlot<128>);
+    const int share = tune(KNOB_PREFILL_IMAGES);
+    if (form == PrefillForm::Q8 && share > 0 && n_qb >= (uint64_t)share && seg_img <= PREFILL_IMAGE_BYTES) {
+        const uint64_t fit = PREFILL_IMAGE_BYTES / seg_img;
+        p.img_segs = fit < n_seg ? (uint32_t)fit : n_seg;
+        p.img_tiles = (uint32_t)tiles;
+        p.img_bytes = (p.img_segs * seg_img + 255) / 256 * 256;
+        n_seg = p.img_segs;
+    }
+    const uint64_t blocks = (uint64_t)n_seg * g.G * n_qb;
+    const double tile_us = form == PrefillForm::Q8 ? (p.img_segs ? 1.8 : 2.1) : g.D == 64 ? 0.84 : 1.14;
     const int forced = tune(KNOB_PREFILL_CHUNKS);
     double best = 0.0;
     for (uint32_t n = 1; n <= PREFILL_MAX_CHUNKS; n++) {
@@ -1289,7 +1446,8 @@ PrefillPlan plan_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint
             p.n_chunks = n;
         }
     }
-    if (p.n_chunks > 1) p.ws_bytes = blocks * p.n_chunks * 64ull * (uint64_t)(g.D + 2) * 4ull;
+    p.ws_bytes = p.img_bytes;
+    if (p.n_chunks > 1) p.ws_bytes += blocks * p.n_chunks * 64ull * (uint64_t)(g.D + 2) * 4ull;
     return p;
 }
 
@@ -1315,23 +1473,51 @@ hipError_t launch_prefill(const Geometry &g, const PrefillPlan &plan, const void
     }
     const uint32_t GS = heads / (uint32_t)g.G;
     const PrefillForm form = prefill_form(g, f16_values);
+    if (form == PrefillForm::Q8 && plan.img_segs) {  // segments by as many as the images hold
+        const uint32_t n_qb = (uint32_t)(((uint64_t)max_tok * GS + 63) / 64), n_ch = plan.n_chunks;
+        uint8_t *img = (uint8_t *)ws;
+        float *part = (float *)(img + plan.img_bytes);
+        for (uint32_t s0 = 0; s0 < n_seg; s0 += plan.img_segs) {
+            const uint32_t ns = n_seg - s0 < plan.img_segs ? n_seg - s0 : plan.img_segs;
+            const uint64_t row_blocks = (uint64_t)ns * g.G * n_qb;
+            const uint32_t n_sub = sub_groups((uint64_t)ns * g.G * n_ch, n_qb);
+            const unsigned grid = prefill_grid((uint64_t)ns * g.G * n_ch, n_sub, n_qb);
+            hipLaunchKernelGGL(k_q8_images<128>, dim3((unsigned)((uint64_t)ns * g.G * plan.img_tiles)),
+                               dim3(256), 0, s, pp, pool_blocks, blocks, n_table, table_at + s0,
+                               pos0 + s0, q_at + s0, n_tok + s0, max_pos, max_tok, q_rows, geo, err,
+                               img, plan.img_tiles);
+            hipLaunchKernelGGL((k_prefill_q8<128, true>), dim3(grid), dim3(256), 0, s, pp, pool_blocks,
+                               q, blocks, n_table, table_at + s0, pos0 + s0, q_at + s0, n_tok + s0, ns,
+                               heads, max_pos, max_tok, q_rows, n_qb, out, geo, err, n_ch, n_sub, part,
+                               row_blocks * n_ch, img, plan.img_tiles);
+            if (n_ch > 1)
+                hipLaunchKernelGGL(k_prefill_merge<128>, dim3((unsigned)(row_blocks * 8)), dim3(256), 0, s,
+                                   part, n_table, table_at + s0, pos0 + s0, q_at + s0, n_tok + s0, heads,
+                                   max_pos, max_tok, q_rows, n_qb, out, geo, n_ch, row_blocks * n_ch);
+            hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     if (form == PrefillForm::F16 || form == PrefillForm::Q8) {
         const uint32_t n_qb = (uint32_t)(((uint64_t)max_tok * GS + 63) / 64);
         const uint32_t n_ch = plan.n_chunks;
         const uint64_t row_blocks = (uint64_t)n_seg * g.G * n_qb;
-        // groups of row blocks (row_block), and the parts that make their number a multiple of 8
         const uint64_t groups = (uint64_t)n_seg * g.G * n_ch;
-        uint32_t n_sub = 1;
-        while (groups < 128 && groups * n_sub % 8 != 0 && n_sub * 2 <= n_qb) n_sub *= 2;
-        const unsigned grid2 = (unsigned)((groups * n_sub + 7) / 8 * 8 * ((n_qb + n_sub - 1) / n_sub));
-        const unsigned pad = form == PrefillForm::F16 ? (unsigned)tune(KNOB_PREFILL_LDS_PAD) : 0u;
+        const uint32_t n_sub = sub_groups(groups, n_qb);
+        const unsigned grid2 = prefill_grid(groups, n_sub, n_qb);
+        const unsigned pad = (unsigned)tune(KNOB_PREFILL_LDS_PAD);
 #define QV_PF2(KERNEL)                                                                         \
     hipLaunchKernelGGL(KERNEL, dim3(grid2), dim3(256), pad, s, pp, pool_blocks, q, blocks,       \
                        n_table, table_at, pos0, q_at, n_tok, n_seg, heads, max_pos, max_tok,    \
                        q_rows, n_qb, out, geo, err, n_ch, n_sub, (float *)ws, row_blocks * n_ch)
         // P as one f16 (the default) or as high part + residual (knob prefill_exact_p=1)
         const bool ps = tune(KNOB_PREFILL_EXACT_P) != 0;
-        if (form == PrefillForm::Q8) QV_PF2((k_prefill_q8<128>));
+        if (form == PrefillForm::Q8)
+            hipLaunchKernelGGL((k_prefill_q8<128, false>), dim3(grid2), dim3(256), 0, s, pp, pool_blocks,
+                               q, blocks, n_table, table_at, pos0, q_at, n_tok, n_seg, heads, max_pos,
+                               max_tok, q_rows, n_qb, out, geo, err, n_ch, n_sub, (float *)ws,
+                               row_blocks * n_ch, nullptr, 0u);
 #define QV_PF2_D(DD)                                                                           \
     do {                                                                                        \
         if (tune(KNOB_PREFILL_DMA)) {                                                           \
