@@ -380,6 +380,53 @@ __device__ __forceinline__ void load_tile_of(Tile<D, Q8> &t, uint32_t tt, uint32
     }
 }
 
+// A q8_0 tile (index tt, in block blk) by buffer loads: the tile's four parts (keys, values and
+// their scales) are scalar bases, and the lane's offset into each never changes, so a fetch
+// needs no vector address arithmetic and no address registers that could clash with loads in
+// flight.  A bad block, or live == false, reads zeros without touching memory (no records), so
+// that a pipelined loop fetches without a branch.  blk and tt are wave-uniform.
+template <int D>
+__device__ __forceinline__ void fetch_tile_q8(Tile<D, true> &t, uint32_t tt, uint32_t blk, bool live,
+                                              const uint8_t *pool, uint64_t pool_blocks, uint32_t g,
+                                              uint32_t c, uint32_t qg, const Geo &geo, int *err) {
+    constexpr int NT = 2, RS = D / 32 * 2;  // cache policy: non-temporal; bytes of a row's scales
+    const uint32_t B = (uint32_t)geo.B;
+    t.p0 = tt * 16u;
+    t.ok = live && blk < pool_blocks;
+    if (live && blk >= pool_blocks && (threadIdx.x & 63u) == 0) flag(err, ERR_BLOCK);
+    const uint8_t *base = pool + (t.ok ? (uint64_t)blk * geo.bb : 0ull);
+    const uint64_t rows = (uint64_t)g * B + (t.p0 - geo.fd_b.div(t.p0) * B);  // the tile's first row
+    auto part = [&](uint64_t off, int row_bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(base + off + rows * row_bytes), 0,
+                                                 t.ok ? 16 * row_bytes : 0, 0x00027000);
+    };
+    const auto rk = part(geo.k_off, D), rks = part(geo.ks_off, RS);
+    const auto rv = part(geo.v_off, D), rvs = part(geo.vs_off, RS);
+    auto get16 = [](auto rsrc, int at, uint32_t *w) {
+        const u4v x = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, NT));
+        w[0] = x.x; w[1] = x.y; w[2] = x.z; w[3] = x.w;
+    };
+#pragma unroll
+    for (int i = 0; i < D / 64; i++) get16(rk, (int)(c * D + qg * (D / 4)) + 16 * i, t.k + 4 * i);
+#pragma unroll
+    for (int i = 0; i < D / 64; i++) get16(rks, (int)(4 * qg * RS) + 16 * i, t.ks + 4 * i);
+#pragma unroll
+    for (int i = 0; i < D / 64; i++) get16(rvs, (int)(4 * qg * RS) + 16 * i, t.vs + 4 * i);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int at = (int)(4 * qg * D + c * (D / 16)) + i * D;
+        if constexpr (D == 64) {
+            t.v[i][0] = __builtin_amdgcn_raw_buffer_load_b32(rv, at, 0, NT);
+        } else if constexpr (D == 128) {
+            const u2v x = __builtin_bit_cast(u2v, __builtin_amdgcn_raw_buffer_load_b64(rv, at, 0, NT));
+            t.v[i][0] = x.x;
+            t.v[i][1] = x.y;
+        } else {
+            get16(rv, at, t.v[i]);
+        }
+    }
+}
+
 template <int D, bool Q8, bool NT>
 __device__ __forceinline__ void load_tile(Tile<D, Q8> &t, uint32_t tt, const uint8_t *pool,
                                           uint64_t pool_blocks, const uint32_t *blocks,

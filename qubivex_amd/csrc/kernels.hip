@@ -907,9 +907,9 @@ __global__ __launch_bounds__(T) void k_block_copy(uint8_t *__restrict__ pool,
     pool, pool_blocks, q, blocks, n_table, table_at, pos, n_items, H, max_pos, out, ws, hc_n,   \
         n_chunks, tpc, geo, err, nr
 
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS = false, int NW = 4>
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS = false, int NW = 4, bool PIPE = false>
 __device__ __forceinline__ void attn_body(QV_ATTN_PARAMS);
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS = false, int NW = 4>
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS = false, int NW = 4, bool PIPE = false>
 __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint64_t pool_blocks,
                                           const float *__restrict__ q,
                                           const uint32_t *__restrict__ blocks, uint32_t H,
@@ -918,9 +918,9 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
                                           uint32_t t_end, float *o_base, uint64_t o_stride,
                                           float *ml_base, uint64_t ml_stride, NewRows nr);
 
-template <int D, bool Q8, bool NT, bool PK>
+template <int D>
 __global__ __launch_bounds__(256) void k_attn_mfma(QV_ATTN_PARAMS) {
-    attn_body<D, Q8, NT, PK, false>(QV_ATTN_ARGS);
+    attn_body<D, false, true, false, false>(QV_ATTN_ARGS);
 }
 // The fused append + attention form (f16; new rows in nr): a separate build, so the plain
 // kernel keeps its registers, held to the plain kernel's occupancy (3 waves/SIMD; 1 at
@@ -937,18 +937,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 void k_attn_mfma_ids(QV_ATTN_PARAMS) {
     attn_body<D, false, true, false, false, true>(QV_ATTN_ARGS);
 }
-// q8_0: held to the plain q8_0 kernel's occupancy (4 waves/SIMD at d = 128)
-template <int D, bool PK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 4 : 1)))
-void k_attn_mfma_q8nr(QV_ATTN_PARAMS) {
-    attn_body<D, true, true, PK, true>(QV_ATTN_ARGS);
+// q8_0, plain and with the new rows (NR).  PIPE (d = 64, 128): the next tile's loads in flight
+// during this tile's arithmetic, at 3 waves/SIMD at d = 128; else one tile at a time at 4.
+// Measured in us, one tile at a time / pipelined: a layer of 64 x 2048, 8 KV heads, fused 65.0 /
+// 56.1, plain 61.9 / 54.8; 256 x 2048 212 / 199; 128 x 8192, 4 KV heads 217 / 193; d = 64,
+// 64 x 2048 48.7 / 37.7.  (A tile costs a wave about 1.5 us at 2 waves/SIMD, a third of it
+// arithmetic.)
+template <int D, bool PK, bool NR, bool PIPE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D != 128 ? 1 : PIPE ? 3 : 4)))
+void k_attn_mfma_q8(QV_ATTN_PARAMS) {
+    attn_body<D, true, true, PK, NR, false, 4, PIPE>(QV_ATTN_ARGS);
 }
 
-// The same kernel held to the registers of W waves per SIMD (512 / W per lane).
-template <int D, bool Q8, bool NT, bool PK, int W>
+// The f16 kernel held to the registers of W waves per SIMD (512 / W per lane).
+template <int D, int W>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W)))
 void k_attn_mfma_w(QV_ATTN_PARAMS) {
-    attn_body<D, Q8, NT, PK, false>(QV_ATTN_ARGS);
+    attn_body<D, false, true, false, false>(QV_ATTN_ARGS);
 }
 
 // Launches of few short units: one workgroup of 12 waves (d = 128) or 16 (d = 64) on each, so
@@ -957,10 +962,10 @@ constexpr int wide_waves(int D) { return D == 64 ? 16 : 12; }
 template <int D, bool Q8, bool PK, bool NR>
 __global__ __launch_bounds__(64 * wide_waves(D)) __attribute__((amdgpu_waves_per_eu(wide_waves(D) / 4)))
 void k_attn_wide(QV_ATTN_PARAMS) {
-    attn_body<D, Q8, true, PK, NR, true, wide_waves(D)>(QV_ATTN_ARGS);
+    attn_body<D, Q8, true, PK, NR, true, wide_waves(D), Q8>(QV_ATTN_ARGS);
 }
 
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS, int NW>
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS, int NW, bool PIPE>
 __device__ __forceinline__ void attn_body(QV_ATTN_PARAMS) {
     const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
     const uint32_t GS = H / G;
@@ -998,14 +1003,71 @@ __device__ __forceinline__ void attn_body(QV_ATTN_PARAMS) {
 
     const uint64_t oh0 = (uint64_t)item * H + (uint64_t)g * GS + hc * 8;
     if (n_chunks == 1) {
-        attn_unit<D, Q8, NT, PK, NR, IDS, NW>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
+        attn_unit<D, Q8, NT, PK, NR, IDS, NW, PIPE>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
                                  t_begin, t_end, out + oh0 * D, D, nullptr, 0, nr);
     } else {
         float *ml = ws + (uint64_t)n_items * H * n_chunks * D;
-        attn_unit<D, Q8, NT, PK, NR, IDS, NW>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
+        attn_unit<D, Q8, NT, PK, NR, IDS, NW, PIPE>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
                                  t_begin, t_end, ws + (oh0 * n_chunks + chunk) * D,
                                  (uint64_t)n_chunks * D, ml + (oh0 * n_chunks + chunk) * 2,
                                  (uint64_t)n_chunks * 2, nr);
+    }
+}
+
+// Tiles tt, tt + step, .. below t_end of a q8_0 unit by one wave (tt and step wave-uniform).  The
+// table entries of the wave's next 64 tiles are fetched one per lane ahead of the tiles; a
+// tile's block id is then a lane read into a scalar register.  NR: the unit's last tile holds
+// the appended position, patched from nrow.  PIPE: the next tile's loads are issued before
+// this tile's arithmetic (two tiles' registers).
+template <int D, bool PK, bool NR, bool PIPE>
+__device__ __forceinline__ void q8_tiles(const uint8_t *__restrict__ pool, uint64_t pool_blocks,
+                                         const uint32_t *__restrict__ blocks, const Geo &geo, int *err,
+                                         uint32_t g, uint32_t hc, uint32_t n, uint32_t tab, uint32_t tt,
+                                         uint32_t t_end, uint32_t step, const float *nrow, const h4 *qf,
+                                         SoftmaxState<D> &st, uint32_t c, uint32_t qg, bool hi_col,
+                                         uint32_t sigma) {
+    const uint32_t B = (uint32_t)geo.B, lane = threadIdx.x & 63u;
+    const uint32_t t_last = NR ? (n - 1) / 16 : t_end;
+    uint32_t ids = 0, k = 0;
+    auto fetch = [&](Tile<D, true> &t, uint32_t at) {
+        if (k == 0) {
+            const uint32_t tl = at + step * lane;
+            ids = tl < t_end ? blocks[tab + geo.fd_b.div(tl * 16u)] : 0u;
+        }
+        fetch_tile_q8<D>(t, at, __builtin_amdgcn_readlane(ids, k), at < t_end, pool, pool_blocks, g, c, qg,
+                         geo, err);
+        k = (k + 1) & 63u;
+    };
+    auto take = [&](Tile<D, true> &t, uint32_t at) {
+        if (NR && at == t_last && t.ok) {  // (the block is valid)
+            // the first head chunk also stores the rows
+            uint8_t *base = hc == 0 ? (uint8_t *)pool + (uint64_t)blocks[tab + (n - 1) / B] * geo.bb : nullptr;
+            const uint64_t rowidx = (uint64_t)g * B + (n - 1) % B;
+            q8_patch_new_row<D>(t, (n - 1) & 15u, nrow, nrow + D,
+                                base ? base + geo.k_off + rowidx * D : nullptr,
+                                base ? base + geo.ks_off + rowidx * (D / 32) * 2u : nullptr,
+                                base ? base + geo.v_off + rowidx * D : nullptr,
+                                base ? base + geo.vs_off + rowidx * (D / 32) * 2u : nullptr, c, qg);
+        }
+        compute_tile<D, true, PK>(t, st, qf, n, n, qg, hi_col, sigma);
+    };
+    if constexpr (!PIPE) {
+        for (; tt < t_end; tt += step) {
+            Tile<D, true> cur;
+            fetch(cur, tt);
+            take(cur, tt);
+        }
+    } else {
+        Tile<D, true> a, b;
+        if (tt < t_end) fetch(a, tt);
+        for (; tt < t_end; tt += 2 * step) {
+            fetch(b, tt + step);
+            __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the arithmetic
+            take(a, tt);
+            fetch(a, tt + 2 * step);
+            __builtin_amdgcn_sched_barrier(0);
+            if (tt + step < t_end) take(b, tt + step);
+        }
     }
 }
 
@@ -1014,7 +1076,7 @@ __device__ __forceinline__ void attn_body(QV_ATTN_PARAMS) {
 // the NW waves.  Head hh's result goes to o_base[hh * o_stride + d]: the output (ml_base
 // null) or, for part of the context, the unnormalised partial with its max and sum at
 // ml_base[hh * ml_stride] (log2 domain).
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS, int NW>
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool IDS, int NW, bool PIPE>
 __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint64_t pool_blocks,
                                           const float *__restrict__ q,
                                           const uint32_t *__restrict__ blocks, uint32_t H,
@@ -1077,33 +1139,8 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
     for (int j = 0; j < NJ; j++) st.acc[j] = f4{0.f, 0.f, 0.f, 0.f};
 
     if constexpr (Q8) {
-        // The table entries of the wave's next 64 tiles are fetched one per lane ahead of
-        // the tiles; a tile's block id is then a lane read into a scalar register.
-        // NR: the unit's last tile holds the appended position, patched from nrow
-        const uint32_t t_last = NR ? (n - 1) / 16 : t_end;
-        uint32_t ids = 0;
-        for (uint32_t tt = t_begin + w, k = 0; tt < t_end; tt += NW, k = (k + 1) & 63u) {
-            if (k == 0) {
-                const uint32_t tl = tt + NW * lane;
-                ids = tl < t_end ? blocks[tab + tl * 16u / B] : 0u;
-            }
-            Tile<D, Q8> cur;
-            load_tile_of<D, Q8, NT>(cur, tt, __builtin_amdgcn_readlane(ids, k), pool, pool_blocks,
-                                    g, c, qg, geo, err);
-            if (NR && tt == t_last && cur.ok) {  // (the block is valid)
-                // the first head chunk also stores the rows
-                uint8_t *base = hc == 0 ? (uint8_t *)pool + (uint64_t)blocks[tab + (n - 1) / B] * geo.bb
-                                        : nullptr;
-                const uint64_t rowidx = (uint64_t)g * B + (n - 1) % B;
-                q8_patch_new_row<D>(cur, (n - 1) & 15u, nrow, nrow + D,
-                                    base ? base + geo.k_off + rowidx * D : nullptr,
-                                    base ? base + geo.ks_off + rowidx * (D / 32) * 2u : nullptr,
-                                    base ? base + geo.v_off + rowidx * D : nullptr,
-                                    base ? base + geo.vs_off + rowidx * (D / 32) * 2u : nullptr,
-                                    c, qg);
-            }
-            compute_tile<D, Q8, PK>(cur, st, qf, n, n, qg, hi_col, sigma);
-        }
+        q8_tiles<D, PK, NR, PIPE>(pool, pool_blocks, blocks, geo, err, g, hc, n, tab, t_begin + w, t_end, NW,
+                                  nrow, qf, st, c, qg, hi_col, sigma);
     } else {
         // NR: the unit's last tile holds the appended position; its wave takes it after
         // the loop (the same order), so the loop body is the plain kernel's
@@ -1201,7 +1238,7 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
 // Tiles t0 .. t1-1 of one unit by one wave (attn_unit's tile loop over consecutive tiles), left
 // in LDS as the wave's unnormalised rows o[8][D] with their max m[8] (log2 domain) and sum l[8].
 // nrow: the wave's own 2 D floats for the new rows (q8_0 NR).
-template <int D, bool Q8, bool NT, bool PK, bool NR>
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool PIPE>
 __device__ __forceinline__ void attn_wave(const uint8_t *__restrict__ pool, uint64_t pool_blocks,
                                           const float *__restrict__ q,
                                           const uint32_t *__restrict__ blocks, uint32_t H,
@@ -1249,29 +1286,8 @@ __device__ __forceinline__ void attn_wave(const uint8_t *__restrict__ pool, uint
 #pragma unroll
     for (int j = 0; j < NJ; j++) st.acc[j] = f4{0.f, 0.f, 0.f, 0.f};
     if constexpr (Q8) {
-        uint32_t ids = 0;  // the table entries of the next 64 tiles, one per lane
-        for (uint32_t tt = t0, k = 0; tt < t1; tt++, k = (k + 1) & 63u) {
-            if (k == 0) {
-                const uint32_t tl = tt + lane;
-                ids = tl < t1 ? blocks[tab + tl * 16u / B] : 0u;
-            }
-            Tile<D, Q8> cur;
-            load_tile_of<D, Q8, NT>(cur, tt, __builtin_amdgcn_readlane(ids, k), pool, pool_blocks,
-                                    g, c, qg, geo, err);
-            if (NR && tt == t_last && cur.ok) {  // (the block is valid)
-                // the first head chunk also stores the rows
-                uint8_t *base = hc == 0 ? (uint8_t *)pool + (uint64_t)blocks[tab + (n - 1) / B] * geo.bb
-                                        : nullptr;
-                const uint64_t rowidx = (uint64_t)g * B + (n - 1) % B;
-                q8_patch_new_row<D>(cur, (n - 1) & 15u, nrow, nrow + D,
-                                    base ? base + geo.k_off + rowidx * D : nullptr,
-                                    base ? base + geo.ks_off + rowidx * (D / 32) * 2u : nullptr,
-                                    base ? base + geo.v_off + rowidx * D : nullptr,
-                                    base ? base + geo.vs_off + rowidx * (D / 32) * 2u : nullptr,
-                                    c, qg);
-            }
-            compute_tile<D, Q8, PK>(cur, st, qf, n, n, qg, hi_col, sigma);
-        }
+        q8_tiles<D, PK, NR, PIPE>(pool, pool_blocks, blocks, geo, err, g, hc, n, tab, t0, t1, 1u, nrow, qf,
+                                      st, c, qg, hi_col, sigma);
     } else {
         uint32_t tt = t0;
         asm volatile("" : "+v"(tt));  // a vector loop: see attn_unit
@@ -1426,7 +1442,7 @@ __device__ __forceinline__ uint64_t uni(uint64_t v) {
            __builtin_amdgcn_readfirstlane((uint32_t)v);
 }
 
-template <int D, bool Q8, bool NT, bool PK, bool NR>
+template <int D, bool Q8, bool NT, bool PK, bool NR, bool PIPE = false>
 __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
     constexpr uint32_t NO_UNIT = 0xffffffffu;
     extern __shared__ __attribute__((aligned(16))) uint64_t cum[];  // [n_items + 1]
@@ -1493,7 +1509,7 @@ __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
         // is taken only by the wave's last unit)
         const bool whole = starts && ends;
         const uint32_t slot = 2 * wv + (whole || n_units != 0 ? 1u : 0u);
-        attn_wave<D, Q8, NT, PK, NR>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
+        attn_wave<D, Q8, NT, PK, NR, PIPE>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
                                      t0, t1, nr, &so[slot][0][0], sm[slot], sl[slot], nrow[wv]);
         if (whole) {
             lds_order();
@@ -1563,9 +1579,9 @@ __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
     }
 }
 
-template <int D, bool Q8, bool NT, bool PK>
+template <int D>
 __global__ __launch_bounds__(256) void k_attn_stream(QV_STREAM_PARAMS) {
-    attn_stream_body<D, Q8, NT, PK, false>(pool, pool_blocks, q, blocks, n_table, table_at, pos, n_items,
+    attn_stream_body<D, false, true, false, false>(pool, pool_blocks, q, blocks, n_table, table_at, pos, n_items,
                                     H, max_pos, out, ws, hc_n, ucost, geo, err, nr);
 }
 template <int D>
@@ -1575,15 +1591,15 @@ void k_attn_stream_nr(QV_STREAM_PARAMS) {
                                                   table_at, pos, n_items, H, max_pos, out, ws,
                                                   hc_n, ucost, geo, err, nr);
 }
-// (3 waves/SIMD at d = 128: at the plain stream kernel's 4 its registers spill.  Its q8_0
-// tile code is the 4-wave builds' source; the 3-wave builds' wrong outputs were the
-// v_exp_f32 -> inline-asm v_mul_legacy_f32 wait state, now in the asm itself.)
-template <int D, bool PK>
+// q8_0, plain and with the new rows: 3 waves/SIMD at d = 128 (the workgroups that a CU takes),
+// where two tiles' registers no longer fit (32 x 4096 in us, pipelined / not: plain 66 / 65, fused
+// 81 / 67); pipelined at d = 64.
+template <int D, bool PK, bool NR, bool PIPE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 3 : 1)))
-void k_attn_stream_q8nr(QV_STREAM_PARAMS) {
-    attn_stream_body<D, true, true, PK, true>(pool, pool_blocks, q, blocks, n_table, table_at,
-                                              pos, n_items, H, max_pos, out, ws, hc_n, ucost, geo,
-                                              err, nr);
+void k_attn_stream_q8(QV_STREAM_PARAMS) {
+    attn_stream_body<D, true, true, PK, NR, PIPE>(pool, pool_blocks, q, blocks, n_table, table_at,
+                                                  pos, n_items, H, max_pos, out, ws, hc_n, ucost, geo,
+                                                  err, nr);
 }
 
 // Merge for k_attn_stream: block = one (item, query head), D threads per slice of the unit's
@@ -2043,6 +2059,13 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
         p->kind = 3;
         return QVKV_OK;
     }
+    // More units than CUs, still short: unsplit, one launch again (256 units of 128-512 positions,
+    // unsplit / split, 16.7 / 22.9 us f16 d = 128, 12.9 / 17.6 d = 64, 17.1 / 23.3 q8_0; of 256-1024
+    // 25.9 / 28.8, 21.0 / 19.8, 26.5 / 26.5).
+    if (units < full && units > 256 && !split_set && max_tiles <= 48) {
+        p->tpc = (uint32_t)max_tiles;
+        return QVKV_OK;
+    }
     // Other launches too small to fill the chip with one workgroup per unit (below 2 per CU)
     // are split.  By work (k_attn_stream, the default): every wave gets an equal share
     // of the (unit, tile) pairs, whatever the contexts.  One workgroup per CU (256) while a wave
@@ -2163,46 +2186,25 @@ hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *po
     }
     float *wsf = (float *)ws;
     const bool q8 = g.dtype == QVKV_Q8_0;
-    // q8_0 at d = 128 runs its 4-wave builds (k_attn_mfma_w / k_attn_stream_w): its dequant
-    // VALU work needs the extra wave (4.82 vs 4.14 TB/s at cfg3).  The 3-wave builds
-    // (knob attn_waves3_q8) are kept for measurement and tested like the others.  f16
-    // selects its 4-wave build by the knob attn_waves4_f16 (measured slower).
-    const bool w4 = q8 ? tune(KNOB_ATTN_WAVES3_Q8) == 0 : tune(KNOB_ATTN_WAVES4_F16) != 0;
     // q8_0 with <= 4 query heads per KV head: two groups' probabilities per A operand
     const bool pk = q8 && heads / (uint32_t)g.G <= 4 && tune(KNOB_ATTN_PACK) != 0;
     if (p.kind == 2) {
         const unsigned P = p.n_chunks;
-#define QV_AS(DD, QQ, PK)                                                                       \
-    hipLaunchKernelGGL((k_attn_stream<DD, QQ, true, PK>), dim3(P), dim3(256), (n_items + 1) * 8, s, pp,          \
-                       pool_blocks, q, blocks, n_table, table_at, pos, n_items, heads, max_pos,  \
-                       out, wsf, p.hc, p.ucost, geo, err, nr)
-#define QV_AS_NR(DD)                                                                            \
-    hipLaunchKernelGGL((k_attn_stream_nr<DD>), dim3(P), dim3(256), (n_items + 1) * 8, s,                        \
-                       pp, pool_blocks, q, blocks, n_table, table_at, pos, n_items, heads,      \
-                       max_pos, out, wsf, p.hc, p.ucost, geo, err, nr)
-#define QV_AS_Q8NR(DD, PK)                                                                      \
-    hipLaunchKernelGGL((k_attn_stream_q8nr<DD, PK>), dim3(P), dim3(256), (n_items + 1) * 8, s, pp, pool_blocks,  \
-                       q, blocks, n_table, table_at, pos, n_items, heads, max_pos, out, wsf,    \
-                       p.hc, p.ucost, geo, err, nr)
-        if (q8 && nr.k) {
-            if (g.D == 64) { if (pk) QV_AS_Q8NR(64, true); else QV_AS_Q8NR(64, false); }
-            else if (g.D == 128) { if (pk) QV_AS_Q8NR(128, true); else QV_AS_Q8NR(128, false); }
-            else { if (pk) QV_AS_Q8NR(256, true); else QV_AS_Q8NR(256, false); }
-        } else if (g.D == 64) {
-            if (!q8) { if (nr.k) QV_AS_NR(64); else QV_AS(64, false, false); }
-            else if (pk) QV_AS(64, true, true);
-            else QV_AS(64, true, false);
-        } else if (g.D == 128) {
-            if (!q8) { if (nr.k) QV_AS_NR(128); else QV_AS(128, false, false); }
-            else if (pk) QV_AS(128, true, true);
-            else QV_AS(128, true, false);
-        } else {
-            if (!q8) { if (nr.k) QV_AS_NR(256); else QV_AS(256, false, false); }
-            else if (pk) QV_AS(256, true, true);
-            else QV_AS(256, true, false);
-        }
-#undef QV_AS_Q8NR
-#undef QV_AS_NR
+#define QV_AS(KERNEL)                                                                           \
+    hipLaunchKernelGGL(KERNEL, dim3(P), dim3(256), (n_items + 1) * 8, s, pp, pool_blocks, q,     \
+                       blocks, n_table, table_at, pos, n_items, heads, max_pos, out, wsf, p.hc, \
+                       p.ucost, geo, err, nr)
+#define QV_AS_Q8(DD, PK, PIPE)                                                                  \
+    do { if (nr.k) QV_AS((k_attn_stream_q8<DD, PK, true, PIPE>));                                \
+         else QV_AS((k_attn_stream_q8<DD, PK, false, PIPE>)); } while (0)
+#define QV_AS_D(DD, PIPE)                                                                       \
+    do { if (q8) { if (pk) QV_AS_Q8(DD, true, PIPE); else QV_AS_Q8(DD, false, PIPE); }           \
+         else if (nr.k) QV_AS(k_attn_stream_nr<DD>); else QV_AS(k_attn_stream<DD>); } while (0)
+        if (g.D == 64) QV_AS_D(64, true);
+        else if (g.D == 128) QV_AS_D(128, false);
+        else QV_AS_D(256, false);
+#undef QV_AS_D
+#undef QV_AS_Q8
 #undef QV_AS
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -2238,58 +2240,36 @@ hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *po
     // launch of every layer lost 2-4 % with it)
     const bool per_layer = grid < (uint64_t)tune(KNOB_ATTN_IDS_BELOW);
     // K/V tiles are streamed with non-temporal loads (read once).
-    // Occupancy: `mode` 0 is the compiler's register choice (3 waves/SIMD at d=128), 4
-    // holds the kernel to 4 waves per SIMD (125 VGPRs, no spill).  Measured (cfg5 f16,
-    // cfg3 q8_0): f16 is best at 0 (6.48 vs 5.90 TB/s), q8_0 at 4 (4.82 vs 4.14 TB/s):
-    // the q8_0 tile has about twice the VALU work per byte and more waves hide it.
-    // Software pipelining one tile ahead (2 waves/SIMD) and 5 waves/SIMD (spills) were
-    // slower for both.
-#define QV_ATTN(DD, QQ, PK)                                                                     \
-    hipLaunchKernelGGL((k_attn_mfma<DD, QQ, true, PK>), dim3((unsigned)grid), dim3(256), 0, s,  \
-                       pp, pool_blocks, q, blocks, n_table, table_at, pos, n_items, heads,      \
-                       max_pos, out, wsf, p.hc, p.n_chunks, p.tpc, geo, err, nr)
-#define QV_ATTN_W4(DD, QQ, PK)                                                                  \
-    hipLaunchKernelGGL((k_attn_mfma_w<DD, QQ, true, PK, 4>), dim3((unsigned)grid), dim3(256),   \
-                       0, s, pp, pool_blocks, q, blocks, n_table, table_at, pos, n_items,       \
-                       heads, max_pos, out, wsf, p.hc, p.n_chunks, p.tpc, geo, err, nr)
-#define QV_ATTN_NR(DD)                                                                          \
-    hipLaunchKernelGGL((k_attn_mfma_nr<DD>), dim3((unsigned)grid),                              \
-                       dim3(256), 0, s, pp, pool_blocks, q, blocks, n_table, table_at, pos,     \
-                       n_items, heads, max_pos, out, wsf, p.hc, p.n_chunks, p.tpc, geo, err, nr)
-#define QV_ATTN_IDS(DD)                                                                         \
-    hipLaunchKernelGGL((k_attn_mfma_ids<DD>), dim3((unsigned)grid), dim3(256), 0, s, pp,        \
-                       pool_blocks, q, blocks, n_table, table_at, pos, n_items, heads, max_pos,  \
-                       out, wsf, p.hc, p.n_chunks, p.tpc, geo, err, nr)
-#define QV_ATTN_Q8NR(DD, PK)                                                                    \
-    hipLaunchKernelGGL((k_attn_mfma_q8nr<DD, PK>), dim3((unsigned)grid), dim3(256), 0, s, pp,    \
-                       pool_blocks, q, blocks, n_table, table_at, pos, n_items, heads, max_pos,  \
-                       out, wsf, p.hc, p.n_chunks, p.tpc, geo, err, nr)
-    if (q8 && nr.k) {
-        if (g.D == 64) { if (pk) QV_ATTN_Q8NR(64, true); else QV_ATTN_Q8NR(64, false); }
-        else if (g.D == 128) { if (pk) QV_ATTN_Q8NR(128, true); else QV_ATTN_Q8NR(128, false); }
-        else { if (pk) QV_ATTN_Q8NR(256, true); else QV_ATTN_Q8NR(256, false); }
+    // Occupancy: f16 runs at the compiler's register choice (3 waves/SIMD at d = 128; the 4-wave
+    // build, knob attn_waves4_f16, 5.90 against 6.48 TB/s at cfg5), q8_0 at d = 128 pipelined at
+    // 3 (attn_waves3_q8 = 1: one tile at a time at 4).  Pipelining the f16 loop one tile ahead
+    // (2 waves/SIMD) and 5 waves/SIMD (spills) were slower.
+#define QV_ATTN(KERNEL)                                                                         \
+    hipLaunchKernelGGL(KERNEL, dim3((unsigned)grid), dim3(256), 0, s, pp, pool_blocks, q, blocks, \
+                       n_table, table_at, pos, n_items, heads, max_pos, out, wsf, p.hc,         \
+                       p.n_chunks, p.tpc, geo, err, nr)
+#define QV_ATTN_Q8_(DD, PK, PIPE)                                                               \
+    do { if (nr.k) QV_ATTN((k_attn_mfma_q8<DD, PK, true, PIPE>));                                \
+         else QV_ATTN((k_attn_mfma_q8<DD, PK, false, PIPE>)); } while (0)
+#define QV_ATTN_Q8(DD, PIPE)                                                                    \
+    do { if (pk) QV_ATTN_Q8_(DD, true, PIPE); else QV_ATTN_Q8_(DD, false, PIPE); } while (0)
+    if (q8) {
+        if (g.D == 64) QV_ATTN_Q8(64, true);
+        else if (g.D == 256) QV_ATTN_Q8(256, false);
+        else if (tune(KNOB_ATTN_WAVES3_Q8) == 0) QV_ATTN_Q8(128, true);
+        else QV_ATTN_Q8(128, false);
     } else if (g.D == 64) {
-        if (!q8) { if (nr.k) QV_ATTN_NR(64); else QV_ATTN(64, false, false); }
-        else if (pk) QV_ATTN(64, true, true);
-        else QV_ATTN(64, true, false);
+        if (nr.k) QV_ATTN(k_attn_mfma_nr<64>); else QV_ATTN(k_attn_mfma<64>);
     } else if (g.D == 128) {
-        if (!q8) {
-            if (nr.k) QV_ATTN_NR(128);
-            else if (w4) QV_ATTN_W4(128, false, false);
-            else if (per_layer) QV_ATTN_IDS(128);
-            else QV_ATTN(128, false, false);
-        }
-        else if (pk) { if (w4) QV_ATTN_W4(128, true, true); else QV_ATTN(128, true, true); }
-        else { if (w4) QV_ATTN_W4(128, true, false); else QV_ATTN(128, true, false); }
+        if (nr.k) QV_ATTN(k_attn_mfma_nr<128>);
+        else if (tune(KNOB_ATTN_WAVES4_F16)) QV_ATTN((k_attn_mfma_w<128, 4>));
+        else if (per_layer) QV_ATTN(k_attn_mfma_ids<128>);
+        else QV_ATTN(k_attn_mfma<128>);
     } else {
-        if (!q8) { if (nr.k) QV_ATTN_NR(256); else QV_ATTN(256, false, false); }
-        else if (pk) QV_ATTN(256, true, true);
-        else QV_ATTN(256, true, false);
+        if (nr.k) QV_ATTN(k_attn_mfma_nr<256>); else QV_ATTN(k_attn_mfma<256>);
     }
-#undef QV_ATTN_Q8NR
-#undef QV_ATTN_IDS
-#undef QV_ATTN_NR
-#undef QV_ATTN_W4
+#undef QV_ATTN_Q8
+#undef QV_ATTN_Q8_
 #undef QV_ATTN
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.n_chunks == 1) return e;
