@@ -184,12 +184,18 @@ struct RowBlock {
 };
 __device__ __forceinline__ RowBlock row_block(uint32_t n_cb, uint32_t n_ch, uint32_t n_sub,
                                               bool xcd_map) {
-    const uint32_t bid = blockIdx.x, per = (n_cb + n_sub - 1) / n_sub;
-    const uint32_t i = xcd_map ? bid / 8 : bid;
-    const uint32_t part = xcd_map ? i / per * 8 + bid % 8 : i / per;
-    const uint32_t at = i % per * n_sub + part % n_sub, group = part / n_sub;
+    // n_sub is a power of two (sub_groups).  A division by a runtime value is tens of
+    // instructions before the first load: one here, and one more where the launch is split
+    // (8 segments of 8 to 64 tokens on 2 047 cached, 32 heads: 45.9 -> 45.5 us).
+    const uint32_t lg = (uint32_t)__builtin_ctz(n_sub), per = (n_cb + n_sub - 1) >> lg;
+    const uint32_t bid = blockIdx.x;
+    const uint32_t i = xcd_map ? bid / 8 : bid, q = i / per;
+    const uint32_t part = xcd_map ? q * 8 + bid % 8 : q;
+    const uint32_t at = ((i - q * per) << lg) + (part & (n_sub - 1)), group = part >> lg;
     // (at >= n_cb, in a last part: past every block, as n_cb - 1 - at wraps)
-    return RowBlock{n_cb - 1 - at, group % n_ch, group / n_ch};
+    if (n_ch == 1) return RowBlock{n_cb - 1 - at, 0u, group};
+    const uint32_t sg = group / n_ch;
+    return RowBlock{n_cb - 1 - at, group - sg * n_ch, sg};
 }
 
 // One wave's 16 rows (row rw0 + 4 (lane / 16) + i at d = 16 j + lane % 16), normalised to
@@ -1378,8 +1384,8 @@ int check_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t ma
     return QVKV_OK;
 }
 
-// The parts that each group of row blocks is cut into (row_block), so that few groups make a
-// multiple of 8, and the launch's workgroups.
+// The parts, a power of two, that each group of row blocks is cut into (row_block), so that
+// few groups make a multiple of 8, and the launch's workgroups.
 static uint32_t sub_groups(uint64_t groups, uint32_t n_qb) {
     uint32_t n_sub = 1;
     while (groups < 128 && groups * n_sub % 8 != 0 && n_sub * 2 <= n_qb) n_sub *= 2;
