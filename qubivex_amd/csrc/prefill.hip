@@ -678,7 +678,10 @@ void k_prefill_f16(QV_PREFILL_SPLIT_PARAMS) {
                     __builtin_amdgcn_global_load_lds(src, lds_dst, 16, 0, 0);
                 }
             } else {
-                // past n_wg or a bad block: through registers, zeros where invalid
+                // past n_wg or a bad block: through registers, zeros where invalid.  This tile
+                // adds no DMA (and, with no valid position, no load), so the counted wait of
+                // the next step would not see that tile t - 1's has landed: wait for it here.
+                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
 #pragma unroll
                 for (int u = 0; u < CPT; u++) {
                     const uint32_t c = chunk_u(u);
@@ -725,8 +728,9 @@ void k_prefill_f16(QV_PREFILL_SPLIT_PARAMS) {
                 return __builtin_bit_cast(h8, u4v{w[0][0], w[0][1], w[1][0], w[1][1]});
             };
         };
-        // waits: this thread's chunks of tile t have landed when at most `ahead` tiles'
-        // chunks (CPT instructions each) are still outstanding
+        // waits: the wave's chunks of tile t have landed when at most CPT loads are still
+        // outstanding.  Tile t + 1 either has its CPT in flight, or went through registers,
+        // after a wait for everything before it (issue).
         auto wait_tile = [&](uint32_t t) {
             if (t + 1 < ntiles) {
                 __builtin_amdgcn_s_waitcnt(0x0f70 | CPT);  // vmcnt(CPT)

@@ -150,3 +150,28 @@ def check_asm(asm_text):
     for name, lines in kernels(asm_text).items():
         out += check_kernel(name, lines)
     return out
+
+
+def lds_dma_stores_without_wait(lines):
+    """Indexes of the LDS stores, in a kernel that streams into LDS by DMA with counted waits,
+    that no ``s_waitcnt vmcnt(0)`` precedes since the last DMA, barrier or uniform branch.  Such a
+    kernel counts a tile's DMA instructions to know that an older tile has landed; a tile
+    that is stored from registers adds none, so the wave has to drain its older ones first."""
+    ls = [ln.split(";")[0].strip() for ln in lines]
+    uniform = set()  # labels that a uniform branch reaches
+    for ln in ls:
+        m = re.match(r"s_c?branch(?:_(?:scc|vcc)\w+)?\s+(\.L\w+)", ln)
+        if m and "exec" not in ln:
+            uniform.add(m.group(1))
+    bad = []
+    for i, ln in enumerate(ls):
+        if not re.match(r"ds_(write|store)_b", ln):
+            continue
+        for p in reversed(ls[:i]):
+            if p.startswith("s_waitcnt") and "vmcnt(0)" in p:
+                break
+            if (p.startswith(("global_load_lds", "s_barrier", "s_branch", "s_cbranch_scc", "s_cbranch_vcc"))
+                    or (p.endswith(":") and p[:-1] in uniform)):
+                bad.append(i)
+                break
+    return bad

@@ -104,3 +104,21 @@ def test_no_kernel_uses_flat_memory_instructions(texts):
             if n:
                 bad.append((src, name, n))
     assert bad == [], bad
+
+
+def test_checker_finds_a_register_store_beside_dma_in_flight():
+    dma = "global_load_lds_dwordx4 v[2:3], off\ns_cbranch_vccnz .LBB0_2\n"
+    store = "ds_write_b128 v4, v[6:9]\n.LBB0_2:\ns_waitcnt vmcnt(2)\ns_barrier"
+    assert H.lds_dma_stores_without_wait((dma + store).splitlines()) == [2]
+    assert H.lds_dma_stores_without_wait((dma + "s_waitcnt vmcnt(0)\n" + store).splitlines()) == []
+
+
+def test_f16_prefill_drains_its_dma_before_register_tiles(texts):
+    """The streaming f16 prefill waits for a tile by counting the next one's DMA instructions.  A
+    tile stored from registers (a partial half, a bad block) issues none, so every one of its
+    stores comes after a wait for all older DMA: without it the other waves could read a tile
+    that has not landed."""
+    found = {name: H.lds_dma_stores_without_wait(lines) for name, lines in H.kernels(texts["prefill.hip"]).items()
+             if "k_prefill_f16" in name and any("global_load_lds" in ln for ln in lines)}
+    assert len(found) == 4  # d = 64 and 128, P as one f16 and exact
+    assert not any(found.values()), found
