@@ -23,6 +23,7 @@
 #include <string.h>
 
 #include "device.h"
+#include "gather_grid.h"
 
 namespace qvkv {
 
@@ -546,7 +547,42 @@ __device__ __forceinline__ void store_f8(float *dst, const float *y) {
     st_g_nt((f4v *)(dst + 4), f4v{y[4], y[5], y[6], y[7]});
 }
 
-// T threads per workgroup; UF: loads in flight per thread (f16 pools).
+// The (item, tile) units of a one-wave workgroup, u0, u0 + step, .. below n_items * tiles_max, those
+// past their item's end left out.  Units are ordered item by item, or (by_tile) tile by tile, in
+// which a batch of uneven items spreads evenly over the workgroups.  After the first unit the
+// lanes look at 64 at a time: one that has nothing to do costs a few instructions.
+template <typename F>
+__device__ __forceinline__ void each_live_tile(uint32_t u0, uint32_t step, uint32_t n_items,
+                                               uint32_t tiles_max, bool by_tile,
+                                               const uint32_t *__restrict__ lens, F &&body) {
+    const uint32_t units = n_items * tiles_max, lane = threadIdx.x & 63u;
+    if (u0 >= units) return;
+    const uint32_t by = by_tile ? n_items : tiles_max;
+    const uint32_t q = u0 / by, r = u0 - q * by;
+    uint32_t item = by_tile ? r : q, tile = by_tile ? q : r, len = lens[item];
+    uint32_t next = u0 + step, items = 0, tiles = 0, ls = 0;  // lane l: the l-th of the 64 last looked at
+    uint64_t live = 0;                                        // those still to do
+    for (;;) {
+        if (tile * 16u < len) body(item, tile, len);
+        while (live == 0) {
+            if (next >= units) return;
+            const uint32_t u = next + lane * step, uq = u / by, ur = u - uq * by;
+            items = by_tile ? ur : uq;
+            tiles = by_tile ? uq : ur;
+            ls = u < units ? lens[items] : 0u;
+            live = __ballot(tiles * 16u < ls);
+            next += 64u * step;
+        }
+        const int k = __builtin_ctzll(live);
+        live &= live - 1;
+        item = __builtin_amdgcn_readlane(items, k);
+        tile = __builtin_amdgcn_readlane(tiles, k);
+        len = __builtin_amdgcn_readlane(ls, k);
+    }
+}
+
+// T threads per workgroup; UF: loads in flight per thread (f16 pools).  One-wave workgroups of
+// the f32 form walk several units (each_live_tile), the others take one each.
 template <int DT, int OUT, int T = 256, int UF = 8>
 __global__ __launch_bounds__(T) void k_gather(const uint8_t *__restrict__ pool,
                                                 uint64_t pool_blocks,
@@ -557,149 +593,154 @@ __global__ __launch_bounds__(T) void k_gather(const uint8_t *__restrict__ pool,
                                                 const uint64_t *__restrict__ out_at,
                                                 uint32_t n_items, uint32_t tiles_max,
                                                 uint64_t out_positions, void *out_k,
-                                                void *out_v, uint32_t parts, Geo geo, int *err) {
+                                                void *out_v, uint32_t parts, bool by_tile, Geo geo,
+                                                int *err) {
     // parts workgroups share one tile (each one batch of loads and stores of it)
     const uint32_t part = blockIdx.x % parts, bt = blockIdx.x / parts;
-    const uint32_t item = bt / tiles_max;
-    const uint32_t tile = bt - item * tiles_max;
-    if (item >= n_items) return;
-    const uint32_t len = lens[item];
-    const uint32_t p0 = tile * 16u;
-    if (p0 >= len) return;
-    const uint32_t D = (uint32_t)geo.D, B = (uint32_t)geo.B, G = (uint32_t)geo.G;
-    const uint32_t tab = table_at[item];
-    const uint32_t nblk = (len + B - 1) / B;
-    if ((uint64_t)tab + nblk > n_table) {
-        if (threadIdx.x == 0) flag(err, ERR_TABLE);
-        return;
-    }
-    const uint64_t oat = out_at[item];
-    if (oat + len > out_positions) {
-        if (threadIdx.x == 0) flag(err, ERR_OUT);
-        return;
-    }
-    const uint32_t blk = blocks[tab + p0 / B];
-    if (blk >= pool_blocks) {
-        if (threadIdx.x == 0) flag(err, ERR_BLOCK);
-        return;
-    }
-    const uint32_t r0 = p0 % B;
-    const uint8_t *base = pool + (uint64_t)blk * geo.bb;
-    const uint32_t c8 = D >> 3;                 // 8-value chunks per row
-    const uint32_t per_kv = G * 16u * c8;       // chunks per tile for K (or V)
-    if (DT == QVKV_F16 && OUT == QVKV_F16) {
-        // A byte copy of the tile's rows: UF loads in flight per thread, then UF stores.
-        constexpr int U = UF;
-        for (uint32_t b0 = part * (uint32_t)T * U; b0 < 2u * per_kv; b0 += parts * (uint32_t)T * U) {
-            u4v x[U];
-            uint16_t *dst[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                dst[u] = nullptr;
-                const uint32_t idx = b0 + u * (uint32_t)T + threadIdx.x;
-                if (idx >= 2u * per_kv) continue;
-                const bool isv = idx >= per_kv;
-                uint32_t r = isv ? idx - per_kv : idx;
-                const uint32_t e = (r % c8) * 8u;
-                r /= c8;
-                const uint32_t row = r & 15u, g = r >> 4, p = p0 + row;
-                if (p >= len) continue;
-                x[u] = __builtin_nontemporal_load(
-                    (const u4v *)(base + (isv ? geo.v_off : geo.k_off) +
-                                  (((uint64_t)g * B + r0 + row) * D + e) * 2u));
-                dst[u] = (uint16_t *)(isv ? out_v : out_k) + oat * (uint64_t)G * D +
-                         ((uint64_t)g * len + p) * D + e;
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                if (dst[u]) st_g_nt((u4v *)dst[u], x[u]);
+    auto one_tile = [&](uint32_t item, uint32_t tile, uint32_t len) {
+        const uint32_t p0 = tile * 16u;
+        if (p0 >= len) return;
+        const uint32_t D = (uint32_t)geo.D, B = (uint32_t)geo.B, G = (uint32_t)geo.G;
+        const uint32_t tab = table_at[item];
+        const uint32_t nblk = (len + B - 1) / B;
+        if ((uint64_t)tab + nblk > n_table) {
+            if (threadIdx.x == 0) flag(err, ERR_TABLE);
+            return;
         }
-        return;
-    }
-    if (DT == QVKV_F16 && OUT == QVKV_F32) {
-        // f16 -> f32: 4 values per thread (an 8-byte load, a 16-byte store), so
-        // consecutive lanes store consecutive 16-byte pieces and every store instruction
-        // covers whole output lines; UF loads in flight per thread.
-        const uint32_t c4 = D >> 2;
-        const uint32_t per4 = G * 16u * c4;
-        constexpr int U = UF;
-        for (uint32_t b0 = part * (uint32_t)T * U; b0 < 2u * per4; b0 += parts * (uint32_t)T * U) {
-            u2v x[U];
-            float *dst[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                dst[u] = nullptr;
-                const uint32_t idx = b0 + u * (uint32_t)T + threadIdx.x;
-                if (idx >= 2u * per4) continue;
-                const bool isv = idx >= per4;
-                uint32_t r = isv ? idx - per4 : idx;
-                const uint32_t e = (r % c4) * 4u;
-                r /= c4;
-                const uint32_t row = r & 15u, g = r >> 4, p = p0 + row;
-                if (p >= len) continue;
-                x[u] = __builtin_nontemporal_load(
-                    (const u2v *)(base + (isv ? geo.v_off : geo.k_off) +
-                                  (((uint64_t)g * B + r0 + row) * D + e) * 2u));
-                dst[u] = (float *)(isv ? out_v : out_k) + oat * (uint64_t)G * D +
-                         ((uint64_t)g * len + p) * D + e;
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (!dst[u]) continue;
-                const uint32_t w0 = x[u].x, w1 = x[u].y;
-                const h2 a = __builtin_bit_cast(h2, w0), b = __builtin_bit_cast(h2, w1);
-                st_g_nt((f4v *)dst[u], f4v{(float)a.x, (float)a.y, (float)b.x, (float)b.y});
-            }
+        const uint64_t oat = out_at[item];
+        if (oat + len > out_positions) {
+            if (threadIdx.x == 0) flag(err, ERR_OUT);
+            return;
         }
-        return;
-    }
-    for (uint32_t idx = part * 256u + threadIdx.x; idx < 2u * per_kv; idx += parts * 256u) {
-        const bool isv = idx >= per_kv;
-        uint32_t r = isv ? idx - per_kv : idx;
-        const uint32_t e = (r % c8) * 8u;
-        r /= c8;
-        const uint32_t row = r & 15u;
-        const uint32_t g = r >> 4;
-        const uint32_t p = p0 + row;
-        if (p >= len) continue;
-        const uint64_t rowidx = (uint64_t)g * B + r0 + row;
-        // out element offset: out_at*G*d + (g*len + p)*d + e
-        const uint64_t o = oat * (uint64_t)G * D + ((uint64_t)g * len + p) * D + e;
-        if (DT == QVKV_F16) {
-            const uint4 x = *(const uint4 *)(base + (isv ? geo.v_off : geo.k_off) +
-                                              (rowidx * D + e) * 2u);
-            if (OUT == QVKV_F16) {
-                st_g_nt((u4v *)((uint16_t *)(isv ? out_v : out_k) + o), u4v{x.x, x.y, x.z, x.w});
-            } else {
-                h2 a = __builtin_bit_cast(h2, x.x), b = __builtin_bit_cast(h2, x.y);
-                h2 c = __builtin_bit_cast(h2, x.z), d2 = __builtin_bit_cast(h2, x.w);
-                const float y[8] = {(float)a.x, (float)a.y, (float)b.x, (float)b.y,
-                                    (float)c.x, (float)c.y, (float)d2.x, (float)d2.y};
+        const uint32_t blk = blocks[tab + p0 / B];
+        if (blk >= pool_blocks) {
+            if (threadIdx.x == 0) flag(err, ERR_BLOCK);
+            return;
+        }
+        const uint32_t r0 = p0 % B;
+        const uint8_t *base = pool + (uint64_t)blk * geo.bb;
+        const uint32_t c8 = D >> 3;                 // 8-value chunks per row
+        const uint32_t per_kv = G * 16u * c8;       // chunks per tile for K (or V)
+        if (DT == QVKV_F16 && OUT == QVKV_F16) {
+            // A byte copy of the tile's rows: UF loads in flight per thread, then UF stores.
+            constexpr int U = UF;
+            for (uint32_t b0 = part * (uint32_t)T * U; b0 < 2u * per_kv; b0 += parts * (uint32_t)T * U) {
+                u4v x[U];
+                uint16_t *dst[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    dst[u] = nullptr;
+                    const uint32_t idx = b0 + u * (uint32_t)T + threadIdx.x;
+                    if (idx >= 2u * per_kv) continue;
+                    const bool isv = idx >= per_kv;
+                    uint32_t r = isv ? idx - per_kv : idx;
+                    const uint32_t e = (r % c8) * 8u;
+                    r /= c8;
+                    const uint32_t row = r & 15u, g = r >> 4, p = p0 + row;
+                    if (p >= len) continue;
+                    x[u] = __builtin_nontemporal_load(
+                        (const u4v *)(base + (isv ? geo.v_off : geo.k_off) +
+                                      (((uint64_t)g * B + r0 + row) * D + e) * 2u));
+                    dst[u] = (uint16_t *)(isv ? out_v : out_k) + oat * (uint64_t)G * D +
+                             ((uint64_t)g * len + p) * D + e;
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (dst[u]) st_g_nt((u4v *)dst[u], x[u]);
+            }
+            return;
+        }
+        if (DT == QVKV_F16 && OUT == QVKV_F32) {
+            // f16 -> f32: 4 values per thread (an 8-byte load, a 16-byte store), so
+            // consecutive lanes store consecutive 16-byte pieces and every store instruction
+            // covers whole output lines; UF loads in flight per thread.
+            const uint32_t c4 = D >> 2;
+            const uint32_t per4 = G * 16u * c4;
+            constexpr int U = UF;
+            for (uint32_t b0 = part * (uint32_t)T * U; b0 < 2u * per4; b0 += parts * (uint32_t)T * U) {
+                u2v x[U];
+                float *dst[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    dst[u] = nullptr;
+                    const uint32_t idx = b0 + u * (uint32_t)T + threadIdx.x;
+                    if (idx >= 2u * per4) continue;
+                    const bool isv = idx >= per4;
+                    uint32_t r = isv ? idx - per4 : idx;
+                    const uint32_t e = (r % c4) * 4u;
+                    r /= c4;
+                    const uint32_t row = r & 15u, g = r >> 4, p = p0 + row;
+                    if (p >= len) continue;
+                    x[u] = __builtin_nontemporal_load(
+                        (const u2v *)(base + (isv ? geo.v_off : geo.k_off) +
+                                      (((uint64_t)g * B + r0 + row) * D + e) * 2u));
+                    dst[u] = (float *)(isv ? out_v : out_k) + oat * (uint64_t)G * D +
+                             ((uint64_t)g * len + p) * D + e;
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    if (!dst[u]) continue;
+                    const uint32_t w0 = x[u].x, w1 = x[u].y;
+                    const h2 a = __builtin_bit_cast(h2, w0), b = __builtin_bit_cast(h2, w1);
+                    st_g_nt((f4v *)dst[u], f4v{(float)a.x, (float)a.y, (float)b.x, (float)b.y});
+                }
+            }
+            return;
+        }
+        for (uint32_t idx = part * 256u + threadIdx.x; idx < 2u * per_kv; idx += parts * 256u) {
+            const bool isv = idx >= per_kv;
+            uint32_t r = isv ? idx - per_kv : idx;
+            const uint32_t e = (r % c8) * 8u;
+            r /= c8;
+            const uint32_t row = r & 15u;
+            const uint32_t g = r >> 4;
+            const uint32_t p = p0 + row;
+            if (p >= len) continue;
+            const uint64_t rowidx = (uint64_t)g * B + r0 + row;
+            // out element offset: out_at*G*d + (g*len + p)*d + e
+            const uint64_t o = oat * (uint64_t)G * D + ((uint64_t)g * len + p) * D + e;
+            if (DT == QVKV_F16) {
+                const uint4 x = *(const uint4 *)(base + (isv ? geo.v_off : geo.k_off) +
+                                                  (rowidx * D + e) * 2u);
+                if (OUT == QVKV_F16) {
+                    st_g_nt((u4v *)((uint16_t *)(isv ? out_v : out_k) + o), u4v{x.x, x.y, x.z, x.w});
+                } else {
+                    h2 a = __builtin_bit_cast(h2, x.x), b = __builtin_bit_cast(h2, x.y);
+                    h2 c = __builtin_bit_cast(h2, x.z), d2 = __builtin_bit_cast(h2, x.w);
+                    const float y[8] = {(float)a.x, (float)a.y, (float)b.x, (float)b.y,
+                                        (float)c.x, (float)c.y, (float)d2.x, (float)d2.y};
+                    store_f8((float *)(isv ? out_v : out_k) + o, y);
+                }
+            } else {  // q8_0 -> f32: y = f32(q) * f32(scale), one multiply (the reference dequant)
+                const uint8_t *rowp = base + (isv ? geo.v_off : geo.k_off) + rowidx * D;
+                const _Float16 sh = *(const _Float16 *)(base + (isv ? geo.vs_off : geo.ks_off) +
+                                                        (rowidx * (D >> 5) + (e >> 5)) * 2u);
+                const float sc = (float)sh;
+                float y[8];
+                if (!isv) {
+                    const uint2 qb = *(const uint2 *)(rowp + kperm(e, D));
+#pragma unroll
+                    for (int t = 0; t < 8; t++) {
+                        const uint32_t w = t < 4 ? qb.x : qb.y;
+                        y[t] = (float)(int8_t)(w >> (8 * (t & 3))) * sc;
+                    }
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 8; t += 2) {
+                        const uint16_t pr = *(const uint16_t *)(rowp + vperm(e + t, D));
+                        y[t] = (float)(int8_t)(pr & 0xff) * sc;
+                        y[t + 1] = (float)(int8_t)(pr >> 8) * sc;
+                    }
+                }
                 store_f8((float *)(isv ? out_v : out_k) + o, y);
             }
-        } else {  // q8_0 -> f32: y = f32(q) * f32(scale), one multiply (the reference dequant)
-            const uint8_t *rowp = base + (isv ? geo.v_off : geo.k_off) + rowidx * D;
-            const _Float16 sh = *(const _Float16 *)(base + (isv ? geo.vs_off : geo.ks_off) +
-                                                    (rowidx * (D >> 5) + (e >> 5)) * 2u);
-            const float sc = (float)sh;
-            float y[8];
-            if (!isv) {
-                const uint2 qb = *(const uint2 *)(rowp + kperm(e, D));
-#pragma unroll
-                for (int t = 0; t < 8; t++) {
-                    const uint32_t w = t < 4 ? qb.x : qb.y;
-                    y[t] = (float)(int8_t)(w >> (8 * (t & 3))) * sc;
-                }
-            } else {
-#pragma unroll
-                for (int t = 0; t < 8; t += 2) {
-                    const uint16_t pr = *(const uint16_t *)(rowp + vperm(e + t, D));
-                    y[t] = (float)(int8_t)(pr & 0xff) * sc;
-                    y[t + 1] = (float)(int8_t)(pr >> 8) * sc;
-                }
-            }
-            store_f8((float *)(isv ? out_v : out_k) + o, y);
         }
+    };
+    if constexpr (T == 64 && OUT == QVKV_F32) {
+        each_live_tile(bt, gridDim.x / parts, n_items, tiles_max, by_tile, lens, one_tile);
+    } else {
+        const uint32_t item = bt / tiles_max;
+        if (item < n_items) one_tile(item, bt - item * tiles_max, lens[item]);
     }
 }
 
@@ -709,8 +750,8 @@ __global__ __launch_bounds__(T) void k_gather(const uint8_t *__restrict__ pool,
 //     d = 32i + 8q .. +7 and 32(i+1) + 8q .. +7;
 //   V (byte c*(D/16) + 2g + u holds d = 32g + 2c + u): a piece holds NC = 256/D (>= 1)
 //     consecutive c of NG = 8/NC groups, i.e. 2*NC consecutive values of each group.
-// The row's D/32 f16 scales come in with one load.  U pieces in flight per thread, T threads
-// per workgroup, `parts` workgroups per tile.
+// The row's D/32 f16 scales come in with one load.  A workgroup is one wave; `parts` of them
+// share a tile, a piece per thread.
 template <int D>
 __device__ __forceinline__ void store_run(float *dst, const float *y, int n) {
     if (n == 8) store_f8(dst, y);
@@ -726,8 +767,8 @@ __device__ __forceinline__ void lds_order() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
-template <int D, int T, int U>
-__global__ __launch_bounds__(T) void k_gather_q8(const uint8_t *__restrict__ pool,
+template <int D>
+__global__ __launch_bounds__(64) void k_gather_q8(const uint8_t *__restrict__ pool,
                                                    uint64_t pool_blocks,
                                                    const uint32_t *__restrict__ blocks,
                                                    uint64_t n_table,
@@ -736,124 +777,110 @@ __global__ __launch_bounds__(T) void k_gather_q8(const uint8_t *__restrict__ poo
                                                    const uint64_t *__restrict__ out_at,
                                                    uint32_t n_items, uint32_t tiles_max,
                                                    uint64_t out_positions, float *out_k,
-                                                   float *out_v, uint32_t parts, Geo geo,
-                                                   int *err) {
-    const uint32_t unit = blockIdx.x / parts, part = blockIdx.x - unit * parts;
-    const uint32_t item = unit / tiles_max;
-    const uint32_t tile = unit - item * tiles_max;
-    if (item >= n_items) return;
-    const uint32_t len = lens[item];
-    const uint32_t p0 = tile * 16u;
-    if (p0 >= len) return;
-    const uint32_t B = (uint32_t)geo.B, G = (uint32_t)geo.G;
-    const uint32_t tab = table_at[item];
-    const uint32_t nblk = (len + B - 1) / B;
-    if ((uint64_t)tab + nblk > n_table) {
-        if (threadIdx.x == 0) flag(err, ERR_TABLE);
-        return;
-    }
-    const uint64_t oat = out_at[item];
-    if (oat + len > out_positions) {
-        if (threadIdx.x == 0) flag(err, ERR_OUT);
-        return;
-    }
-    const uint32_t blk = blocks[tab + p0 / B];
-    if (blk >= pool_blocks) {
-        if (threadIdx.x == 0) flag(err, ERR_BLOCK);
-        return;
-    }
-    const uint32_t r0 = p0 % B;
-    const uint8_t *base = pool + (uint64_t)blk * geo.bb;
-    // d = 128 keys: a per-wave LDS copy of the wave's 8 rows (row stride 132 floats)
-    __shared__ __attribute__((aligned(16))) float kx[T / 64][D == 128 ? 8 * 132 : 4];
-    constexpr uint32_t PR = D / 16;           // pieces per row
-    constexpr uint32_t NS = D / 32;           // scales per row
-    constexpr uint32_t NC = D >= 256 ? 1 : 256 / D, NG = 8 / NC;
-    const uint32_t per_kv = G * 16u * PR;
-    {
-        const uint32_t b0 = part * (uint32_t)(T * U);
-        u4v x[U];
-        u4v sc[U];
-        float *dst[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            dst[u] = nullptr;
-            const uint32_t idx = b0 + u * (uint32_t)T + threadIdx.x;
-            if (idx >= 2u * per_kv) continue;
-            const bool isv = idx >= per_kv;
-            const uint32_t r = isv ? idx - per_kv : idx;
-            const uint32_t j = r % PR, row = (r / PR) & 15u, g = r / (PR * 16u);
-            const uint32_t p = p0 + row;
-            if (p >= len) continue;
-            const uint64_t rowidx = (uint64_t)g * B + r0 + row;
-            x[u] = __builtin_nontemporal_load(
-                (const u4v *)(base + (isv ? geo.v_off : geo.k_off) + rowidx * D + 16u * j));
-            const uint8_t *sp = base + (isv ? geo.vs_off : geo.ks_off) + rowidx * NS * 2u;
-            if constexpr (NS == 2) sc[u] = u4v{*(const uint32_t *)sp, 0u, 0u, 0u};
-            else if constexpr (NS == 4) { const u2v t = *(const u2v *)sp; sc[u] = u4v{t.x, t.y, 0u, 0u}; }
-            else sc[u] = *(const u4v *)sp;
-            dst[u] = (isv ? out_v : out_k) + oat * (uint64_t)G * D + ((uint64_t)g * len + p) * D;
+                                                   float *out_v, uint32_t parts, bool by_tile,
+                                                   Geo geo, int *err) {
+    // d = 128 keys: an LDS copy of the wave's 8 rows (row stride 132 floats)
+    __shared__ __attribute__((aligned(16))) float kx[D == 128 ? 8 * 132 : 4];
+    const uint32_t part = blockIdx.x % parts;
+    each_live_tile(blockIdx.x / parts, gridDim.x / parts, n_items, tiles_max, by_tile, lens,
+                   [&](uint32_t item, uint32_t tile, uint32_t len) {
+        const uint32_t p0 = tile * 16u;
+        const uint32_t B = (uint32_t)geo.B, G = (uint32_t)geo.G;
+        const uint32_t tab = table_at[item];
+        const uint32_t nblk = (len + B - 1) / B;
+        if ((uint64_t)tab + nblk > n_table) {
+            if (threadIdx.x == 0) flag(err, ERR_TABLE);
+            return;
         }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (!dst[u]) continue;
-            const uint32_t idx = b0 + u * (uint32_t)T + threadIdx.x;
-            const bool isv = idx >= per_kv;
-            const uint32_t j = (isv ? idx - per_kv : idx) % PR;
-            const uint32_t w[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
-            auto qv = [&](uint32_t b) { return (float)(int8_t)(w[b >> 2] >> (8u * (b & 3u))); };
-            auto scale = [&](uint32_t grp) {
-                const uint32_t word = sc[u][grp >> 1];
-                return (float)__builtin_bit_cast(_Float16, (uint16_t)(word >> (16u * (grp & 1u))));
-            };
-            if (!isv) {
-                const uint32_t qq = (16u * j) / (D / 4), i0 = ((16u * j) % (D / 4)) / 8u;
-                if constexpr (D == 128) {
-                    // The piece's two 8-value runs go through the row's LDS copy in
-                    // logical order, and lane j writes d = 32 k + 4 j .. +3 for k = 0..3:
-                    // each store instruction then covers whole 128-byte output lines.
-                    float *rowbuf = kx[threadIdx.x >> 6] + ((threadIdx.x & 63u) >> 3) * 132u;
-#pragma unroll
-                    for (uint32_t h = 0; h < 2; h++) {
-                        const float s = scale(i0 + h);
-                        float y[8];
-#pragma unroll
-                        for (uint32_t t = 0; t < 8; t++) y[t] = qv(8u * h + t) * s;
-                        *(f4v *)(rowbuf + 32u * (i0 + h) + 8u * qq) = f4v{y[0], y[1], y[2], y[3]};
-                        *(f4v *)(rowbuf + 32u * (i0 + h) + 8u * qq + 4) = f4v{y[4], y[5], y[6], y[7]};
-                    }
-                    lds_order();
-#pragma unroll
-                    for (uint32_t k = 0; k < 4; k++)
-                        st_g_nt((f4v *)(dst[u] + 32u * k + 4u * j),
-                                *(const f4v *)(rowbuf + 32u * k + 4u * j));
-                    lds_order();
-                } else {
+        const uint64_t oat = out_at[item];
+        if (oat + len > out_positions) {
+            if (threadIdx.x == 0) flag(err, ERR_OUT);
+            return;
+        }
+        const uint32_t blk = blocks[tab + p0 / B];
+        if (blk >= pool_blocks) {
+            if (threadIdx.x == 0) flag(err, ERR_BLOCK);
+            return;
+        }
+        const uint32_t r0 = p0 % B;
+        const uint8_t *base = pool + (uint64_t)blk * geo.bb;
+        constexpr uint32_t PR = D / 16;           // pieces per row
+        constexpr uint32_t NS = D / 32;           // scales per row
+        constexpr uint32_t NC = D >= 256 ? 1 : 256 / D, NG = 8 / NC;
+        const uint32_t per_kv = G * 16u * PR;
+        const uint32_t idx = part * 64u + threadIdx.x;
+        if (idx >= 2u * per_kv) return;
+        const bool isv = idx >= per_kv;
+        const uint32_t r = isv ? idx - per_kv : idx;
+        const uint32_t j = r % PR, row = (r / PR) & 15u, g = r / (PR * 16u);
+        const uint32_t p = p0 + row;
+        if (p >= len) return;
+        const uint64_t rowidx = (uint64_t)g * B + r0 + row;
+        const u4v x = __builtin_nontemporal_load(
+            (const u4v *)(base + (isv ? geo.v_off : geo.k_off) + rowidx * D + 16u * j));
+        const uint8_t *sp = base + (isv ? geo.vs_off : geo.ks_off) + rowidx * NS * 2u;
+        u4v sc;
+        if constexpr (NS == 2) sc = u4v{*(const uint32_t *)sp, 0u, 0u, 0u};
+        else if constexpr (NS == 4) { const u2v t = *(const u2v *)sp; sc = u4v{t.x, t.y, 0u, 0u}; }
+        else sc = *(const u4v *)sp;
+        float *dst = (isv ? out_v : out_k) + oat * (uint64_t)G * D + ((uint64_t)g * len + p) * D;
+        const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+        auto qv = [&](uint32_t b) { return (float)(int8_t)(w[b >> 2] >> (8u * (b & 3u))); };
+        auto scale = [&](uint32_t grp) {
+            const uint32_t word = sc[grp >> 1];
+            return (float)__builtin_bit_cast(_Float16, (uint16_t)(word >> (16u * (grp & 1u))));
+        };
+        if (!isv) {
+            const uint32_t qq = (16u * j) / (D / 4), i0 = ((16u * j) % (D / 4)) / 8u;
+            if constexpr (D == 128) {
+                // The piece's two 8-value runs go through the row's LDS copy in
+                // logical order, and lane j writes d = 32 k + 4 j .. +3 for k = 0..3:
+                // each store instruction then covers whole 128-byte output lines.
+                float *rowbuf = kx + (threadIdx.x >> 3) * 132u;
 #pragma unroll
                 for (uint32_t h = 0; h < 2; h++) {
                     const float s = scale(i0 + h);
                     float y[8];
 #pragma unroll
                     for (uint32_t t = 0; t < 8; t++) y[t] = qv(8u * h + t) * s;
-                    store_f8(dst[u] + 32u * (i0 + h) + 8u * qq, y);
+                    *(f4v *)(rowbuf + 32u * (i0 + h) + 8u * qq) = f4v{y[0], y[1], y[2], y[3]};
+                    *(f4v *)(rowbuf + 32u * (i0 + h) + 8u * qq + 4) = f4v{y[4], y[5], y[6], y[7]};
                 }
-                }
+                lds_order();
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++)
+                    st_g_nt((f4v *)(dst + 32u * k + 4u * j),
+                            *(const f4v *)(rowbuf + 32u * k + 4u * j));
+                lds_order();
             } else {
-                const uint32_t c0 = (16u * j) / PR, g0 = ((16u * j) % PR) / 2u;
 #pragma unroll
-                for (uint32_t gi = 0; gi < NG; gi++) {
-                    const float s = scale(g0 + gi);
-                    float y[2 * NC];
+                for (uint32_t h = 0; h < 2; h++) {
+                    const float s = scale(i0 + h);
+                    float y[8];
 #pragma unroll
-                    for (uint32_t ci = 0; ci < NC; ci++) {
-                        y[2 * ci] = qv(ci * PR + 2u * gi) * s;
-                        y[2 * ci + 1] = qv(ci * PR + 2u * gi + 1u) * s;
-                    }
-                    store_run<D>(dst[u] + 32u * (g0 + gi) + 2u * c0, y, 2 * NC);
+                    for (uint32_t t = 0; t < 8; t++) y[t] = qv(8u * h + t) * s;
+                    store_f8(dst + 32u * (i0 + h) + 8u * qq, y);
                 }
             }
+            // (the branches' last stores are not merged into one after them: apart from the
+            // stores they share output lines with, they cost 20-40 % at d = 64)
+            asm volatile("; keys" ::: "memory");
+        } else {
+            const uint32_t c0 = (16u * j) / PR, g0 = ((16u * j) % PR) / 2u;
+#pragma unroll
+            for (uint32_t gi = 0; gi < NG; gi++) {
+                const float s = scale(g0 + gi);
+                float y[2 * NC];
+#pragma unroll
+                for (uint32_t ci = 0; ci < NC; ci++) {
+                    y[2 * ci] = qv(ci * PR + 2u * gi) * s;
+                    y[2 * ci + 1] = qv(ci * PR + 2u * gi + 1u) * s;
+                }
+                store_run<D>(dst + 32u * (g0 + gi) + 2u * c0, y, 2 * NC);
+            }
+            asm volatile("; values" ::: "memory");
         }
-    }
+    });
 }
 
 // ---------------------------------------------------------------------------------
@@ -1924,33 +1951,27 @@ hipError_t launch_gather(const Geometry &g, const void *pool, uint64_t pool_bloc
     const uint64_t grid = (uint64_t)tiles * n_items;
     if (grid > 0x7fffffffull) return hipErrorInvalidValue;
     const uint8_t *p = (const uint8_t *)pool;
-    // f16 tiles of many heads: several workgroups per tile, each one batch of 8 loads in
-    // flight per thread (the f16 -> f16 copy moves 8 values per load, f16 -> f32 4)
-    const uint64_t per_batch = 256ull * 8 * (out_dtype == QVKV_F16 ? 8 : 4);
+    // f16 -> f16 tiles of many heads: several workgroups per tile, each one batch of 8 loads
+    // of 8 values in flight per thread
+    const uint64_t per_batch = 256ull * 8 * 8;
     const uint64_t vals = 2ull * g.G * 16 * g.D;
     uint32_t parts = tune(KNOB_GATHER_SPLIT) ? (uint32_t)((vals + per_batch - 1) / per_batch) : 1u;
     if (g.dtype != QVKV_F16 || grid * parts > 0x7fffffffull) parts = 1;
 #define QV_GATHER(DT, OT)                                                                      \
     hipLaunchKernelGGL((k_gather<DT, OT>), dim3((unsigned)(grid * parts)), dim3(256), 0, s, p,  \
                        pool_blocks, blocks, n_table, table_at, lens, out_at, n_items, tiles,   \
-                       out_positions, out_k, out_v, parts, geo, err)
-    // One-wave workgroups, each one batch of a tile, as for the block copy: many short workgroups
-    // keep the stores, most of the traffic, spread over time.  Against 256 threads x 8 pieces (a
-    // tile per workgroup), in us: q8_0 d = 128, 64 items of 1024-2048, 236 -> 192 (1.02 GB, 5.3
-    // TB/s; 2, 4 and 8 pieces per thread 187, 191, 241), d = 64 197 -> 108 (8 pieces took 185
-    // VGPRs), d = 256 252 -> 209; f16 -> f32 with 4 pieces 228 -> 217 (1: 286, 2: 223, 8: 226).
-    // A launch whose workgroups would pass the grid's limit takes the larger ones.
-    auto fits = [&](uint64_t per_tile) { return grid * per_tile * 64 <= 0xffffffffull; };
-#define QV_GATHER_Q8T(DD, TT, UU)                                                              \
-    hipLaunchKernelGGL((k_gather_q8<DD, TT, UU>), dim3((unsigned)(grid * parts_of(TT * UU))),    \
-                       dim3(TT), 0, s, p, pool_blocks, blocks, n_table, table_at, lens, out_at, \
-                       n_items, tiles, out_positions, (float *)out_k, (float *)out_v,           \
-                       parts_of(TT * UU), geo, err)
+                       out_positions, out_k, out_v, parts, false, geo, err)
+    if (out_dtype == QVKV_F32 && grid * 256 > 0xffffffffull) return hipErrorInvalidValue;
+    auto to_f32 = [&](uint32_t per_tile) {  // (tiles * n_items is within its limit)
+        return gather_grid(n_items, tiles, per_tile, out_positions, n_table, g.B);
+    };
 #define QV_GATHER_Q8(DD)                                                                       \
     do {                                                                                        \
-        auto parts_of = [&](uint32_t n) { return (2u * (uint32_t)g.G * (uint32_t)DD + n - 1) / n; }; \
-        if (fits(parts_of(64))) QV_GATHER_Q8T(DD, 64, 1);                                        \
-        else QV_GATHER_Q8T(DD, 256, 8);                                                          \
+        const uint32_t pq = (2u * (uint32_t)g.G * (uint32_t)DD + 63u) / 64u;                     \
+        const GatherGrid gg = to_f32(pq);                                                        \
+        hipLaunchKernelGGL(k_gather_q8<DD>, dim3(gg.wgs), dim3(64), 0, s, p, pool_blocks, blocks, \
+                           n_table, table_at, lens, out_at, n_items, tiles, out_positions,      \
+                           (float *)out_k, (float *)out_v, pq, gg.by_tile, geo, err);           \
     } while (0)
     const bool q8fast = tune(KNOB_GATHER_Q8_FAST) != 0;
     if (g.dtype == QVKV_Q8_0 && q8fast && g.D == 64) QV_GATHER_Q8(64);
@@ -1966,23 +1987,23 @@ hipError_t launch_gather(const Geometry &g, const void *pool, uint64_t pool_bloc
 #define QV_G64(UU)                                                                              \
     hipLaunchKernelGGL((k_gather<QVKV_F16, QVKV_F16, 64, UU>), dim3((unsigned)(grid * parts64)),  \
                        dim3(64), 0, s, p, pool_blocks, blocks, n_table, table_at, lens, out_at,  \
-                       n_items, tiles, out_positions, out_k, out_v, parts64, geo, err)
+                       n_items, tiles, out_positions, out_k, out_v, parts64, false, geo, err)
         if (grid * parts64 > 0x7fffffffull) return hipErrorInvalidValue;
         if (UFv == 8) QV_G64(8); else if (UFv == 4) QV_G64(4); else if (UFv == 2) QV_G64(2);
         else QV_G64(1);
 #undef QV_G64
     }
     else if (g.dtype == QVKV_F16 && out_dtype == QVKV_F16) QV_GATHER(QVKV_F16, QVKV_F16);
-    else if (g.dtype == QVKV_F16 && fits((vals + 1023) / 1024)) {
-        const uint32_t pf = (uint32_t)((vals + 1023) / 1024);  // 64 threads x 4 pieces x 4 values
-        hipLaunchKernelGGL((k_gather<QVKV_F16, QVKV_F32, 64, 4>), dim3((unsigned)(grid * pf)),
-                           dim3(64), 0, s, p, pool_blocks, blocks, n_table, table_at, lens, out_at,
-                           n_items, tiles, out_positions, out_k, out_v, pf, geo, err);
+    else if (g.dtype == QVKV_F16) {
+        // 64 threads x 4 pieces x 4 values (1, 2 and 8 pieces per thread were slower)
+        const uint32_t pf = (uint32_t)((vals + 1023) / 1024);
+        const GatherGrid gg = to_f32(pf);
+        hipLaunchKernelGGL((k_gather<QVKV_F16, QVKV_F32, 64, 4>), dim3(gg.wgs), dim3(64), 0, s, p,
+                           pool_blocks, blocks, n_table, table_at, lens, out_at, n_items, tiles,
+                           out_positions, out_k, out_v, pf, gg.by_tile, geo, err);
     }
-    else if (g.dtype == QVKV_F16) QV_GATHER(QVKV_F16, QVKV_F32);
     else QV_GATHER(QVKV_Q8_0, QVKV_F32);
 #undef QV_GATHER_Q8
-#undef QV_GATHER_Q8T
 #undef QV_GATHER
     return hipGetLastError();
 }
