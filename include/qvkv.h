@@ -243,9 +243,10 @@ int qvkv_attention_noalloc_async(qvkv_dev *dev, const qvkv_layout *layout, const
  * (causally) over positions 0..pos0[i]+j of its table exactly as qvkv_attention_async
  * would for an item with pos = pos0[i]+j; max_pos bounds pos0[i]+n_tok[i]-1 and max_tok
  * bounds n_tok[i].  A launch with few rows shares each row block's context out to several
- * workgroups, whose partial results go to a workspace of the stream (grown on first use; on
- * a stream being captured that would have to grow it, the launch runs unsplit instead).  Replaces the host prefill of the reference's forward pass, which
- * stores a segment's rows and then runs math::attend per (token, head)
+ * workgroups, whose partial results go to a workspace of the stream (grown on first use).  A
+ * launch under capture never uses it: it runs unsplit, so its graph may be replayed on any
+ * stream, beside any other launch.  Replaces the host prefill of the reference's forward
+ * pass, which stores a segment's rows and then runs math::attend per (token, head)
  * (crates/qubivex-arch/src/lib.rs:1296-1320); the reference has no device prefill.
  * q8_0 pools at d = 128 use a form that holds dequantised values in f16: a value scale
  * above 512 (values that may pass 65504) makes the next qvkv_check return

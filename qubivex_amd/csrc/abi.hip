@@ -73,12 +73,10 @@ struct StreamState {
     int *d_err = nullptr;  // [0]: latched bits (ERR_*), [1]: taken by the last check
     void *ws = nullptr;    // attention workspace (partials of context chunks)
     uint64_t ws_bytes = 0;
-    // prefill workspace (partials of split row blocks): its own buffer, so that a prefill
-    // never replaces the attention workspace that a captured decode step replays with
+    // prefill workspace (partials of split row blocks, tile images): its own buffer, so that a
+    // prefill never replaces the attention workspace that a captured decode step replays with
     void *pws = nullptr;
     uint64_t pws_bytes = 0;
-    bool pws_captured = false;                          // a capture has recorded pws
-    std::vector<std::pair<void *, uint64_t>> pws_kept;  // outgrown, but recorded by a capture
     std::mutex check_mu;   // one check at a time per stream
     // The attention launches of this stream, one at a time: the workspace is grown (which
     // waits for this stream to drain) and handed to the launch under it.  Other streams'
@@ -208,11 +206,11 @@ int ensure_attention(qvkv_dev *dev, StreamState *st, const qvkv::AttnPlan &p) {
     return ensure(dev, st->stream, &st->ws, &st->ws_bytes, p.ws_bytes);
 }
 
-// A prefill plan with the stream's prefill workspace grown for its split, or the plan without
-// the split where it cannot grow: on a stream that is being captured (no allocation, no
-// wait there), and when the device has no memory for it (the unsplit launch needs none).
-// A buffer that a capture has recorded is never freed before the device closes: its graph
-// may be replayed after a larger launch.  Caller holds st->ws_mu.
+// A prefill plan with the stream's prefill workspace grown for its split and its images, or the
+// plan without either where the device has no memory for it (that launch needs none).  A launch
+// that is being captured always runs without: its graph may be replayed on any stream, beside
+// this stream's own launches and other graphs captured on it, which would all write the one
+// workspace.  Caller holds st->ws_mu.
 qvkv::PrefillPlan ensure_prefill(qvkv_dev *dev, StreamState *st, const qvkv::PrefillPlan &p) {
     if (p.ws_bytes == 0) return p;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -220,19 +218,9 @@ qvkv::PrefillPlan ensure_prefill(qvkv_dev *dev, StreamState *st, const qvkv::Pre
         (void)hipGetLastError();
         return qvkv::PrefillPlan{};
     }
-    const bool capturing = cap != hipStreamCaptureStatusNone;
-    if (st->pws_bytes < p.ws_bytes) {
-        if (capturing) return qvkv::PrefillPlan{};
-        if (st->pws_captured) {
-            st->pws_kept.push_back({st->pws, st->pws_bytes});
-            st->pws = nullptr;
-            st->pws_bytes = 0;
-            st->pws_captured = false;
-        }
-        if (ensure(dev, st->stream, &st->pws, &st->pws_bytes, p.ws_bytes) != QVKV_OK)
-            return qvkv::PrefillPlan{};
-    }
-    st->pws_captured |= capturing;
+    if (cap != hipStreamCaptureStatusNone ||
+        ensure(dev, st->stream, &st->pws, &st->pws_bytes, p.ws_bytes) != QVKV_OK)
+        return qvkv::PrefillPlan{};
     return p;
 }
 
@@ -532,7 +520,6 @@ void qvkv_close(qvkv_dev *dev) {
     for (StreamState *st : dev->streams) {
         dev_free(dev, st->ws, st->ws_bytes);
         dev_free(dev, st->pws, st->pws_bytes);
-        for (const auto &k : st->pws_kept) dev_free(dev, k.first, k.second);
         dev_free(dev, st->d_err, 256);
         delete st;
     }

@@ -85,8 +85,8 @@ def test_split_prefill_matches_the_oracle(hip, knobs, dtype, H, G, D, B, chunks)
 
 @pytest.mark.gpu
 def test_captured_split_prefill_survives_a_larger_launch(hip, knobs):
-    """A captured split launch replays from its own workspace after a later launch outgrew it; on
-    a stream without a workspace, capture takes the unsplit form and allocates nothing."""
+    """A launch captured on a stream with a workspace, and on one without, allocates nothing and
+    replays right after a later launch that outgrew the workspace."""
     from test_gpu_kernels import cf32, cu32, fill_items, layout, new_pool
 
     knobs("prefill_chunks", 4)
@@ -132,3 +132,61 @@ def test_captured_split_prefill_survives_a_larger_launch(hip, knobs):
             assert torch.equal(outs[0][:n], ref[:n])
         assert attn_errors(outs[0][:n].cpu().numpy(), outs[1][:n].cpu().numpy())[1] <= REL_L2
         hip.check(s)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F16, Q8_0])
+def test_captured_prefill_shares_no_workspace(hip, knobs, dtype):
+    """A launch captured on a warmed stream is the unsplit form without images, bit for bit, and
+    replays on another stream beside that stream's own split launches and a second graph
+    captured there, none of them waiting for another."""
+    from test_gpu_kernels import cf32, cu32, fill_items, layout, new_pool
+
+    knobs("prefill_images", 1)
+    r, H, G, D, n = rng(6), 16, 4, 128, 4
+    L = layout(dtype, G, D)
+    N = n * 38 + 3
+    pool = new_pool(L, N, fill=2)
+    blocks, table_at, _ = fill_items(hip, L, pool, N, [600] * n, r)
+    b, ta = cu32(blocks), cu32(table_at)
+    p0, qa, nt = (cu32(x) for x in (np.full(n, 536), np.arange(n) * 64, np.full(n, 64)))
+    qs = [cf32(normal(r, (n * 64, H, D))) for _ in range(3)]
+    outs = [torch.empty(n * 64 * H * D, device="cuda") for _ in range(3)]
+
+    def attend(i):
+        hip.prefill_attention(L, pool, N, qs[i], b, ta, p0, qa, nt, H, 599, 64, outs[i])
+
+    knobs("prefill_images", 0)
+    knobs("prefill_chunks", 1)
+    plain = []
+    for i in range(2):
+        attend(i)
+        plain.append(outs[i].clone())
+    knobs("prefill_images", 1)
+    knobs("prefill_chunks", 4)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        attend(2)
+        split = outs[2].clone()
+    s.synchronize()
+    graphs = []
+    for i in range(2):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            attend(i)
+        graphs.append(g)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for _ in range(4):
+        for o in outs:
+            o.zero_()
+        torch.cuda.synchronize()
+        for g, t in zip(graphs, streams):
+            with torch.cuda.stream(t):
+                g.replay()
+        with torch.cuda.stream(s):
+            attend(2)
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], plain[0]) and torch.equal(outs[1], plain[1])
+        assert torch.equal(outs[2], split)
+    hip.check(s)
