@@ -14,6 +14,7 @@
 
 #include "internal.h"
 #include "qvkv.h"
+#include "workspace.h"
 
 using qvkv::Geometry;
 
@@ -75,8 +76,7 @@ struct StreamState {
     uint64_t ws_bytes = 0;
     // prefill workspace (partials of split row blocks, tile images): its own buffer, so that a
     // prefill never replaces the attention workspace that a captured decode step replays with
-    void *pws = nullptr;
-    uint64_t pws_bytes = 0;
+    qvkv::Workspace pws;
     std::mutex check_mu;   // one check at a time per stream
     // The attention launches of this stream, one at a time: the workspace is grown (which
     // waits for this stream to drain) and handed to the launch under it.  Other streams'
@@ -97,7 +97,7 @@ struct qvkv_dev {
     // device stream's state are theirs); mu: the list of stream states (held briefly, never
     // across a wait).  Order: host_mu, then mu, then a stream's ws_mu.
     std::mutex host_mu, mu;
-    std::atomic<uint64_t> used{0}, peak{0}, refused{0};
+    std::atomic<uint64_t> used{0}, peak{0}, refused{0}, frees{0};
     std::atomic<uint64_t> uploads{0}, upload_bytes{0}, downloads{0}, download_bytes{0};
     std::atomic<uint64_t> submissions{0}, wait_ns{0}, timed{0}, gpu_ns{0}, last_gpu_ns{0};
     std::atomic<uint64_t> stream_waits{0};
@@ -181,6 +181,7 @@ void dev_free(qvkv_dev *dev, void *p, uint64_t n) {
     if (!p) return;
     (void)hipFree(p);
     dev->used.fetch_sub(n);
+    dev->frees.fetch_add(1);
 }
 
 // Grows a device buffer used only on stream `s` to at least `need` bytes (contents not
@@ -206,22 +207,42 @@ int ensure_attention(qvkv_dev *dev, StreamState *st, const qvkv::AttnPlan &p) {
     return ensure(dev, st->stream, &st->ws, &st->ws_bytes, p.ws_bytes);
 }
 
-// A prefill plan with the stream's prefill workspace grown for its split and its images, or the
-// plan without either where the device has no memory for it (that launch needs none).  A launch
-// that is being captured always runs without: its graph may be replayed on any stream, beside
-// this stream's own launches and other graphs captured on it, which would all write the one
-// workspace.  Caller holds st->ws_mu.
-qvkv::PrefillPlan ensure_prefill(qvkv_dev *dev, StreamState *st, const qvkv::PrefillPlan &p) {
+// The prefill workspace of a stream grown to `need` bytes, if the device has the memory.  Nothing
+// fails where it has not: such a call counts in neither `refused` nor the last error.
+bool grow_prefill(qvkv_dev *dev, StreamState *st, uint64_t need) {
+    auto alloc = [&](uint64_t n) -> void * {
+        void *p = nullptr;
+        if (hipMalloc(&p, n) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        account_alloc(dev, n);
+        return p;
+    };
+    auto retire = [&](void *p, uint64_t n) {
+        (void)hipStreamSynchronize(st->stream);  // its launches still read the old buffer
+        dev_free(dev, p, n);
+    };
+    return qvkv::grow(st->pws, need, qvkv::PREFILL_IMAGE_BYTES, dev->frees.load(), alloc, retire);
+}
+
+// A prefill launch's plan, with the stream's prefill workspace grown for its split and its images;
+// where the device has no memory for them, what the workspace at hand holds.  A launch that is
+// being captured always runs without: its graph may be replayed on any stream, beside this
+// stream's own launches and other graphs captured on it, which would all write the one
+// workspace.  plan(limit): the launch's plan of at most `limit` workspace bytes.  Caller holds
+// st->ws_mu.
+template <class Plan>
+qvkv::PrefillPlan ensure_prefill(qvkv_dev *dev, StreamState *st, Plan plan) {
+    const qvkv::PrefillPlan p = plan(~0ull);
     if (p.ws_bytes == 0) return p;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st->stream, &cap) != hipSuccess) {
         (void)hipGetLastError();
         return qvkv::PrefillPlan{};
     }
-    if (cap != hipStreamCaptureStatusNone ||
-        ensure(dev, st->stream, &st->pws, &st->pws_bytes, p.ws_bytes) != QVKV_OK)
-        return qvkv::PrefillPlan{};
-    return p;
+    if (cap != hipStreamCaptureStatusNone) return qvkv::PrefillPlan{};
+    return grow_prefill(dev, st, p.ws_bytes) ? p : plan(st->pws.bytes);
 }
 
 // The state of `stream`, created on first use.  Caller holds dev->mu.
@@ -519,7 +540,7 @@ void qvkv_close(qvkv_dev *dev) {
     (void)hipDeviceSynchronize();
     for (StreamState *st : dev->streams) {
         dev_free(dev, st->ws, st->ws_bytes);
-        dev_free(dev, st->pws, st->pws_bytes);
+        dev_free(dev, st->pws.p, st->pws.bytes);
         dev_free(dev, st->d_err, 256);
         delete st;
     }
@@ -850,11 +871,12 @@ int qvkv_prefill_attention_async(qvkv_dev *dev, const qvkv_layout *layout, const
     StreamState *st;
     if (int rc = state_of(dev, stream, &st)) return rc;
     std::lock_guard<std::mutex> wl(st->ws_mu);
-    const qvkv::PrefillPlan p = ensure_prefill(
-        dev, st, qvkv::plan_prefill(g, n_seg, heads, max_pos, max_tok));
+    const qvkv::PrefillPlan p = ensure_prefill(dev, st, [&](uint64_t limit) {
+        return qvkv::plan_prefill(g, n_seg, heads, max_pos, max_tok, limit);
+    });
     return launched(dev, qvkv::launch_prefill(g, p, pool, pool_blocks, q, blocks, n_table, table_at,
                                               pos0, q_at, n_tok, n_seg, heads, max_pos, max_tok,
-                                              q_rows, out, st->pws, st->d_err, st->stream),
+                                              q_rows, out, st->pws.p, st->d_err, st->stream),
                     "prefill attention launch");
 }
 
@@ -1027,12 +1049,14 @@ hipError_t attend_tokens(qvkv_dev *dev, const Geometry &g, const qvkv::AttnPlan 
                          bool f16_values = true) {
     if (sg.max_tok >= 2) {
         const uint32_t n_seg = (uint32_t)sg.n_tok.size();
-        const qvkv::PrefillPlan pp = ensure_prefill(
-            dev, dev->own, qvkv::plan_prefill(g, n_seg, heads, max_pos, sg.max_tok, f16_values));
+        std::lock_guard<std::mutex> wl(dev->own->ws_mu);
+        const qvkv::PrefillPlan pp = ensure_prefill(dev, dev->own, [&](uint64_t limit) {
+            return qvkv::plan_prefill(g, n_seg, heads, max_pos, sg.max_tok, limit, f16_values);
+        });
         return qvkv::launch_prefill(g, pp, pool, held, dq, dblocks, n_table,
                                     st.at<uint32_t>(dev, ss.ta), st.at<uint32_t>(dev, ss.p0),
                                     st.at<uint32_t>(dev, ss.qa), st.at<uint32_t>(dev, ss.nt),
-                                    n_seg, heads, max_pos, sg.max_tok, s, dout, dev->own->pws,
+                                    n_seg, heads, max_pos, sg.max_tok, s, dout, dev->own->pws.p,
                                     dev->own->d_err, dev->stream, f16_values);
     }
     return qvkv::launch_attention(g, plan, pool, held, dq, dblocks, n_table, dtable_at, dpos, s,

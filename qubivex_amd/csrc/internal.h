@@ -5,6 +5,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "prefill_plan.h"
 #include "qvkv.h"
 
 namespace qvkv {
@@ -127,20 +128,9 @@ void reset_tune();
 // Paged prefill attention over segments of consecutive tokens (kernels.hip).
 int check_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t max_tok,
                   const char **why);
-// The plan of a prefill launch: workgroups per row block (64 query rows of a (segment, KV
-// head)), and the workspace that a split launch (n_chunks > 1) keeps its partials in.
-// q8_0 launches may also keep images of their tiles there (img_segs segments at once, img_tiles
-// each per KV head, img_bytes in all); the default plan needs no workspace.
-constexpr uint32_t PREFILL_MAX_CHUNKS = 16;
-constexpr uint64_t PREFILL_IMAGE_BYTES = 512ull << 20;
-struct PrefillPlan {
-    uint32_t n_chunks = 1;
-    uint32_t img_segs = 0, img_tiles = 0;
-    uint64_t img_bytes = 0;
-    uint64_t ws_bytes = 0;
-};
+// The plan of a prefill launch within `limit` bytes of workspace (prefill_plan.h).
 PrefillPlan plan_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t max_pos,
-                         uint32_t max_tok, bool f16_values = true);
+                         uint32_t max_tok, uint64_t limit, bool f16_values = true);
 hipError_t launch_prefill(const Geometry &g, const PrefillPlan &plan, const void *pool,
                           uint64_t pool_blocks, const float *q, const uint32_t *blocks,
                           uint64_t n_table, const uint32_t *table_at, const uint32_t *pos0,

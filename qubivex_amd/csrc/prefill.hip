@@ -1411,54 +1411,14 @@ static PrefillForm prefill_form(const Geometry &g, bool f16_values) {
 }
 
 PrefillPlan plan_prefill(const Geometry &g, uint32_t n_seg, uint32_t heads, uint32_t max_pos,
-                         uint32_t max_tok, bool f16_values) {
-    PrefillPlan p;
+                         uint32_t max_tok, uint64_t limit, bool f16_values) {
+    static_assert(PREFILL_IMAGE_TILE == sizeof(Q8PrefillSlot<128>), "a tile's image");
     const PrefillForm form = prefill_form(g, f16_values);
-    if (form != PrefillForm::F16 && form != PrefillForm::Q8) return p;
-    // Chunks per row block: the count whose estimated time is least.  A CU holds 3
-    // workgroups (4 at d = 64); a 32-position tile takes a workgroup about `tile_us` with
-    // its CU full and down to 0.55-0.6 of that alone on it; each workgroup spends about
-    // 4 us outside its tiles, and a split launch 5 us more on its merge plus the partials'
-    // traffic (written and read once).  Measured at 2 k positions, f16, d = 128, in us by
-    // chunks 1 / 2 / 3 / 4 / 8: 32 row blocks 49 / 32 / 26 / 22 / 20, 128 blocks 51 / 36 /
-    // 33 / 31 / 41, 256 blocks 53 / 45 / 46 / 53 / 67, 512 blocks 65 / 83 / 81 / 92 / 134; a
-    // 512-token chunk at 8 k (256 blocks of 272 tiles) 188 -> 124 us with 3; d = 64, the same
-    // chunk by 1 / 2 / 3 / 4 / 6: 132 / 83 / 76 / 75 / 78.
-    const uint64_t cus = 256, slots = (form == PrefillForm::F16 && g.D == 64 ? 4 : 3) * cus;
-    const uint64_t n_qb = ((uint64_t)max_tok * (heads / (uint32_t)g.G) + 63) / 64;
-    const uint64_t tiles = ((uint64_t)max_pos + 32) / 32;
-    // q8_0: tile images where enough row blocks share them (knob prefill_images: the least
-    // number), for as many segments at once as 512 MiB hold.  Measured at 2 k positions, 16
-    // segments, without / with images: 4 row blocks 143 / 150 us, 8 247 / 234, 16 427 / 388, 64 1839 /
-    // 1533; 4 segments at 8 k: 8 blocks 213 / 217, 32 794 / 685.
-    const uint64_t seg_img = (uint64_t)g.G * tiles * sizeof(Q8PrefillSlot<128>);
-    const int share = tune(KNOB_PREFILL_IMAGES);
-    if (form == PrefillForm::Q8 && share > 0 && n_qb >= (uint64_t)share && seg_img <= PREFILL_IMAGE_BYTES) {
-        const uint64_t fit = PREFILL_IMAGE_BYTES / seg_img;
-        p.img_segs = fit < n_seg ? (uint32_t)fit : n_seg;
-        p.img_tiles = (uint32_t)tiles;
-        p.img_bytes = (p.img_segs * seg_img + 255) / 256 * 256;
-        n_seg = p.img_segs;
-    }
-    const uint64_t blocks = (uint64_t)n_seg * g.G * n_qb;
-    const double tile_us = form == PrefillForm::Q8 ? (p.img_segs ? 1.8 : 2.1) : g.D == 64 ? 0.84 : 1.14;
-    const int forced = tune(KNOB_PREFILL_CHUNKS);
-    double best = 0.0;
-    for (uint32_t n = 1; n <= PREFILL_MAX_CHUNKS; n++) {
-        if (n > 1 && (tiles < 2ull * n || blocks * n > 8 * slots) && forced == 0) break;
-        const uint64_t per_cu = (blocks * n % slots + cus - 1) / cus;  // of the last round
-        const double rounds = (double)(blocks * n / slots) +
-                              (per_cu == 0 ? 0.0 : 0.4 + 0.6 * (double)(per_cu * cus) / (double)slots);
-        double us = rounds * ((double)((tiles + n - 1) / n) * tile_us + 4.0);
-        if (n > 1) us += 5.0 + (double)(blocks * n) * 64.0 * (g.D + 2) * 8.0 / 4e6;
-        if (n == 1 || (forced == 0 ? us < best : (int)n <= forced)) {
-            best = us;
-            p.n_chunks = n;
-        }
-    }
-    p.ws_bytes = p.img_bytes;
-    if (p.n_chunks > 1) p.ws_bytes += blocks * p.n_chunks * 64ull * (uint64_t)(g.D + 2) * 4ull;
-    return p;
+    if (form != PrefillForm::F16 && form != PrefillForm::Q8) return PrefillPlan{};
+    return plan_prefill_shape(
+        PrefillShape{form == PrefillForm::Q8, (uint32_t)g.G, (uint32_t)g.D, heads / (uint32_t)g.G,
+                     n_seg, max_pos, max_tok, tune(KNOB_PREFILL_IMAGES), tune(KNOB_PREFILL_CHUNKS)},
+        limit);
 }
 
 hipError_t launch_prefill(const Geometry &g, const PrefillPlan &plan, const void *pool,
