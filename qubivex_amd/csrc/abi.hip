@@ -207,6 +207,14 @@ int ensure_attention(qvkv_dev *dev, StreamState *st, const qvkv::AttnPlan &p) {
     return ensure(dev, st->stream, &st->ws, &st->ws_bytes, p.ws_bytes);
 }
 
+// Allocations and waits of this thread while another stream is being captured: in the default
+// capture mode they would fail and invalidate that capture, which they have no part in.
+struct UncapturedScope {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    UncapturedScope() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~UncapturedScope() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // The prefill workspace of a stream grown to `need` bytes, if the device has the memory.  Nothing
 // fails where it has not: such a call counts in neither `refused` nor the last error.
 bool grow_prefill(qvkv_dev *dev, StreamState *st, uint64_t need) {
@@ -223,6 +231,8 @@ bool grow_prefill(qvkv_dev *dev, StreamState *st, uint64_t need) {
         (void)hipStreamSynchronize(st->stream);  // its launches still read the old buffer
         dev_free(dev, p, n);
     };
+    if (st->pws.bytes >= need) return true;
+    UncapturedScope scope;
     return qvkv::grow(st->pws, need, qvkv::PREFILL_IMAGE_BYTES, dev->frees.load(), alloc, retire);
 }
 

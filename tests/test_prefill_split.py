@@ -190,3 +190,49 @@ def test_captured_prefill_shares_no_workspace(hip, knobs, dtype):
         assert torch.equal(outs[0], plain[0]) and torch.equal(outs[1], plain[1])
         assert torch.equal(outs[2], split)
     hip.check(s)
+
+
+@pytest.mark.gpu
+def test_workspace_grows_while_another_stream_is_captured(hip, knobs):
+    """Split launches that allocate and replace their stream's workspace leave a capture that is
+    under way on another stream whole."""
+    from test_gpu_kernels import cf32, cu32, fill_items, layout, new_pool
+
+    knobs("prefill_chunks", 4)
+    r, H, G, D = rng(7), 16, 4, 128
+    L = layout(F16, G, D)
+    N = 40 * 38 + 3
+    pool = new_pool(L, N, fill=2)
+    blocks, table_at, _ = fill_items(hip, L, pool, N, [600] * 40, r)
+    q, b, ta = cf32(normal(r, (40 * 64, H, D))), cu32(blocks), cu32(table_at)
+    args = {n: [cu32(x) for x in (np.full(n, 536), np.arange(n) * 64, np.full(n, 64))] for n in (2, 40)}
+    outs = [torch.zeros(40 * 64 * H * D, device="cuda") for _ in range(3)]
+
+    def attend(n, out):
+        p0, qa, nt = args[n]
+        hip.prefill_attention(L, pool, N, q, b, ta, p0, qa, nt, H, 599, 64, out)
+
+    a, s = torch.cuda.Stream(), torch.cuda.Stream()
+    for t in (a, s):  # the streams' state, without a workspace
+        with torch.cuda.stream(t):
+            hip.append(L, pool, N, q[:0], q[:0], b[:0])
+        hip.check(t)
+    torch.cuda.synchronize()
+    used = hip.usage()["used"]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=a):
+        attend(2, outs[0])
+        with torch.cuda.stream(s):
+            attend(2, outs[1])
+            attend(40, outs[2])
+        attend(2, outs[0])
+    assert hip.usage()["used"] > used
+    for _ in range(3):
+        outs[0].zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        n = 2 * 64 * H * D
+        for o in outs[:2]:
+            assert attn_errors(o[:n].cpu().numpy(), outs[2][:n].cpu().numpy())[1] <= REL_L2
+    hip.check(s)
+    hip.check(a)
