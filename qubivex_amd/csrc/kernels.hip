@@ -1377,8 +1377,7 @@ __device__ __forceinline__ void attn_wave(const uint8_t *__restrict__ pool, uint
 // a unit cut by the workgroup's own range leaves a partial in the workgroup's slot 0 (its
 // first unit) or 1 (its last), merged by k_attn_stream_merge.  The bookkeeping is restated
 // in tests/test_attention_split.py.
-// A launch streams at 6.5-6.7 TB/s (f16, d = 128) after about 15 us of launch, prefix
-// sums, first tiles and merge: 64 units of 2176 / 8704 positions 26 / 59 us.
+// (f16 at d = 128: the workgroups share units, k_attn_stream_wg.)
 // Each workgroup computes the units' prefix sums itself from pos (n_items <= 2048).
 // Workspace: partials [P][2][8][D], their (max, sum) [P][2][8][2], the prefix sums
 // [n_items + 1] (u64), then at the next 16-byte boundary one record per unit for the
@@ -1469,6 +1468,34 @@ __device__ __forceinline__ uint64_t uni(uint64_t v) {
            __builtin_amdgcn_readfirstlane((uint32_t)v);
 }
 
+// The prefix sums and the units' records, for the merge (by one workgroup).
+__device__ __forceinline__ void stream_records(const uint64_t *cum, uint32_t n_items, uint32_t upi,
+                                               uint32_t P, uint32_t D, uint32_t ucost, float *ws) {
+    const uint64_t T = cum[n_items];
+    float *ml = ws + (uint64_t)P * 2 * 8 * D;
+    uint64_t *wc = (uint64_t *)(ml + (uint64_t)P * 2 * 8 * 2);
+    for (uint32_t i = threadIdx.x; i <= n_items; i += 256) wc[i] = cum[i];
+    StreamRec *rec = (StreamRec *)((uint8_t *)ws + stream_rec_at(P, D, n_items));
+    for (uint32_t u = threadIdx.x; u < n_items * upi; u += 256) {
+        const uint32_t item = u / upi, ul = u % upi;
+        const uint64_t per_unit = (cum[item + 1] - cum[item]) / upi;
+        StreamRec r{0u, 0u, 0u, 0u};
+        if (per_unit != 0) {
+            // the unit's slots [a0, b): ucost set-up slots, then its tiles [a, b)
+            const uint64_t a0 = cum[item] + (uint64_t)ul * per_unit, a = a0 + ucost;
+            const uint64_t b = a0 + per_unit;
+            // workgroup holding position x: the largest v with floor(v T / P) <= x
+            auto owner = [&](uint64_t x) { return (uint32_t)(((x + 1) * P + T - 1) / T - 1); };
+            r.w0 = owner(a);
+            r.w1 = owner(b - 1);
+            // slot 1 when w0 took tiles of an earlier unit: its range starts before a0
+            // (the slot before a0 is the previous unit's last tile)
+            r.s0 = (uint64_t)r.w0 * T / P < a0 ? 1u : 0u;
+        }
+        rec[u] = r;
+    }
+}
+
 template <int D, bool Q8, bool NT, bool PK, bool NR, bool PIPE = false>
 __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
     constexpr uint32_t NO_UNIT = 0xffffffffu;
@@ -1485,29 +1512,8 @@ __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
     const uint64_t T = uni(cum[n_items]);
     const uint32_t P = gridDim.x, w = blockIdx.x;
     float *ml = ws + (uint64_t)P * 2 * 8 * D;
-    if (w == 0) {  // the prefix sums and the units' records, for the merge
-        uint64_t *wc = (uint64_t *)(ml + (uint64_t)P * 2 * 8 * 2);
-        for (uint32_t i = threadIdx.x; i <= n_items; i += 256) wc[i] = cum[i];
-        StreamRec *rec = (StreamRec *)((uint8_t *)ws + stream_rec_at(P, D, n_items));
-        for (uint32_t u = threadIdx.x; u < n_items * upi; u += 256) {
-            const uint32_t item = u / upi, ul = u % upi;
-            const uint64_t per_unit = (cum[item + 1] - cum[item]) / upi;
-            StreamRec r{0u, 0u, 0u, 0u};
-            if (per_unit != 0) {
-                // the unit's slots [a0, b): ucost set-up slots, then its tiles [a, b)
-                const uint64_t a0 = cum[item] + (uint64_t)ul * per_unit, a = a0 + ucost;
-                const uint64_t b = a0 + per_unit;
-                // workgroup holding position x: the largest v with floor(v T / P) <= x
-                auto owner = [&](uint64_t x) { return (uint32_t)(((x + 1) * P + T - 1) / T - 1); };
-                r.w0 = owner(a);
-                r.w1 = owner(b - 1);
-                // slot 1 when w0 took tiles of an earlier unit: its range starts before a0
-                // (the slot before a0 is the previous unit's last tile)
-                r.s0 = (uint64_t)r.w0 * T / P < a0 ? 1u : 0u;
-            }
-            rec[u] = r;
-        }
-    }
+    if (w == 0) stream_records(cum, n_items, upi, P, D, ucost, ws);
+
     // ---- the wave's share, unit by unit
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint64_t v4 = 4ull * w + wv;
@@ -1618,6 +1624,53 @@ void k_attn_stream_nr(QV_STREAM_PARAMS) {
                                                   table_at, pos, n_items, H, max_pos, out, ws,
                                                   hc_n, ucost, geo, err, nr);
 }
+// f16 at d = 128: the same split among P workgroups whose 4 waves share each unit's tiles.  A
+// workgroup works through its range with attn_unit; the partials, their slots and the merge are
+// those above.  Measured against waves on their own, in us (fused with the append), 768 workgroups
+// and 512 for at most 8 units: one sequence of 2 k, 8 KV heads 16.7 -> 14.1, of 32 k, 4 KV heads
+// 28.8 -> 25.8, 8 of 256-4096 26.6 -> 25.3, 16 of 1024-4096 40.6 -> 40.3, 32 of 2048 55.1 -> 51.3, of
+// 256-4096 59.7 -> 58.1, 100 of 512-4096 with 4 KV heads 97.9 -> 94.7.
+template <bool NR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NR ? 3 : 1)))
+void k_attn_stream_wg(QV_STREAM_PARAMS) {
+    constexpr int D = 128;
+    extern __shared__ __attribute__((aligned(16))) uint64_t cum[];  // [n_items + 1]
+    const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
+    const uint32_t GS = H / G;
+    const uint32_t upi = G * hc_n;  // units per item
+    stream_prefix(cum, pos, table_at, n_table, n_items, max_pos, upi, B, ucost, err);
+    const uint64_t T = uni(cum[n_items]);
+    const uint32_t P = gridDim.x, w = blockIdx.x;
+    const uint64_t s0 = (uint64_t)w * T / P, s1 = (uint64_t)(w + 1) * T / P;
+    float *ml = ws + (uint64_t)P * 2 * 8 * D;
+    if (w == 0) stream_records(cum, n_items, upi, P, D, ucost, ws);
+    bool first = true;
+    for (uint64_t x = s0; x < s1;) {
+        const uint32_t item = uni(stream_item(cum, n_items, x));
+        const uint64_t c0 = uni(cum[item]);
+        const uint64_t per_unit = (uni(cum[item + 1]) - c0) / upi;  // slots of a unit
+        const uint32_t ul = (uint32_t)((x - c0) / per_unit);        // unit within the item
+        const uint32_t g = ul / hc_n, hc = ul % hc_n;
+        const uint64_t tiles_at = c0 + (uint64_t)ul * per_unit + ucost;  // its first tile
+        const uint64_t unit_end = c0 + (uint64_t)(ul + 1) * per_unit;
+        const uint64_t seg_end = unit_end < s1 ? unit_end : s1;
+        if (seg_end > tiles_at) {  // (else only set-up slots of this unit)
+            const uint32_t t0 = x > tiles_at ? (uint32_t)(x - tiles_at) : 0u;
+            const uint32_t t1 = (uint32_t)(seg_end - tiles_at);
+            const uint32_t n = uni(pos[item]) + 1, tab = uni(table_at[item]);
+            const bool whole = t0 == 0 && seg_end == unit_end;
+            const uint64_t oh0 = (uint64_t)item * H + (uint64_t)g * GS + hc * 8;
+            const uint64_t slot = 2ull * w + (first ? 0u : 1u);
+            attn_unit<D, false, true, false, NR>(pool, pool_blocks, q, blocks, H, geo, err, item, g,
+                                                 hc, n, tab, t0, t1,
+                                                 whole ? out + oh0 * D : ws + slot * 8 * D, D,
+                                                 whole ? nullptr : ml + slot * 8 * 2, 2, nr);
+            first = false;
+        }
+        x = seg_end;
+    }
+}
+
 // q8_0, plain and with the new rows: 3 waves/SIMD at d = 128 (the workgroups that a CU takes),
 // where two tiles' registers no longer fit (32 x 4096 in us, pipelined / not: plain 66 / 65, fused
 // 81 / 67); pipelined at d = 64.
@@ -2066,16 +2119,21 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     const bool q8 = g.dtype == QVKV_Q8_0;
     // Few short units: a wide workgroup each, in one launch.  A CU draws about 37 GB/s from
     // HBM however many waves it has, so longer contexts are spread over the chip below, at
-    // the price of a merge launch.  Measured in us per call in a graph, wide / split, f16
-    // d = 128: 8 units of 512 positions 13.2 / 15.3, of 1024 20.4 / 15.9; 256 units of
-    // 256-1024 23.3 / 28.3, of 512-2048 40.2 / 41.5; d = 64: 8 units of 1024 11.3 / 12.4, of 2048
-    // 20.6 / 12.5; q8_0 d = 128: 8 units of 1024 17.2 / 17.3, 256 units of 512-2048 28.4 / 34.5.
+    // the price of a merge launch.  With more units the split has more cut units to merge, and
+    // the line moves out.  Measured in us per call, 8 KV heads, contexts of half to all of n, wide /
+    // split: f16 d = 128, 8 units of n = 640 12.2 / 12.4, of 960 15.6 / 12.8; 128 of 640 16.0 / 18.1, of
+    // 960 21.6 / 20.2; 192 of 960 22.1 / 25.2, of 1280 26.8 / 29.4; 256 of 1280 28.4 / 34.1.  f16 d = 64,
+    // 8 units of 960 12.0 / 12.6, of 1280 14.6 / 12.8; 64 of 1280 15.9 / 15.7; 128 of 1408 16.7 / 18.3, of
+    // 2048 22.6 / 20.4; 256 of 2048 25.5 / 28.7.  q8_0 d = 128, 8 units of 960 18.5 / 17.5; 64 of 1280
+    // 20.3 / 21.4, of 1408 22.5 / 21.2; 128 of 2048 27.2 / 27.4, 256 29.7 / 36.4; d = 64, 8 units of 1408
+    // 14.1 / 14.7, of 2048 17.4 / 15.0; 128 of 2816 20.3 / 33.9.
     const uint64_t base = q8 ? (g.D == 64 ? 88 : 64) : (g.D == 64 ? 64 : 40);
     // (a caller that sets the split's own knobs gets the split)
     const bool split_set = full != (uint64_t)kKnobDefault[KNOB_ATTN_FULL] ||
                            tune(KNOB_ATTN_STREAM) != 1 || tune(KNOB_ATTN_STREAM_WG) > 0;
     const int wide = tune(KNOB_ATTN_WIDE);
-    const uint64_t wide_tiles = wide >= 0 ? (uint64_t)wide : split_set ? 0 : units >= 128 ? 2 * base : base;
+    const uint64_t many = !q8 && g.D == 128 ? 192 : 128;
+    const uint64_t wide_tiles = wide >= 0 ? (uint64_t)wide : split_set ? 0 : units >= many ? 2 * base : base;
     if (units < full && units <= 256 && g.D != 256 && max_tiles <= wide_tiles) {
         p->kind = 3;
         return QVKV_OK;
@@ -2088,12 +2146,13 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
         return QVKV_OK;
     }
     // Other launches too small to fill the chip with one workgroup per unit (below 2 per CU)
-    // are split.  By work (k_attn_stream, the default): every wave gets an equal share
-    // of the (unit, tile) pairs, whatever the contexts.  One workgroup per CU (256) while a wave
-    // has few tiles (fewer partials to merge: one sequence of 32 k, 4 KV heads, 28.7 us against
-    // 30.3 with 512 and 32.9 with 768), two from 16384 tiles of 8 KiB (a ragged cfg2-like layer
-    // 55.6 us, 57.3 with 256, 55.9 with 768) or 4096 smaller ones (d = 64, 64 units of 2048
-    // 18.2 against 20.3), and three for large q8_0 launches, whose tiles cost more arithmetic
+    // are split.  By work (the default): every wave (k_attn_stream) or, f16 at d = 128, every
+    // workgroup (k_attn_stream_wg) gets an equal share of the (unit, tile) pairs, whatever the
+    // contexts.  f16 at d = 128: three workgroups per CU (24 of 4096, 8 KV heads 71.5 us, 76.0 with 512,
+    // 98.8 with 256; 4 of 2000-3000 18.4, 19.7, 20.2), two while each of few units would leave more
+    // than 64 partials to merge (one sequence of 32 k, 4 KV heads 25.8 us, 27.4 with 768).  d = 64 and
+    // q8_0: one per CU while a wave has few tiles, two from 4096 tiles (d = 64, 64 units of 2048
+    // 18.2 us, 20.3 with 256), and three for large q8_0 launches, whose tiles cost more arithmetic
     // (256 units of 1024-4096 52.1 us, 53.2 with 512, 72.9 with 256).  d = 256 runs one workgroup
     // per CU (its registers): 128 units of 1024-4096 82 us with 256, 94 with 512, 112 with 768;
     // q8_0 73, 91, 108.  Launches of 512 units
@@ -2101,10 +2160,10 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     // 5.7 and 3.3-4.3 split by work.
     if (tune(KNOB_ATTN_STREAM) != 0 && units < full && n_items <= STREAM_MAX_ITEMS) {
         const uint64_t work = units * max_tiles;  // bound: the actual work is known on the device
-        const bool big = !q8 && g.D >= 128;       // tiles of 8 KiB and more
-        uint64_t wgs = g.D == 256      ? 256
-                       : work >= 16384 ? (q8 ? 768 : 512)
-                                       : (work >= 4096 && !big ? 512 : 256);
+        uint64_t wgs = g.D == 256          ? 256
+                       : !q8 && g.D == 128 ? (units <= 8 ? 512 : 768)
+                       : work >= 16384     ? (q8 ? 768 : 512)
+                                           : (work >= 4096 ? 512 : 256);
         if (tune(KNOB_ATTN_STREAM_WG) > 0) wgs = (uint64_t)tune(KNOB_ATTN_STREAM_WG);
         if (wgs > (work + 3) / 4) wgs = (work + 3) / 4;  // at least a tile per wave
         if (wgs < 1) wgs = 1;
@@ -2222,8 +2281,10 @@ hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *po
     do { if (q8) { if (pk) QV_AS_Q8(DD, true, PIPE); else QV_AS_Q8(DD, false, PIPE); }           \
          else if (nr.k) QV_AS(k_attn_stream_nr<DD>); else QV_AS(k_attn_stream<DD>); } while (0)
         if (g.D == 64) QV_AS_D(64, true);
-        else if (g.D == 128) QV_AS_D(128, false);
-        else QV_AS_D(256, false);
+        else if (g.D == 256) QV_AS_D(256, false);
+        else if (!q8) { if (nr.k) QV_AS(k_attn_stream_wg<true>); else QV_AS(k_attn_stream_wg<false>); }
+        else if (pk) QV_AS_Q8(128, true, false);
+        else QV_AS_Q8(128, false, false);
 #undef QV_AS_D
 #undef QV_AS_Q8
 #undef QV_AS
