@@ -84,6 +84,20 @@ def test_split_prefill_matches_the_oracle(hip, knobs, dtype, H, G, D, B, chunks)
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("knob", [{"prefill_dma": 0}, {"prefill_dma": 0, "prefill_exact_p": 1},
+                                  {"prefill_exact_p": 1}, {"prefill_v2": 0}], ids=str)
+@pytest.mark.parametrize("chunks", [1, 3])
+@pytest.mark.parametrize("H,G,D,B", [(32, 8, 128, 16), (8, 2, 64, 48)])
+def test_other_f16_builds_match_the_oracle(hip, knobs, H, G, D, B, chunks, knob):
+    """The register-staged builds, those that carry P exactly, and the form without a split (which
+    takes no chunks), on the same segments."""
+    print(f"{knob}", flush=True)
+    for k, v in knob.items():
+        knobs(k, v)
+    test_split_prefill_matches_the_oracle(hip, knobs, F16, H, G, D, B, chunks)
+
+
+@pytest.mark.gpu
 def test_captured_split_prefill_survives_a_larger_launch(hip, knobs):
     """A launch captured on a stream with a workspace, and on one without, allocates nothing and
     replays right after a later launch that outgrew the workspace."""
