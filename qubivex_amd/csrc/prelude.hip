@@ -178,10 +178,9 @@ __device__ __forceinline__ float rms_scale_of(float ss, float n, float eps) {
 
 __global__ __launch_bounds__(64) void k_prelude(float *__restrict__ q, float *__restrict__ k,
                                                 float *__restrict__ v, uint32_t heads,
-                                                uint32_t kvh, uint32_t d, uint32_t parts,
-                                                PreludeArgs a) {
+                                                uint32_t kvh, uint32_t d, PreludeArgs a) {
     extern __shared__ float xs[];
-    const uint32_t t = blockIdx.x / parts, part = blockIdx.x % parts, lane = threadIdx.x;
+    const uint32_t t = blockIdx.x, part = blockIdx.y, lane = threadIdx.x;
     const uint32_t n = part == 0 ? heads * d : kvh * d;
     float *x = (part == 0 ? q : part == 1 ? k : v) + (uint64_t)t * n;
     const float *bias = part == 0 ? a.q_bias : part == 1 ? a.k_bias : a.v_bias;
@@ -567,8 +566,12 @@ hipError_t launch_prelude(float *q, float *k, float *v, uint32_t s, uint32_t hea
         return hipGetLastError();
     }
     const uint64_t lds = (uint64_t)(heads > kvh ? heads : kvh) * d * 4;
-    hipLaunchKernelGGL(k_prelude, dim3(s * parts), dim3(64), (uint32_t)lds, st, q, k, v, heads, kvh,
-                       d, parts, a);
+    // The rows of a part are consecutive workgroups, so that the q rows, the longest, go to all 8
+    // XCDs: alternating with the k rows they took every second one.  2000 tokens of 128 query and 8
+    // KV heads of 128, full norm, 657 us against 1274 (683 with the v rows between them); 4000 of
+    // 32 and 8 of 96, per-head norms, 83 against 130 (109).
+    hipLaunchKernelGGL(k_prelude, dim3(s, parts), dim3(64), (uint32_t)lds, st, q, k, v, heads, kvh,
+                       d, a);
     return hipGetLastError();
 }
 
