@@ -109,7 +109,7 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     X(PREFILL_EXACT_P, "prefill_exact_p", 0)                                                    \
     X(PREFILL_DMA, "prefill_dma", 1)                                                            \
     X(PREFILL_CHUNKS, "prefill_chunks", 0)      /* chunks per row block; 0: by the plan */     \
-    X(PREFILL_IMAGES, "prefill_images", 12)     /* q8_0: row blocks that share images; 0: off */ \
+    X(PREFILL_IMAGES, "prefill_images", 12)     /* q8_0: row blocks that share images; 0: off, 1: always */ \
     X(PREFILL_Q8_FAST, "prefill_q8_fast", 1)                                                    \
     X(PRELUDE_FAST, "prelude_fast", 1)                                                          \
     X(PRELUDE_WIDE, "prelude_wide", 1)                                                          \

@@ -1038,7 +1038,8 @@ void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS, const uint8_t *__restrict__ img, uint
     const uint32_t t_first = tr.first, ntiles = tr.end;  // tiles t_first .. ntiles - 1
     if (t_first >= ntiles) return;
 
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t w = [&]() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }();
     const uint32_t col = lane & 15u, grp = lane >> 4;
     const uint32_t rw0 = r0 + w * 16u;
     const bool wave_live = rw0 < nrows;
@@ -1236,17 +1237,16 @@ void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS, const uint8_t *__restrict__ img, uint
         }
     } else {
         const uint8_t *const head_img = img + (uint64_t)sg * img_tiles * sizeof(Q8PrefillSlot<D>);
-        const uint32_t ws_ = [&]() { return __builtin_amdgcn_readfirstlane(w); }();
         auto issue = [&](uint32_t t, Q8PrefillSlot<D> &sl) {
             const uint8_t *from = head_img + (uint64_t)t * sizeof(Q8PrefillSlot<D>);
             uint8_t *to = (uint8_t *)&sl;
 #pragma unroll
             for (uint32_t x = 0; x < 6; x++) {  // K, V high, V residual: 6 x 4 KiB
                 const uint8_t *src = from + (x * 4096u + threadIdx.x * 16u);
-                uint8_t *lds_dst = to + (x * 4096u + ws_ * 1024u);
+                uint8_t *lds_dst = to + (x * 4096u + w * 1024u);
                 __builtin_amdgcn_global_load_lds(src, lds_dst, 16, 0, 0);
             }
-            if (ws_ == 0 && lane < 16u) {       // the key scales: 256 bytes
+            if (w == 0 && lane < 16u) {       // the key scales: 256 bytes
                 const uint8_t *src = from + (24576u + lane * 16u);
                 uint8_t *lds_dst = to + 24576u;
                 __builtin_amdgcn_global_load_lds(src, lds_dst, 16, 0, 0);

@@ -42,7 +42,9 @@ struct PrefillShape {
 // q8_0: tile images where enough row blocks share them (knob prefill_images: the least
 // number), for as many segments at once as 512 MiB hold.  Measured at 2 k positions, 16
 // segments, without / with images: 4 row blocks 143 / 150 us, 8 247 / 234, 16 427 / 388, 64 1839 /
-// 1533; 4 segments at 8 k: 8 blocks 213 / 217, 32 794 / 685.  A limit below that makes passes of
+// 1533; 4 segments at 8 k: 8 blocks 213 / 217, 32 794 / 685.  Contexts of fewer than 8 tiles do
+// not pay for the extra launch: prompts of 180 tokens (12 row blocks, 6 tiles), 4 of them 18.4 / 19.6
+// us, 16 37.8 / 41.5; of 256 tokens (8 tiles) 24.0 / 24.5, 55.4 / 54.7.  A limit below that makes passes of
 // fewer segments only while each still fills the CUs: an underfilled pass costs more than the
 // conversions that it shares.
 inline PrefillPlan plan_prefill_shape(const PrefillShape &s, uint64_t limit) {
@@ -52,7 +54,8 @@ inline PrefillPlan plan_prefill_shape(const PrefillShape &s, uint64_t limit) {
     const uint64_t tiles = ((uint64_t)s.max_pos + 32) / 32;
     const uint64_t seg_img = (uint64_t)s.G * tiles * PREFILL_IMAGE_TILE;
     uint64_t n_seg = s.n_seg;
-    if (s.q8 && s.images > 0 && n_qb >= (uint64_t)s.images && seg_img <= PREFILL_IMAGE_BYTES) {
+    if (s.q8 && s.images > 0 && n_qb >= (uint64_t)s.images && (tiles >= 8 || s.images == 1) &&
+        seg_img <= PREFILL_IMAGE_BYTES) {
         auto bytes = [&](uint64_t segs) { return (segs * seg_img + 255) / 256 * 256; };
         const uint64_t most = std::min<uint64_t>(PREFILL_IMAGE_BYTES / seg_img, s.n_seg);
         uint64_t fit = most;

@@ -100,6 +100,11 @@ int main() {
     CHECK(plan_prefill_shape(b, ~0ull).img_segs == 16);
     CHECK(plan_prefill_shape(b, 100ull << 20).img_segs == 8);
     CHECK(plan_prefill_shape(b, 30ull << 20).img_segs == 0);
+    // short contexts take none, unless always asked for
+    PrefillShape c{true, 8, 128, 4, 16, 179, 180, 12, 0};
+    CHECK(plan_prefill_shape(c, ~0ull).img_segs == 0);
+    c.images = 1;
+    CHECK(plan_prefill_shape(c, ~0ull).img_segs == 16);
     // one chunk at 8 k: without room for images the split is kept
     const PrefillShape one{true, 4, 128, 8, 1, 8703, 512, 12, 0};
     const PrefillPlan p = plan_prefill_shape(one, 20ull << 20);
