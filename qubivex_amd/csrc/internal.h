@@ -74,6 +74,7 @@ struct AttnPlan {
     uint32_t tpc;       // 16-position tiles per chunk
     uint64_t ws_bytes;  // workspace for partial results (0 when n_chunks == 1)
     uint32_t ucost;     // kind 2: a unit's set-up cost in tiles (its share of the split)
+    bool by_wg;         // kind 2: shares by workgroup (attn_stream_wg), else by wave
 };
 int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t max_pos,
                    AttnPlan *p, const char **why);
@@ -100,7 +101,7 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     X(ATTN_TARGET, "attn_target", 1536)         /* context-chunk split: workgroups aimed at */  \
     X(FUSED_Q8, "fused_q8", 1)                  /* fused append + attention for q8_0 */         \
     X(ATTN_WAVES4_F16, "attn_waves4_f16", 0)                                                    \
-    X(ATTN_WAVES3_Q8, "attn_waves3_q8", 0)      /* q8_0 d = 128: 0 pipelined, 1 one tile */     \
+    X(ATTN_WAVES3_Q8, "attn_waves3_q8", 0)      /* q8_0 d = 128: 0 rule, 1 one tile, 2 piped */     \
     X(ATTN_PACK, "attn_pack", 1)                                                                \
     X(ATTN_IDS_BELOW, "attn_ids_below", 2048)                                                   \
     X(ATTN_XCD, "attn_xcd", 1)                                                                  \

@@ -966,10 +966,8 @@ void k_attn_mfma_ids(QV_ATTN_PARAMS) {
 }
 // q8_0, plain and with the new rows (NR).  PIPE (d = 64, 128): the next tile's loads in flight
 // during this tile's arithmetic, at 3 waves/SIMD at d = 128; else one tile at a time at 4.
-// Measured in us, one tile at a time / pipelined: a layer of 64 x 2048, 8 KV heads, fused 65.0 /
-// 56.1, plain 61.9 / 54.8; 256 x 2048 212 / 199; 128 x 8192, 4 KV heads 217 / 193; d = 64,
-// 64 x 2048 48.7 / 37.7.  (A tile costs a wave about 1.5 us at 2 waves/SIMD, a third of it
-// arithmetic.)
+// (A tile costs a wave about 1.5 us at 2 waves/SIMD, a third of it arithmetic.)  d = 64, 64 x
+// 2048, 8 KV heads 48.7 / 37.7 us; the line at d = 128 stands in q8_pipelined.
 template <int D, bool PK, bool NR, bool PIPE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D != 128 ? 1 : PIPE ? 3 : 4)))
 void k_attn_mfma_q8(QV_ATTN_PARAMS) {
@@ -1265,7 +1263,7 @@ __device__ __forceinline__ void attn_unit(const uint8_t *__restrict__ pool, uint
 // Tiles t0 .. t1-1 of one unit by one wave (attn_unit's tile loop over consecutive tiles), left
 // in LDS as the wave's unnormalised rows o[8][D] with their max m[8] (log2 domain) and sum l[8].
 // nrow: the wave's own 2 D floats for the new rows (q8_0 NR).
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool PIPE>
+template <int D, bool Q8, bool NT, bool PK, bool NR>
 __device__ __forceinline__ void attn_wave(const uint8_t *__restrict__ pool, uint64_t pool_blocks,
                                           const float *__restrict__ q,
                                           const uint32_t *__restrict__ blocks, uint32_t H,
@@ -1313,7 +1311,7 @@ __device__ __forceinline__ void attn_wave(const uint8_t *__restrict__ pool, uint
 #pragma unroll
     for (int j = 0; j < NJ; j++) st.acc[j] = f4{0.f, 0.f, 0.f, 0.f};
     if constexpr (Q8) {
-        q8_tiles<D, PK, NR, PIPE>(pool, pool_blocks, blocks, geo, err, g, hc, n, tab, t0, t1, 1u, nrow, qf,
+        q8_tiles<D, PK, NR, false>(pool, pool_blocks, blocks, geo, err, g, hc, n, tab, t0, t1, 1u, nrow, qf,
                                       st, c, qg, hi_col, sigma);
     } else {
         uint32_t tt = t0;
@@ -1377,7 +1375,7 @@ __device__ __forceinline__ void attn_wave(const uint8_t *__restrict__ pool, uint
 // a unit cut by the workgroup's own range leaves a partial in the workgroup's slot 0 (its
 // first unit) or 1 (its last), merged by k_attn_stream_merge.  The bookkeeping is restated
 // in tests/test_attention_split.py.
-// (f16 at d = 128: the workgroups share units, k_attn_stream_wg.)
+// (f16 at d = 64, and large launches at d = 256; the rest run attn_stream_wg below.)
 // Each workgroup computes the units' prefix sums itself from pos (n_items <= 2048).
 // Workspace: partials [P][2][8][D], their (max, sum) [P][2][8][2], the prefix sums
 // [n_items + 1] (u64), then at the next 16-byte boundary one record per unit for the
@@ -1496,7 +1494,7 @@ __device__ __forceinline__ void stream_records(const uint64_t *cum, uint32_t n_i
     }
 }
 
-template <int D, bool Q8, bool NT, bool PK, bool NR, bool PIPE = false>
+template <int D, bool Q8, bool NT, bool PK, bool NR>
 __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
     constexpr uint32_t NO_UNIT = 0xffffffffu;
     extern __shared__ __attribute__((aligned(16))) uint64_t cum[];  // [n_items + 1]
@@ -1542,7 +1540,7 @@ __device__ __forceinline__ void attn_stream_body(QV_STREAM_PARAMS) {
         // is taken only by the wave's last unit)
         const bool whole = starts && ends;
         const uint32_t slot = 2 * wv + (whole || n_units != 0 ? 1u : 0u);
-        attn_wave<D, Q8, NT, PK, NR, PIPE>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
+        attn_wave<D, Q8, NT, PK, NR>(pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab,
                                      t0, t1, nr, &so[slot][0][0], sm[slot], sl[slot], nrow[wv]);
         if (whole) {
             lds_order();
@@ -1624,16 +1622,21 @@ void k_attn_stream_nr(QV_STREAM_PARAMS) {
                                                   table_at, pos, n_items, H, max_pos, out, ws,
                                                   hc_n, ucost, geo, err, nr);
 }
-// f16 at d = 128: the same split among P workgroups whose 4 waves share each unit's tiles.  A
-// workgroup works through its range with attn_unit; the partials, their slots and the merge are
-// those above.  Measured against waves on their own, in us (fused with the append), 768 workgroups
-// and 512 for at most 8 units: one sequence of 2 k, 8 KV heads 16.7 -> 14.1, of 32 k, 4 KV heads
-// 28.8 -> 25.8, 8 of 256-4096 26.6 -> 25.3, 16 of 1024-4096 40.6 -> 40.3, 32 of 2048 55.1 -> 51.3, of
-// 256-4096 59.7 -> 58.1, 100 of 512-4096 with 4 KV heads 97.9 -> 94.7.
-template <bool NR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NR ? 3 : 1)))
-void k_attn_stream_wg(QV_STREAM_PARAMS) {
-    constexpr int D = 128;
+// The same split among P workgroups whose 4 waves share each unit's tiles: a workgroup works
+// through its range with attn_unit; the partials, their slots and the merge are those above.  Which
+// form a launch takes is by measurement, in us per call (fused with the append, 8 KV heads, waves on
+// their own / workgroups), contexts of 1000-4000 unless said:
+//   f16 d = 128, 768 workgroups: 16 sequences 40.7 / 40.4, 32 of 256-4096 59.6 / 58.4, 32 of 2048 54.7 /
+//     51.5, one of 2048 17.1 / 14.4; 64 of 4096 with 4 KV heads 99.4 / 92.7;
+//   q8_0 d = 128, 768: 16 sequences 33.7 / 34.0, 32 48.7 / 49.4, 60 of 300-3000 59.0 / 62.2; 16 of 4000
+//     40.7 / 37.9, 48 of 2048 55.3 / 52.0, one of 2000 17.4 / 14.8;
+//   q8_0 d = 64, 768 (pipelined): 16 35.9 / 25.8, 32 of 4000 63.3 / 37.9, one of 2000 14.6 / 12.6;
+//   f16 d = 64: 8 19.5 / 20.5, 32 39.4 / 44.5, 32 of 2048 27.2 / 36.1: waves on their own;
+//   d = 256, 256 workgroups: waves on their own above 8192 (unit, tile) pairs (f16 16 sequences 79.3 /
+//     82.3, 63 of 1000-2000 157.6 / 178.3), else workgroups (4 of 258 22.3 / 17.7, 4 of 2000 31.3 / 28.1,
+//     one of 16000 40.9 / 39.9; q8_0 4 of 258 26.0 / 21.5).
+template <int D, bool Q8, bool PK, bool NR, bool PIPE>
+__device__ __forceinline__ void attn_stream_wg(QV_STREAM_PARAMS) {
     extern __shared__ __attribute__((aligned(16))) uint64_t cum[];  // [n_items + 1]
     const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
     const uint32_t GS = H / G;
@@ -1661,25 +1664,36 @@ void k_attn_stream_wg(QV_STREAM_PARAMS) {
             const bool whole = t0 == 0 && seg_end == unit_end;
             const uint64_t oh0 = (uint64_t)item * H + (uint64_t)g * GS + hc * 8;
             const uint64_t slot = 2ull * w + (first ? 0u : 1u);
-            attn_unit<D, false, true, false, NR>(pool, pool_blocks, q, blocks, H, geo, err, item, g,
-                                                 hc, n, tab, t0, t1,
-                                                 whole ? out + oh0 * D : ws + slot * 8 * D, D,
-                                                 whole ? nullptr : ml + slot * 8 * 2, 2, nr);
+            attn_unit<D, Q8, true, PK, NR, false, 4, PIPE>(
+                pool, pool_blocks, q, blocks, H, geo, err, item, g, hc, n, tab, t0, t1,
+                whole ? out + oh0 * D : ws + slot * 8 * D, D, whole ? nullptr : ml + slot * 8 * 2, 2,
+                nr);
             first = false;
         }
         x = seg_end;
     }
 }
 
-// q8_0, plain and with the new rows: 3 waves/SIMD at d = 128 (the workgroups that a CU takes),
-// where two tiles' registers no longer fit (32 x 4096 in us, pipelined / not: plain 66 / 65, fused
-// 81 / 67); pipelined at d = 64.
-template <int D, bool PK, bool NR, bool PIPE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 3 : 1)))
-void k_attn_stream_q8(QV_STREAM_PARAMS) {
-    attn_stream_body<D, true, true, PK, NR, PIPE>(pool, pool_blocks, q, blocks, n_table, table_at,
-                                                  pos, n_items, H, max_pos, out, ws, hc_n, ucost, geo,
-                                                  err, nr);
+#define QV_STREAM_ARGS                                                                          \
+    pool, pool_blocks, q, blocks, n_table, table_at, pos, n_items, H, max_pos, out, ws, hc_n, ucost, \
+        geo, err, nr
+template <int D, bool NR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NR && D == 128 ? 3 : 1)))
+void k_attn_stream_wg(QV_STREAM_PARAMS) {
+    attn_stream_wg<D, false, false, NR, false>(QV_STREAM_ARGS);
+}
+// (d = 128: 4 waves/SIMD, 3 with the new rows, whose registers would spill at 4; pipelined
+// at d = 64)
+template <int D, bool PK, bool NR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D != 128 ? 1 : NR ? 3 : 4)))
+void k_attn_stream_wg_q8(QV_STREAM_PARAMS) {
+    attn_stream_wg<D, true, PK, NR, D == 64>(QV_STREAM_ARGS);
+}
+
+// q8_0 at d = 256, waves on their own, plain and with the new rows.
+template <bool PK, bool NR>
+__global__ __launch_bounds__(256) void k_attn_stream_q8(QV_STREAM_PARAMS) {
+    attn_stream_body<256, true, true, PK, NR>(QV_STREAM_ARGS);
 }
 
 // Merge for k_attn_stream: block = one (item, query head), D threads per slice of the unit's
@@ -2109,6 +2123,7 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     p->tpc = 0;
     p->ws_bytes = 0;
     p->ucost = 0;
+    p->by_wg = false;
     if (!mfma) {
         if ((uint64_t)n_items * heads > 0x7fffffffull) { *why = "batch too large"; return QVKV_E_SHAPE; }
         return QVKV_OK;
@@ -2146,24 +2161,23 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
         return QVKV_OK;
     }
     // Other launches too small to fill the chip with one workgroup per unit (below 2 per CU)
-    // are split.  By work (the default): every wave (k_attn_stream) or, f16 at d = 128, every
-    // workgroup (k_attn_stream_wg) gets an equal share of the (unit, tile) pairs, whatever the
-    // contexts.  f16 at d = 128: three workgroups per CU (24 of 4096, 8 KV heads 71.5 us, 76.0 with 512,
-    // 98.8 with 256; 4 of 2000-3000 18.4, 19.7, 20.2), two while each of few units would leave more
-    // than 64 partials to merge (one sequence of 32 k, 4 KV heads 25.8 us, 27.4 with 768).  d = 64 and
-    // q8_0: one per CU while a wave has few tiles, two from 4096 tiles (d = 64, 64 units of 2048
-    // 18.2 us, 20.3 with 256), and three for large q8_0 launches, whose tiles cost more arithmetic
-    // (256 units of 1024-4096 52.1 us, 53.2 with 512, 72.9 with 256).  d = 256 runs one workgroup
-    // per CU (its registers): 128 units of 1024-4096 82 us with 256, 94 with 512, 112 with 768;
-    // q8_0 73, 91, 108.  Launches of 512 units
+    // are split.  By work (the default): every workgroup (attn_stream_wg) or, in the layouts that
+    // its comment names, every wave (k_attn_stream) gets an equal share of the (unit, tile) pairs,
+    // whatever the contexts.  Workgroups: three per CU (f16 d = 128, 24 of 4096, 8 KV heads 71.5 us, 76.0
+    // with 512, 98.8 with 256; 4 of 2000-3000 18.4, 19.7, 20.2; q8_0 32 of 4000 60.2, 62.5, 88.6; d = 64
+    // 37.9, 41.9, 54.2), two while each of few units would leave more than 64 partials to merge (f16
+    // d = 128, one sequence of 32 k, 4 KV heads 25.8 us, 27.4 with 768; q8_0 16 k, 8 heads 21.2, 23.4).
+    // f16 at d = 64: one per CU while a wave has few tiles, two from 4096 (64 units of 2048 18.2 us, 20.3
+    // with 256).  d = 256 runs one workgroup per CU (its registers): 128 units of 1024-4096 82 us with
+    // 256, 94 with 512, 112 with 768; q8_0 73, 91, 108.  Launches of 512 units
     // and more (a layer of 128 x 8k, or of cfg3) run best unsplit: 6.0 and 4.8 TB/s, against
     // 5.7 and 3.3-4.3 split by work.
     if (tune(KNOB_ATTN_STREAM) != 0 && units < full && n_items <= STREAM_MAX_ITEMS) {
         const uint64_t work = units * max_tiles;  // bound: the actual work is known on the device
-        uint64_t wgs = g.D == 256          ? 256
-                       : !q8 && g.D == 128 ? (units <= 8 ? 512 : 768)
-                       : work >= 16384     ? (q8 ? 768 : 512)
-                                           : (work >= 4096 ? 512 : 256);
+        p->by_wg = g.D == 128 || (g.D == 64 && q8) || (g.D == 256 && work <= 8192);
+        uint64_t wgs = g.D == 256 ? 256
+                       : p->by_wg ? (units <= 8 ? 512 : 768)
+                                  : (work >= 4096 ? 512 : 256);
         if (tune(KNOB_ATTN_STREAM_WG) > 0) wgs = (uint64_t)tune(KNOB_ATTN_STREAM_WG);
         if (wgs > (work + 3) / 4) wgs = (work + 3) / 4;  // at least a tile per wave
         if (wgs < 1) wgs = 1;
@@ -2245,6 +2259,21 @@ hipError_t launch_slots_at(const Geometry &g, const uint32_t *blocks, uint64_t n
     return hipGetLastError();
 }
 
+// Whether an unsplit q8_0 launch at d = 128 of `units` workgroups, each of at most `tiles` tiles,
+// runs pipelined (3 workgroups per CU) or one tile at a time (4).  Short contexts gain nothing from
+// the next tile's loads, and launches between 3 and 4 workgroups per CU run in one round only one
+// tile at a time.  Measured in us per layer (8 KV heads), one tile / pipelined: 512 units of 128-256
+// positions 15.1 / 15.7, of 256-512 20.7 / 19.6, of 2048 58.6 / 56.2, of 2048-4096 96.1 / 89.3; 640 of
+// 512-1024 38.1 / 38.9, of 2048-4096 121.6 / 120.2; 800 of 64-128 16.4 / 20.1, of 1024-2048 89.2 / 82.8;
+// 1024 of 64-128 17.8 / 21.7, of 512 34.2 / 40.1, of 2048 108.1 / 119.4; 1280 of 256-512 41.9 / 43.8, of
+// 2048 143.2 / 133.3; 2048 of 256-512 57.3 / 63.1, of 2048 203.0 / 204.3.
+static bool q8_pipelined(uint64_t units, uint64_t tiles) {
+    const int knob = tune(KNOB_ATTN_WAVES3_Q8);
+    if (knob != 0) return knob != 1;
+    if (units <= 576) return tiles >= 24;
+    return tiles >= 128 && (units <= 896 || units > 1152);
+}
+
 hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *pool,
                             uint64_t pool_blocks, const float *q, const uint32_t *blocks,
                             uint64_t n_table, const uint32_t *table_at, const uint32_t *pos,
@@ -2274,19 +2303,20 @@ hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *po
     hipLaunchKernelGGL(KERNEL, dim3(P), dim3(256), (n_items + 1) * 8, s, pp, pool_blocks, q,     \
                        blocks, n_table, table_at, pos, n_items, heads, max_pos, out, wsf, p.hc, \
                        p.ucost, geo, err, nr)
-#define QV_AS_Q8(DD, PK, PIPE)                                                                  \
-    do { if (nr.k) QV_AS((k_attn_stream_q8<DD, PK, true, PIPE>));                                \
-         else QV_AS((k_attn_stream_q8<DD, PK, false, PIPE>)); } while (0)
-#define QV_AS_D(DD, PIPE)                                                                       \
-    do { if (q8) { if (pk) QV_AS_Q8(DD, true, PIPE); else QV_AS_Q8(DD, false, PIPE); }           \
-         else if (nr.k) QV_AS(k_attn_stream_nr<DD>); else QV_AS(k_attn_stream<DD>); } while (0)
-        if (g.D == 64) QV_AS_D(64, true);
-        else if (g.D == 256) QV_AS_D(256, false);
-        else if (!q8) { if (nr.k) QV_AS(k_attn_stream_wg<true>); else QV_AS(k_attn_stream_wg<false>); }
-        else if (pk) QV_AS_Q8(128, true, false);
-        else QV_AS_Q8(128, false, false);
-#undef QV_AS_D
-#undef QV_AS_Q8
+#define QV_AS_NR(KERNEL, ...)                                                                   \
+    do { if (nr.k) QV_AS((KERNEL<__VA_ARGS__, true>)); else QV_AS((KERNEL<__VA_ARGS__, false>)); } while (0)
+#define QV_AS_WG(DD)                                                                            \
+    do { if (!q8) QV_AS_NR(k_attn_stream_wg, DD);                                                \
+         else if (pk) QV_AS_NR(k_attn_stream_wg_q8, DD, true);                                   \
+         else QV_AS_NR(k_attn_stream_wg_q8, DD, false); } while (0)
+        if (g.D == 128) QV_AS_WG(128);
+        else if (g.D == 256 && p.by_wg) QV_AS_WG(256);
+        else if (q8 && g.D == 64) { if (pk) QV_AS_NR(k_attn_stream_wg_q8, 64, true); else QV_AS_NR(k_attn_stream_wg_q8, 64, false); }
+        else if (q8) { if (pk) QV_AS_NR(k_attn_stream_q8, true); else QV_AS_NR(k_attn_stream_q8, false); }
+        else if (g.D == 64) { if (nr.k) QV_AS(k_attn_stream_nr<64>); else QV_AS(k_attn_stream<64>); }
+        else { if (nr.k) QV_AS(k_attn_stream_nr<256>); else QV_AS(k_attn_stream<256>); }
+#undef QV_AS_WG
+#undef QV_AS_NR
 #undef QV_AS
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -2324,7 +2354,7 @@ hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *po
     // K/V tiles are streamed with non-temporal loads (read once).
     // Occupancy: f16 runs at the compiler's register choice (3 waves/SIMD at d = 128; the 4-wave
     // build, knob attn_waves4_f16, 5.90 against 6.48 TB/s at cfg5), q8_0 at d = 128 pipelined at
-    // 3 (attn_waves3_q8 = 1: one tile at a time at 4).  Pipelining the f16 loop one tile ahead
+    // 3 or one tile at a time at 4 (q8_pipelined).  Pipelining the f16 loop one tile ahead
     // (2 waves/SIMD) and 5 waves/SIMD (spills) were slower.
 #define QV_ATTN(KERNEL)                                                                         \
     hipLaunchKernelGGL(KERNEL, dim3((unsigned)grid), dim3(256), 0, s, pp, pool_blocks, q, blocks, \
@@ -2338,7 +2368,7 @@ hipError_t launch_attention(const Geometry &g, const AttnPlan &p, const void *po
     if (q8) {
         if (g.D == 64) QV_ATTN_Q8(64, true);
         else if (g.D == 256) QV_ATTN_Q8(256, false);
-        else if (tune(KNOB_ATTN_WAVES3_Q8) == 0) QV_ATTN_Q8(128, true);
+        else if (q8_pipelined(grid, p.n_chunks == 1 ? ((uint64_t)max_pos + 16) / 16 : p.tpc)) QV_ATTN_Q8(128, true);
         else QV_ATTN_Q8(128, false);
     } else if (g.D == 64) {
         if (nr.k) QV_ATTN(k_attn_mfma_nr<64>); else QV_ATTN(k_attn_mfma<64>);

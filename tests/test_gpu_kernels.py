@@ -269,7 +269,7 @@ def test_attention_within_tolerance(hip, dtype, H, G, D, lens):
 SWITCH_CASES = [ATTN_CASES[i] for i in (0, 1, 8, 9)] + ATTN_CASES[-4:]
 
 
-@pytest.mark.parametrize("env", [{"attn_waves4_f16": "1"}, {"attn_waves3_q8": "1"},
+@pytest.mark.parametrize("env", [{"attn_waves4_f16": "1"}, {"attn_waves3_q8": "1"}, {"attn_waves3_q8": "2"},
                                  {"attn_pack": "0"},
                                  {"attn_xcd": "0"}, {"attn_ids_below": "0"},
                                  {"stream_unit_cost": "0"}, {"stream_unit_cost": "40"},
