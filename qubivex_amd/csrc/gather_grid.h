@@ -16,11 +16,13 @@ struct GatherGrid {
 // tile), as for the block copy: many short workgroups keep the stores, most of the traffic, spread
 // over time.  Against 256 threads x 8 pieces (a tile per workgroup), in us: q8_0 d = 128, 64 items
 // of 1024-2048, 202 -> 184 (1.02 GB), d = 64 166 -> 105, f16 -> f32 225 -> 217.
-// At most 2^18 of them, which walk the units (each_live_tile): a workgroup costs about 0.22 ns of
-// dispatch over the chip also where it finds nothing to do.  held: the units with something
-// in them, by the room for the output and by the tables.  An uneven batch, one with three times
-// as many in all, takes a workgroup per held unit and walks tile by tile, which spreads the long
-// items evenly; an even one keeps a tile's neighbours together.  In us, at 256 threads x 8 / one
+// They walk the units (each_live_tile) where there are more than the grid.  held: the units with
+// something in them, by the room for the output and by the tables.  An even batch takes a
+// workgroup per piece of every unit, as many as a launch holds (at most 2^18 that walk, in us, 512
+// of 2048, q8_0 d = 128 2054 -> 1934, d = 64 1245 -> 1080, f16 d = 128, 256 of 2048 1170 -> 1081).  An
+// uneven one, with three times as many units as are held, would pay about 0.22 ns of dispatch over
+// the chip for each that finds nothing to do: it takes a workgroup per held unit, at most 2^18,
+// and walks tile by tile, which spreads the long items evenly.  In us, at 256 threads x 8 / one
 // workgroup per piece of every unit / this, 8 KV heads, q8_0 d = 128, d = 64, f16 d = 128:
 //   one item of 32 k beside 63 of 1 k    188 / 935 / 197, 192 / 477 / 118, 276 / 944 / 239
 //   one of 32 k beside 255 of 64         251 / 3570 / 103, 364 / 1800 / 62, 680 / 3580 / 138
@@ -34,8 +36,8 @@ inline GatherGrid gather_grid(uint64_t n_items, uint64_t tiles, uint64_t per_til
     if (units * 256 > 0xffffffffull) return r;
     const uint64_t held = std::min(out_positions / 16, n_table * (block / 16)) + n_items;
     r.by_tile = units > 3 * held;
-    uint64_t at_once = (1ull << 18) / per_tile;
-    if (r.by_tile) at_once = std::min(at_once, held);
+    uint64_t at_once = ((1ull << 26) - 1) / per_tile;  // 2^32 threads in all
+    if (r.by_tile) at_once = std::min<uint64_t>((1ull << 18) / per_tile, held);
     at_once = std::max<uint64_t>(at_once, 1);
     // (a stride without a common factor with the inner count: the items of a tile, or the starts
     // of the items, then fall to different workgroups)

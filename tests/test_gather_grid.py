@@ -18,7 +18,8 @@ static int bad(const char *what, unsigned long long a, unsigned long long b) {
 // the walk of each_live_tile by the workgroups of one piece
 static int covers(uint64_t items, uint64_t tiles, uint64_t per_tile, uint64_t positions) {
     const qvkv::GatherGrid g = qvkv::gather_grid(items, tiles, per_tile, positions, 1ull << 40, 16);
-    if (g.wgs == 0 || g.wgs % per_tile || g.wgs > (1u << 18) + per_tile) return bad("wgs", g.wgs, per_tile);
+    const uint64_t most = g.by_tile ? (1u << 18) + per_tile : (1u << 26) - 1;
+    if (g.wgs == 0 || g.wgs % per_tile || g.wgs > most) return bad("wgs", g.wgs, per_tile);
     const uint64_t units = items * tiles, step = g.wgs / per_tile;
     if (g.by_tile && step > positions / 16 + items) return bad("more than held", step, positions);
     std::vector<uint8_t> seen(units, 0);
@@ -38,6 +39,8 @@ int main() {
                                   {7, 5, 3, 560}, {64, 128, 32, 131072}, {33, 4096, 2, 4096}, {4096, 1024, 128, 65536},
                                   {1000, 1000, 1, 16000000}, {3, 1, 300000, 48}, {100, 63, 512, 6400}};
     for (auto &s : shapes) rc |= covers(s[0], s[1], s[2], s[3]);
+    // an even batch: a workgroup per piece of every unit
+    if (qvkv::gather_grid(512, 128, 32, 512 * 2048, 512 * 128, 16).wgs != 512 * 128 * 32) rc |= bad("even", 0, 0);
     // an uneven batch: far fewer workgroups than pieces (a workgroup costs its dispatch)
     const qvkv::GatherGrid g = qvkv::gather_grid(64, 2048, 32, 32768 + 63 * 1024, 6080, 16);
     if (!g.by_tile || g.wgs > 6144 * 32) rc |= bad("uneven", g.wgs, g.by_tile);
