@@ -5,11 +5,18 @@
 #include <numeric>
 #include <stdint.h>
 
+#ifdef __HIPCC__
+#define QVKV_HOST_DEVICE __host__ __device__
+#else
+#define QVKV_HOST_DEVICE
+#endif
+
 namespace qvkv {
 
 struct GatherGrid {
     uint32_t wgs = 0;      // workgroups; 0: the launch is refused
     bool by_tile = false;  // units in order of tile, then item (else item, then tile)
+    bool by_xcd = false;   // the pieces of a unit on one XCD (workgroups go to the 8 in turn)
 };
 
 // One-wave workgroups, each one batch of a tile's pieces at a time (per_tile of them share a
@@ -28,9 +35,13 @@ struct GatherGrid {
 //   one of 32 k beside 255 of 64         251 / 3570 / 103, 364 / 1800 / 62, 680 / 3580 / 138
 //   one of 4096 beside 15 of 64          17.6 / 31.1 / 13.2, 20.4 / 16.0 / 9.3, 19.8 / 35.1 / 17.3
 //   32 of 256-4096                       155 / 150 / 147, 122 / 86 / 83, 179 / 173 / 177
+// Large even q8_0 batches (one_xcd) write a unit's output from one XCD: 512 items of 2048, d = 128
+// 2058 -> 1962, 128 of 2048 500 -> 493, d = 256 1268 -> 1080; 64 of 1024-2048 184 -> 189, so from 16384
+// units on, and not at d = 64 (1083 -> 1120).
 // A launch of more units than 2^32 threads hold at 256 each is refused.
 inline GatherGrid gather_grid(uint64_t n_items, uint64_t tiles, uint64_t per_tile,
-                              uint64_t out_positions, uint64_t n_table, uint64_t block) {
+                              uint64_t out_positions, uint64_t n_table, uint64_t block,
+                              bool one_xcd = false) {
     GatherGrid r;
     const uint64_t units = n_items * tiles;
     if (units * 256 > 0xffffffffull) return r;
@@ -43,8 +54,18 @@ inline GatherGrid gather_grid(uint64_t n_items, uint64_t tiles, uint64_t per_til
     // of the items, then fall to different workgroups)
     if (units > at_once)
         while (std::gcd(at_once, r.by_tile ? n_items : tiles) != 1) at_once--;
-    r.wgs = (uint32_t)(std::min(units, at_once) * per_tile);
+    r.by_xcd = one_xcd && !r.by_tile && units >= 16384 && units + 7 <= at_once;
+    r.wgs = (uint32_t)((r.by_xcd ? (units + 7) / 8 * 8 : std::min(units, at_once)) * per_tile);
     return r;
+}
+
+// The unit and piece of a workgroup (the first unit of its walk).
+struct GatherPlace {
+    uint32_t unit, part;
+};
+inline QVKV_HOST_DEVICE GatherPlace gather_place(uint32_t wg, uint32_t parts, bool by_xcd) {
+    const uint32_t i = by_xcd ? wg / 8u : wg, q = i / parts;
+    return GatherPlace{by_xcd ? q * 8u + wg % 8u : q, i - q * parts};
 }
 
 }  // namespace qvkv

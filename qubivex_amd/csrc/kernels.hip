@@ -778,11 +778,12 @@ __global__ __launch_bounds__(64) void k_gather_q8(const uint8_t *__restrict__ po
                                                    uint32_t n_items, uint32_t tiles_max,
                                                    uint64_t out_positions, float *out_k,
                                                    float *out_v, uint32_t parts, bool by_tile,
-                                                   Geo geo, int *err) {
+                                                   bool by_xcd, Geo geo, int *err) {
     // d = 128 keys: an LDS copy of the wave's 8 rows (row stride 132 floats)
     __shared__ __attribute__((aligned(16))) float kx[D == 128 ? 8 * 132 : 4];
-    const uint32_t part = blockIdx.x % parts;
-    each_live_tile(blockIdx.x / parts, gridDim.x / parts, n_items, tiles_max, by_tile, lens,
+    const GatherPlace at = gather_place(blockIdx.x, parts, by_xcd);
+    const uint32_t part = at.part;
+    each_live_tile(at.unit, gridDim.x / parts, n_items, tiles_max, by_tile, lens,
                    [&](uint32_t item, uint32_t tile, uint32_t len) {
         const uint32_t p0 = tile * 16u;
         const uint32_t B = (uint32_t)geo.B, G = (uint32_t)geo.G;
@@ -2029,16 +2030,16 @@ hipError_t launch_gather(const Geometry &g, const void *pool, uint64_t pool_bloc
                        pool_blocks, blocks, n_table, table_at, lens, out_at, n_items, tiles,   \
                        out_positions, out_k, out_v, parts, false, geo, err)
     if (out_dtype == QVKV_F32 && grid * 256 > 0xffffffffull) return hipErrorInvalidValue;
-    auto to_f32 = [&](uint32_t per_tile) {  // (tiles * n_items is within its limit)
-        return gather_grid(n_items, tiles, per_tile, out_positions, n_table, g.B);
+    auto to_f32 = [&](uint32_t per_tile, bool one_xcd) {  // (tiles * n_items is within its limit)
+        return gather_grid(n_items, tiles, per_tile, out_positions, n_table, g.B, one_xcd);
     };
 #define QV_GATHER_Q8(DD)                                                                       \
     do {                                                                                        \
         const uint32_t pq = (2u * (uint32_t)g.G * (uint32_t)DD + 63u) / 64u;                     \
-        const GatherGrid gg = to_f32(pq);                                                        \
+        const GatherGrid gg = to_f32(pq, DD != 64);                                                        \
         hipLaunchKernelGGL(k_gather_q8<DD>, dim3(gg.wgs), dim3(64), 0, s, p, pool_blocks, blocks, \
                            n_table, table_at, lens, out_at, n_items, tiles, out_positions,      \
-                           (float *)out_k, (float *)out_v, pq, gg.by_tile, geo, err);           \
+                           (float *)out_k, (float *)out_v, pq, gg.by_tile, gg.by_xcd, geo, err); \
     } while (0)
     const bool q8fast = tune(KNOB_GATHER_Q8_FAST) != 0;
     if (g.dtype == QVKV_Q8_0 && q8fast && g.D == 64) QV_GATHER_Q8(64);
@@ -2064,7 +2065,7 @@ hipError_t launch_gather(const Geometry &g, const void *pool, uint64_t pool_bloc
     else if (g.dtype == QVKV_F16) {
         // 64 threads x 4 pieces x 4 values (1, 2 and 8 pieces per thread were slower)
         const uint32_t pf = (uint32_t)((vals + 1023) / 1024);
-        const GatherGrid gg = to_f32(pf);
+        const GatherGrid gg = to_f32(pf, false);
         hipLaunchKernelGGL((k_gather<QVKV_F16, QVKV_F32, 64, 4>), dim3(gg.wgs), dim3(64), 0, s, p,
                            pool_blocks, blocks, n_table, table_at, lens, out_at, n_items, tiles,
                            out_positions, out_k, out_v, pf, gg.by_tile, geo, err);

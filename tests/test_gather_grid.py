@@ -16,13 +16,19 @@ static int bad(const char *what, unsigned long long a, unsigned long long b) {
     return 1;
 }
 // the walk of each_live_tile by the workgroups of one piece
-static int covers(uint64_t items, uint64_t tiles, uint64_t per_tile, uint64_t positions) {
-    const qvkv::GatherGrid g = qvkv::gather_grid(items, tiles, per_tile, positions, 1ull << 40, 16);
+static int covers(uint64_t items, uint64_t tiles, uint64_t per_tile, uint64_t positions, bool one_xcd) {
+    const qvkv::GatherGrid g = qvkv::gather_grid(items, tiles, per_tile, positions, 1ull << 40, 16, one_xcd);
     const uint64_t most = g.by_tile ? (1u << 18) + per_tile : (1u << 26) - 1;
     if (g.wgs == 0 || g.wgs % per_tile || g.wgs > most) return bad("wgs", g.wgs, per_tile);
     const uint64_t units = items * tiles, step = g.wgs / per_tile;
     if (g.by_tile && step > positions / 16 + items) return bad("more than held", step, positions);
     std::vector<uint8_t> seen(units, 0);
+    std::vector<uint8_t> starts(step * per_tile, 0);
+    for (uint32_t wg = 0; wg < g.wgs; wg++) {
+        const qvkv::GatherPlace at = qvkv::gather_place(wg, (uint32_t)per_tile, g.by_xcd);
+        if (at.part >= per_tile || at.unit >= step || starts[at.unit * per_tile + at.part]++) return bad("place", wg, step);
+        if (g.by_xcd && wg % 8 != at.unit % 8) return bad("xcd", wg, at.unit);
+    }
     for (uint64_t u0 = 0; u0 < step; u0++)
         for (uint64_t u = u0; u < units; u += step) {
             const uint64_t by = g.by_tile ? items : tiles, q = u / by, r = u - q * by;
@@ -38,7 +44,10 @@ int main() {
     const uint64_t shapes[][4] = {{1, 1, 1, 16}, {64, 64, 32, 65536}, {64, 2048, 32, 97280}, {256, 2048, 16, 49088},
                                   {7, 5, 3, 560}, {64, 128, 32, 131072}, {33, 4096, 2, 4096}, {4096, 1024, 128, 65536},
                                   {1000, 1000, 1, 16000000}, {3, 1, 300000, 48}, {100, 63, 512, 6400}};
-    for (auto &s : shapes) rc |= covers(s[0], s[1], s[2], s[3]);
+    for (auto &s : shapes)
+        for (bool one_xcd : {false, true}) rc |= covers(s[0], s[1], s[2], s[3], one_xcd);
+    for (uint64_t tiles : {128, 129, 131}) rc |= covers(128, tiles, 32, 128 * 16 * tiles, true);
+    if (!qvkv::gather_grid(128, 129, 32, 128 * 16 * 129, 1 << 20, 16, true).by_xcd) rc |= bad("by_xcd", 0, 0);
     // an even batch: a workgroup per piece of every unit
     if (qvkv::gather_grid(512, 128, 32, 512 * 2048, 512 * 128, 16).wgs != 512 * 128 * 32) rc |= bad("even", 0, 0);
     // an uneven batch: far fewer workgroups than pieces (a workgroup costs its dispatch)

@@ -63,12 +63,18 @@ def uneven(hip, dtype, G, D, lens, max_len, seed=3):
 
 @pytest.mark.parametrize("dtype,G,D", [(Q8_0, 8, 128), (Q8_0, 1, 64), (Q8_0, 3, 256), (F16, 8, 128), (F16, 3, 64)])
 def test_gather_of_uneven_items(hip, dtype, G, D):
-    """One item far longer than the rest (units tile by tile), and a batch of more pieces than
-    workgroups (units item by item)."""
+    """One item far longer than the rest (units tile by tile), and batches of many pieces (units item
+    by item)."""
     uneven(hip, dtype, G, D, [9001] + [1 + i % 40 for i in range(150)], 9001)
     uneven(hip, dtype, G, D, [17] * 70 + [20000], 20000)
     if G == 8:
         uneven(hip, dtype, G, D, [1 + (i * 37) % 1024 for i in range(160)], 1024)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_gather_of_many_even_items(hip, D):
+    """More than 16384 units, their number not a multiple of 8 (d = 128, 256: one XCD each)."""
+    uneven(hip, Q8_0, 1, D, [200 + i % 61 for i in range(1101)], 260)
 
 
 def test_gather_of_more_units_than_a_launch_holds(hip):
