@@ -23,11 +23,13 @@
  *    a flag of that stream and reported by the next qvkv_check() of the same stream.
  *    Kernels never touch memory outside the pool for such input.
  *  - Threads: any thread may call (the trait is Send + Sync).  The library keeps an error
- *    flag and an attention workspace per stream, so callers on different streams never
- *    see each other's errors or overwrite each other's partial results.  The first launch
- *    on a stream sets its state up (a small device allocation), and an attention launch
- *    may grow the stream's workspace: before capturing a stream into a HIP graph, run the
- *    launches once uncaptured (or use qvkv_attention_noalloc_async).
+ *    flag, an attention workspace and a prefill workspace per stream, so callers on different
+ *    streams never see each other's errors or overwrite each other's partial results.  The
+ *    first launch on a stream sets its state up (a small device allocation), and a launch
+ *    may grow the stream's workspaces: before capturing a stream into a HIP graph, run the
+ *    launches once uncaptured (or use qvkv_attention_noalloc_async).  A captured attention
+ *    launch uses the capture stream's workspace: replay its graph in order with that stream's
+ *    attention launches.  A captured prefill launch uses none.
  *  - A pool position is `slot = block * layout.block + offset` (the reference's
  *    `sync_to`, crates/qubivex-compute/src/discrete.rs:301-304).  Item t of a batch is
  *    one (sequence, layer) pair: its blocks are blocks[table_at[t] ..], in position order
@@ -242,12 +244,18 @@ int qvkv_attention_noalloc_async(qvkv_dev *dev, const qvkv_layout *layout, const
  * q row q_at[i] + j ([q_rows][heads][d] f32) and writes the same out row.  It attends
  * (causally) over positions 0..pos0[i]+j of its table exactly as qvkv_attention_async
  * would for an item with pos = pos0[i]+j; max_pos bounds pos0[i]+n_tok[i]-1 and max_tok
- * bounds n_tok[i].  A launch with few rows shares each row block's context out to several
- * workgroups, whose partial results go to a workspace of the stream (grown on first use).  A
- * launch under capture never uses it: it runs unsplit, so its graph may be replayed on any
- * stream, beside any other launch.  Replaces the host prefill of the reference's forward
- * pass, which stores a segment's rows and then runs math::attend per (token, head)
+ * bounds n_tok[i].  Replaces the host prefill of the reference's forward pass, which
+ * stores a segment's rows and then runs math::attend per (token, head)
  * (crates/qubivex-arch/src/lib.rs:1296-1320); the reference has no device prefill.
+ * Workspace: a launch with few rows shares each row block's context out to several
+ * workgroups, whose partial results (up to about 200 MiB) go to a prefill workspace of the
+ * stream; a q8_0 launch at d = 128 whose max_tok gives 12 or more blocks of 64 query rows per
+ * KV head keeps f16 images of its segments' contexts there, 776 bytes per position and KV
+ * head, for as many segments at once as 512 MiB hold.  It grows by doubling when a launch needs
+ * more (which waits for the stream's earlier work) and is held until qvkv_close; usage()
+ * counts it.  Where the device has no memory for it the launch runs with what there is, down
+ * to none, and still succeeds.  A launch under capture never uses it: it runs unsplit and
+ * without images, so its graph may be replayed on any stream, beside any other launch.
  * q8_0 pools at d = 128 use a form that holds dequantised values in f16: a value scale
  * above 512 (values that may pass 65504) makes the next qvkv_check return
  * QVKV_E_UNSUPPORTED.  The synchronous entry points (qvkv_decode_attention,
