@@ -185,8 +185,7 @@ struct RowBlock {
 __device__ __forceinline__ RowBlock row_block(uint32_t n_cb, uint32_t n_ch, uint32_t n_sub,
                                               bool xcd_map) {
     // n_sub is a power of two (sub_groups).  A division by a runtime value is tens of
-    // instructions before the first load: one here, and one more where the launch is split
-    // (8 segments of 8 to 64 tokens on 2 047 cached, 32 heads: 45.9 -> 45.5 us).
+    // instructions before the first load: one here, and one more where the launch is split.
     const uint32_t lg = (uint32_t)__builtin_ctz(n_sub), per = (n_cb + n_sub - 1) >> lg;
     const uint32_t bid = blockIdx.x;
     const uint32_t i = xcd_map ? bid / 8 : bid, q = i / per;

@@ -1,4 +1,4 @@
-"""The bookkeeping of decode attention split by work (k_attn_stream and
+"""The bookkeeping of decode attention split by work (attn_stream_wg, k_attn_stream and
 k_attn_stream_merge in qubivex_amd/csrc/kernels.hip), restated on the CPU: workgroup w
 takes the slots [floor(w T / P), floor((w + 1) T / P)) of the unit-major work order, where
 each unit holds `cost` set-up slots (its per-unit overhead, no tiles) and then one slot per
