@@ -2138,7 +2138,7 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     // the price of a merge launch.  With more units the split has more cut units to merge, and
     // the line moves out.  Measured in us per call, 8 KV heads, contexts of half to all of n, wide /
     // split: f16 d = 128, 8 units of n = 640 12.2 / 12.4, of 960 15.6 / 12.8; 128 of 640 16.0 / 18.1, of
-    // 960 21.6 / 20.2; 192 of 960 22.1 / 25.2, of 1280 26.8 / 29.4; 256 of 1280 28.4 / 34.1.  f16 d = 64,
+    // 960 21.6 / 20.2 (all of 953 22.4 / 24.0); 192 of 960 22.1 / 25.2, of 1280 26.8 / 29.4; 256 of 1280 28.4 / 34.1.  f16 d = 64,
     // 8 units of 960 12.0 / 12.6, of 1280 14.6 / 12.8; 64 of 1280 15.9 / 15.7; 128 of 1408 16.7 / 18.3, of
     // 2048 22.6 / 20.4; 256 of 2048 25.5 / 28.7.  q8_0 d = 128, 8 units of 960 18.5 / 17.5; 64 of 1280
     // 20.3 / 21.4, of 1408 22.5 / 21.2; 128 of 2048 27.2 / 27.4, 256 29.7 / 36.4; d = 64, 8 units of 1408
@@ -2148,8 +2148,7 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     const bool split_set = full != (uint64_t)kKnobDefault[KNOB_ATTN_FULL] ||
                            tune(KNOB_ATTN_STREAM) != 1 || tune(KNOB_ATTN_STREAM_WG) > 0;
     const int wide = tune(KNOB_ATTN_WIDE);
-    const uint64_t many = !q8 && g.D == 128 ? 192 : 128;
-    const uint64_t wide_tiles = wide >= 0 ? (uint64_t)wide : split_set ? 0 : units >= many ? 2 * base : base;
+    const uint64_t wide_tiles = wide >= 0 ? (uint64_t)wide : split_set ? 0 : units >= 128 ? 2 * base : base;
     if (units < full && units <= 256 && g.D != 256 && max_tiles <= wide_tiles) {
         p->kind = 3;
         return QVKV_OK;
