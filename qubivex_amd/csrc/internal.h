@@ -97,7 +97,7 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
     X(ATTN_WIDE, "attn_wide", -1)               /* tiles up to which units run wide; -1: rule */ \
     X(ATTN_STREAM, "attn_stream", 1)            /* 1: split by work, 0: context chunks */       \
     X(ATTN_STREAM_WG, "attn_stream_wg", 0)      /* 0: by the launch's tiles */                  \
-    X(STREAM_UNIT_COST, "stream_unit_cost", 8)  /* a unit's set-up cost in tiles */             \
+    X(STREAM_UNIT_COST, "stream_unit_cost", -1) /* a unit's set-up cost in tiles; -1: rule */   \
     X(ATTN_TARGET, "attn_target", 1536)         /* context-chunk split: workgroups aimed at */  \
     X(FUSED_Q8, "fused_q8", 1)                  /* fused append + attention for q8_0 */         \
     X(ATTN_WAVES4_F16, "attn_waves4_f16", 0)                                                    \

@@ -1629,9 +1629,9 @@ void k_attn_stream_nr(QV_STREAM_PARAMS) {
 // their own / workgroups), contexts of 1000-4000 unless said:
 //   f16 d = 128, 768 workgroups: 16 sequences 40.7 / 40.4, 32 of 256-4096 59.6 / 58.4, 32 of 2048 54.7 /
 //     51.5, one of 2048 17.1 / 14.4; 64 of 4096 with 4 KV heads 99.4 / 92.7;
-//   q8_0 d = 128, 768: 16 sequences 33.7 / 34.0, 32 48.7 / 49.4, 60 of 300-3000 59.0 / 62.2; 16 of 4000
-//     40.7 / 37.9, 48 of 2048 55.3 / 52.0, one of 2000 17.4 / 14.8;
-//   q8_0 d = 64, 768 (pipelined): 16 35.9 / 25.8, 32 of 4000 63.3 / 37.9, one of 2000 14.6 / 12.6;
+//   q8_0 d = 128, 768: 16 sequences 33.7 / 32.3, 32 48.6 / 48.2, 60 of 300-3000 59.4 / 59.5; 16 of 4000
+//     40.7 / 38.0, 48 of 2048 55.1 / 53.6, one of 2000 17.4 / 14.8;
+//   q8_0 d = 64, 768 (pipelined): 16 36.1 / 24.8, 32 of 4000 63.0 / 38.1, one of 2000 15.2 / 13.3;
 //   f16 d = 64: 8 19.5 / 20.5, 32 39.4 / 44.5, 32 of 2048 27.2 / 36.1: waves on their own;
 //   d = 256, 256 workgroups: waves on their own above 8192 (unit, tile) pairs (f16 16 sequences 79.3 /
 //     82.3, 63 of 1000-2000 157.6 / 178.3), else workgroups (4 of 258 22.3 / 17.7, 4 of 2000 31.3 / 28.1,
@@ -2186,8 +2186,12 @@ int plan_attention(const Geometry &g, uint32_t n_items, uint32_t heads, uint32_t
         // Each unit also costs set-up work (its query rows, table start, the workgroup's
         // LDS merge and output) worth about 8 tiles: counting it in the shares evens out
         // workgroups that start several short units (cfg2-like layer of 32 ragged items:
-        // 64.2 -> 60.1 us; contexts / 8: 31.7 -> 22.0 us; 4-24 within 2 % of 8).
-        p->ucost = (uint32_t)tune(KNOB_STREAM_UNIT_COST);
+        // 64.2 -> 60.1 us; contexts / 8: 31.7 -> 22.0 us; 4-24 within 2 % of 8).  Workgroups of
+        // q8_0, whose tiles are half the bytes, do best with 14, in us with 8 / 12 / 16 (8 KV heads):
+        // d = 128, 60 of 300-3000 62.1 / 60.1 / 58.6, 8 of 1000-4000 26.4 / 24.6 / 24.6, 48 of 2048
+        // 52.1 / 53.1 / 53.6; d = 64, 24 of 3000-3500 32.3 / 32.1 / 31.1.
+        const int cost = tune(KNOB_STREAM_UNIT_COST);
+        p->ucost = cost >= 0 ? (uint32_t)cost : q8 && p->by_wg && g.D != 256 ? 14 : 8;
         p->ws_bytes = stream_rec_at(wgs, g.D, n_items) +
                       (uint64_t)n_items * g.G * p->hc * sizeof(StreamRec);
         return QVKV_OK;
