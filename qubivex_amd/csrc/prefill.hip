@@ -23,10 +23,11 @@ namespace qvkv {
         const uint32_t *__restrict__ q_at, const uint32_t *__restrict__ n_tok, uint32_t n_seg,  \
         uint32_t H, uint32_t max_pos, uint32_t max_tok, uint64_t q_rows, uint32_t n_cb,         \
         float *__restrict__ out, Geo geo, int *err
-// (the forms that split the context: n_ch chunks per row block, their partials in ws; n_sub:
-// row_block)
+// (the forms that split the context: n_ch chunks per row block, their partials in ws; n_sub and
+// n_il: row_block)
 #define QV_PREFILL_SPLIT_PARAMS                                                                 \
-    QV_PREFILL_PARAMS, uint32_t n_ch, uint32_t n_sub, float *__restrict__ ws, uint64_t n_parts
+    QV_PREFILL_PARAMS, uint32_t n_ch, uint32_t n_sub, uint32_t n_il, float *__restrict__ ws,     \
+        uint64_t n_parts
 
 template <int D, bool Q8>
 __global__ __launch_bounds__(256) void k_prefill_mfma(QV_PREFILL_PARAMS) {
@@ -178,19 +179,27 @@ __device__ __forceinline__ TileRange chunk_tiles(uint32_t n, uint32_t ch, uint32
 // different XCDs: segments of different lengths then load the XCDs alike (with each XCD
 // taking an eighth of the launch in order, 8 segments of 8 to 64 tokens put the longest
 // on one XCD).  Few groups are cut into n_sub interleaved parts each, so that their number
-// is a multiple of 8.  Blocks of later tokens, whose contexts are longest, start first.
+// is a multiple of 8.  Blocks of later tokens, whose contexts are longest, start first: part by
+// part, so that few parts' tiles are in the L2 at once, or (n_il: parts per XCD), where every
+// workgroup of the launch runs at once, the longest of all parts before the next, so that two of
+// the longest do not share a CU while another has a short one alone.  In us, part by part / block
+// by block: 4 prompts of 700, 8 heads x 1, 26.8 / 24.5; 5 tails of 241, 2 x 8, 20.0 / 18.4; 8 of 200-400,
+// 8 x 2, 34.6 / 31.7; q8_0 4 prompts of 300 27.0 / 25.9; more workgroups than run at once, 16 prompts
+// of 512, 8 x 4, 109.1 / 113.6.
 struct RowBlock {
     uint32_t qb, ch, sg;
 };
-__device__ __forceinline__ RowBlock row_block(uint32_t n_cb, uint32_t n_ch, uint32_t n_sub,
+__device__ __forceinline__ RowBlock row_block(uint32_t n_cb, uint32_t n_ch, uint32_t n_sub, uint32_t n_il,
                                               bool xcd_map) {
     // n_sub is a power of two (sub_groups).  A division by a runtime value is tens of
     // instructions before the first load: one here, and one more where the launch is split.
     const uint32_t lg = (uint32_t)__builtin_ctz(n_sub), per = (n_cb + n_sub - 1) >> lg;
     const uint32_t bid = blockIdx.x;
-    const uint32_t i = xcd_map ? bid / 8 : bid, q = i / per;
+    // part q of the XCD (of all), block b of the part
+    const uint32_t i = xcd_map ? bid / 8 : bid, d = i / (n_il ? n_il : per);
+    const uint32_t r = i - d * (n_il ? n_il : per), q = n_il ? r : d, b = n_il ? d : r;
     const uint32_t part = xcd_map ? q * 8 + bid % 8 : q;
-    const uint32_t at = ((i - q * per) << lg) + (part & (n_sub - 1)), group = part >> lg;
+    const uint32_t at = (b << lg) + (part & (n_sub - 1)), group = part >> lg;
     // (at >= n_cb, in a last part: past every block, as n_cb - 1 - at wraps)
     if (n_ch == 1) return RowBlock{n_cb - 1 - at, 0u, group};
     const uint32_t sg = group / n_ch;
@@ -289,7 +298,7 @@ void k_prefill_f16(QV_PREFILL_SPLIT_PARAMS) {
 
     const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
     const uint32_t GS = H / G;
-    const RowBlock rb = row_block(n_cb, n_ch, n_sub, geo.xcd_map != 0);
+    const RowBlock rb = row_block(n_cb, n_ch, n_sub, n_il, geo.xcd_map != 0);
     const uint32_t qb = rb.qb, ch = rb.ch, sg = rb.sg;
     if (qb >= n_cb) return;
     const uint32_t g = sg % G;
@@ -1006,7 +1015,7 @@ void k_prefill_q8(QV_PREFILL_SPLIT_PARAMS, const uint8_t *__restrict__ img, uint
 
     const uint32_t G = (uint32_t)geo.G, B = (uint32_t)geo.B;
     const uint32_t GS = H / G;
-    const RowBlock rb = row_block(n_cb, n_ch, n_sub, geo.xcd_map != 0);
+    const RowBlock rb = row_block(n_cb, n_ch, n_sub, n_il, geo.xcd_map != 0);
     const uint32_t qb = rb.qb, ch = rb.ch, sg = rb.sg;
     if (qb >= n_cb) return;
     const uint32_t g = sg % G;
@@ -1398,6 +1407,14 @@ static unsigned prefill_grid(uint64_t groups, uint32_t n_sub, uint32_t n_qb) {
     return (unsigned)((groups * n_sub + 7) / 8 * 8 * ((n_qb + n_sub - 1) / n_sub));
 }
 
+// The parts per XCD (of all, without the XCD mapping) of a launch that takes them in turn, block by
+// block (row_block), or 0: those whose workgroups, `grid`, all run at once.
+static uint32_t interleaved(uint64_t groups, uint32_t n_sub, unsigned grid, unsigned slots, bool xcd_map) {
+    if (grid > slots) return 0;
+    const uint64_t parts = (groups * n_sub + 7) / 8 * 8;
+    return (uint32_t)(xcd_map ? parts / 8 : parts);
+}
+
 // Which kernel a prefill launch runs.
 enum class PrefillForm { GENERIC, TILE, F16, Q8 };
 static PrefillForm prefill_form(const Geometry &g, bool f16_values) {
@@ -1451,13 +1468,14 @@ hipError_t launch_prefill(const Geometry &g, const PrefillPlan &plan, const void
             const uint64_t row_blocks = (uint64_t)ns * g.G * n_qb;
             const uint32_t n_sub = sub_groups((uint64_t)ns * g.G * n_ch, n_qb);
             const unsigned grid = prefill_grid((uint64_t)ns * g.G * n_ch, n_sub, n_qb);
+            const uint32_t n_il = interleaved((uint64_t)ns * g.G * n_ch, n_sub, grid, 768, geo.xcd_map != 0);
             hipLaunchKernelGGL(k_q8_images<128>, dim3((unsigned)((uint64_t)ns * g.G * plan.img_tiles)),
                                dim3(256), 0, s, pp, pool_blocks, blocks, n_table, table_at + s0,
                                pos0 + s0, q_at + s0, n_tok + s0, max_pos, max_tok, q_rows, geo, err,
                                img, plan.img_tiles);
             hipLaunchKernelGGL((k_prefill_q8<128, true>), dim3(grid), dim3(256), 0, s, pp, pool_blocks,
                                q, blocks, n_table, table_at + s0, pos0 + s0, q_at + s0, n_tok + s0, ns,
-                               heads, max_pos, max_tok, q_rows, n_qb, out, geo, err, n_ch, n_sub, part,
+                               heads, max_pos, max_tok, q_rows, n_qb, out, geo, err, n_ch, n_sub, n_il, part,
                                row_blocks * n_ch, img, plan.img_tiles);
             if (n_ch > 1)
                 hipLaunchKernelGGL(k_prefill_merge<128>, dim3((unsigned)(row_blocks * 8)), dim3(256), 0, s,
@@ -1475,17 +1493,19 @@ hipError_t launch_prefill(const Geometry &g, const PrefillPlan &plan, const void
         const uint64_t groups = (uint64_t)n_seg * g.G * n_ch;
         const uint32_t n_sub = sub_groups(groups, n_qb);
         const unsigned grid2 = prefill_grid(groups, n_sub, n_qb);
+        const uint32_t n_il = interleaved(groups, n_sub, grid2, form == PrefillForm::F16 && g.D == 64 ? 1024 : 768,
+                                          geo.xcd_map != 0);
         const unsigned pad = (unsigned)tune(KNOB_PREFILL_LDS_PAD);
 #define QV_PF2(KERNEL)                                                                         \
     hipLaunchKernelGGL(KERNEL, dim3(grid2), dim3(256), pad, s, pp, pool_blocks, q, blocks,       \
                        n_table, table_at, pos0, q_at, n_tok, n_seg, heads, max_pos, max_tok,    \
-                       q_rows, n_qb, out, geo, err, n_ch, n_sub, (float *)ws, row_blocks * n_ch)
+                       q_rows, n_qb, out, geo, err, n_ch, n_sub, n_il, (float *)ws, row_blocks * n_ch)
         // P as one f16 (the default) or as high part + residual (knob prefill_exact_p=1)
         const bool ps = tune(KNOB_PREFILL_EXACT_P) != 0;
         if (form == PrefillForm::Q8)
             hipLaunchKernelGGL((k_prefill_q8<128, false>), dim3(grid2), dim3(256), 0, s, pp, pool_blocks,
                                q, blocks, n_table, table_at, pos0, q_at, n_tok, n_seg, heads, max_pos,
-                               max_tok, q_rows, n_qb, out, geo, err, n_ch, n_sub, (float *)ws,
+                               max_tok, q_rows, n_qb, out, geo, err, n_ch, n_sub, n_il, (float *)ws,
                                row_blocks * n_ch, nullptr, 0u);
 #define QV_PF2_D(DD)                                                                           \
     do {                                                                                        \

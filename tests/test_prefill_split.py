@@ -20,11 +20,12 @@ def launch(groups_seg, n_ch, n_qb):
     return n_sub, -(-groups * n_sub // 8) * 8 * -(-n_qb // n_sub)
 
 
-def row_block(bid, n_cb, n_ch, n_sub, xcd_map):
+def row_block(bid, n_cb, n_ch, n_sub, n_il, xcd_map):
     per = -(-n_cb // n_sub)
     i = bid // 8 if xcd_map else bid
-    part = i // per * 8 + bid % 8 if xcd_map else i // per
-    return (n_cb - 1 - (i % per * n_sub + part % n_sub)) % 2**32, part // n_sub % n_ch, part // n_sub // n_ch
+    q, b = (i % n_il, i // n_il) if n_il else (i // per, i % per)
+    part = q * 8 + bid % 8 if xcd_map else q
+    return (n_cb - 1 - (b * n_sub + part % n_sub)) % 2**32, part // n_sub % n_ch, part // n_sub // n_ch
 
 
 @pytest.mark.parametrize("xcd_map", [True, False])
@@ -33,9 +34,11 @@ def test_every_row_block_and_chunk_has_one_workgroup(xcd_map):
     for _ in range(300):
         sg, n_ch, n_qb = r.randint(1, 70), r.randint(1, 16), r.choice([1, 2, 3, 5, 8, 33, 64])
         n_sub, grid = launch(sg, n_ch, n_qb)
-        seen = [b for b in (row_block(x, n_qb, n_ch, n_sub, xcd_map) for x in range(grid))
-                if b[0] < n_qb and b[2] < sg]
-        assert len(seen) == len(set(seen)) == sg * n_ch * n_qb, (sg, n_ch, n_qb)
+        parts = -(-sg * n_ch * n_sub // 8) * 8
+        for n_il in (0, parts // 8 if xcd_map else parts):
+            seen = [b for b in (row_block(x, n_qb, n_ch, n_sub, n_il, xcd_map) for x in range(grid))
+                    if b[0] < n_qb and b[2] < sg]
+            assert len(seen) == len(set(seen)) == sg * n_ch * n_qb, (sg, n_ch, n_qb, n_il)
 
 
 @pytest.mark.gpu
